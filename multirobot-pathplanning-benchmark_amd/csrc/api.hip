@@ -541,7 +541,7 @@ int tune_defaults(const SceneRec* sc, const mrcc_tune* tune, mrcc_tune* t) {
     memset(t, 0, sizeof(*t));
     if (tune) *t = *tune;
     const bool arms = sc->kind == KIND_ARMS;
-    if (t->slots_per_pass <= 0) t->slots_per_pass = arms ? 4 : 8;
+    if (t->slots_per_pass <= 0) t->slots_per_pass = arms ? 1 : 8;
     if (t->slots_per_ticket <= 0) t->slots_per_ticket = arms ? 16 : 4;
     if (t->waves_per_cu <= 0) t->waves_per_cu = 16;
     if (!tune) {
@@ -591,8 +591,15 @@ void launch_plan_sequence(const SceneRec& sc, const EdgeBatchView& B, const Plan
                           int grid, hipStream_t st) {
     launch_plan_build(sc, B, W, lgG, st);
     launch_plan_run(sc, B, W, lgG, spt, grid, st);
-    // edges with more passes than the queue holds: one workgroup per edge
-    launch_direct(sc, B, W.long_list, 0, W.meta + 3, 1, 0, 4 * ::device_cus(), W.stats, st);
+    launch_long_edges(sc, B, W, st);
+}
+
+// Edges with more passes than the queue holds: disk and planar scenes one workgroup per edge, arm
+// scenes every resident wave on one edge after another (16,385 states or more, one per wave and
+// turn).
+void launch_long_edges(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, hipStream_t st) {
+    const int waves = (sc.kind == KIND_ARMS ? 16 : 4) * ::device_cus();
+    launch_direct(sc, B, W.long_list, 0, W.meta + 3, sc.kind == KIND_ARMS ? waves : 1, 0, waves, W.stats, st);
 }
 }  // namespace mrcc_internal
 
@@ -621,9 +628,7 @@ static void plan_launch_sequence(mrcc_edge_plan* p, hipStream_t st) {
         (void)hipEventRecord(p->ev[1], st);
         launch_plan_run(*p->sc, p->B, p->W, p->lgG, p->tune.slots_per_ticket, p->grid, st);
         (void)hipEventRecord(p->ev[2], st);
-        // edges with more passes than the queue holds: one workgroup per edge
-        launch_direct(*p->sc, p->B, p->W.long_list, 0, p->W.meta + 3, 1, 0, 4 * device_cus(),
-                      p->W.stats, st);
+        mrcc_internal::launch_long_edges(*p->sc, p->B, p->W, st);
     } else {
         if (ev) (void)hipEventRecord(p->ev[1], st);
         launch_direct(*p->sc, p->B, nullptr, p->B.n, nullptr, 1, 1, 1 << 20, p->W.stats, st);

@@ -65,6 +65,13 @@ void launch_arm_edge_spread(const SceneRec& sc, const EdgeBatchView& B, int bloc
 void launch_configs(const SceneRec& sc, const double* q, long long n, long long rs, long long ds,
                     const int* modes, unsigned mask, unsigned char* out, int max_grid,
                     hipStream_t st);
+// self-collision screen of arm states (screen.hip), ahead of the full evaluators
+bool arm_screen_applies(const SceneRec& sc, long long n, long long n_min);
+#define MRCC_SCREEN_MIN_EDGES 1536
+#define MRCC_SCREEN_MIN_CONFIGS 49152
+void launch_screen_edges(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, hipStream_t st);
+void launch_screen_configs(const SceneRec& sc, const double* q, long long n, long long rs, long long ds,
+                           const int* modes, unsigned mask, unsigned char* out, hipStream_t st);
 void launch_arm_fk(const SceneRec& sc, const double* q, long long n, long long rs, long long ds,
                    double* out, hipStream_t st);
 void launch_sincos(const double* x, long long n, double* s, double* c, hipStream_t st);
@@ -102,6 +109,7 @@ int tune_defaults(const SceneRec* sc, const mrcc_tune* tune, mrcc_tune* t);
 int plan_grid(const SceneRec* sc, const mrcc_tune& t);
 // Bytes of a plan's workspace for n_edges edges of D coordinates; with W, lays it out from base.
 size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W);
+void launch_long_edges(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, hipStream_t st);
 // queue build, persistent kernel and long-edge fallback on stream st
 void launch_plan_sequence(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, int spt,
                           int grid, hipStream_t st);

@@ -309,6 +309,32 @@ __device__ inline long long claim_chunk(const WV& W, int& q, long long nchunks) 
     return -1;
 }
 
+// A chunk of any counter that has some left (`q`: its place after `home`, where the wave continues),
+// or -1.  The counters are read before one is drawn from: near the end of a queue every wave comes
+// here, and an atomic on each drained counter in turn cost 30 us of a launch (4096 waves, 8
+// counters).  Wave-uniform, all lanes.
+template <class WV>
+__device__ inline long long steal_chunk(const WV& W, int home, int& q, long long nchunks) {
+    const int lane = threadIdx.x & 63;
+    const int xl = (home + lane) & 7;
+    const long long have = (nchunks - xl + 7) >> 3;  // chunks of counter xl
+    for (;;) {
+        bool left = false;
+        if (lane < 8)
+            left = (long long)__hip_atomic_load(W.ticket + 32 * xl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < have;
+        const unsigned long long m = __ballot(left);
+        if (m == 0ull) return -1;
+        q = __builtin_ctzll(m);
+        const int x = (home + q) & 7;
+        unsigned long long k = 0;
+        if (lane == 0) k = atomicAdd(W.ticket + 32 * x, 1ull);
+        k = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(k >> 32)) << 32) |
+            (unsigned)__builtin_amdgcn_readfirstlane((unsigned)k);
+        const long long c = x + 8 * (long long)k;
+        if (c < nchunks) return c;
+    }
+}
+
 // The verdict byte of an edge in the persistent kernels, as every XCD sees it: another wave
 // writes an edge's 0 when one of its states collides, and the later slots of the edge are skipped
 // when they read it.  Each XCD has its own L2 and plain accesses may stay in it (a plain read can
@@ -566,6 +592,12 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
     const ArmRegs R = arm_regs(V, Wl);
     const int lane = wave_lane();
     const long long T = W.meta[0];
+    const int nw = blockDim.x >> 6;
+    const long long n_waves = (long long)gridDim.x * nw;
+    // short queues: at most two slots per wave in one chunk each; longer ones at least 8 chunks per
+    // wave, so that no wave still evaluates a chunk's states one after another when others are done
+    if (T <= 2 * n_waves) spt = min(spt, T > n_waves ? 2 : 1);
+    else if (T < 8 * n_waves * spt) spt = min(spt, max(2, (int)(T / (8 * n_waves))));
     // statistics (compiled away without STATS)
     typename std::conditional<STATS, unsigned long long, NoCount>::type n_eval{}, n_dead{}, n_slots{};
     RecheckT<STATS> rechecks{};
@@ -576,6 +608,7 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
     unsigned recent = 0xffffu;
     const long long nchunks = (T + spt - 1) / spt;
     const int home = blockIdx.x & 7;
+    const int n_pass = (int)W.meta[1];  // passes with slots; pass_start[n_pass] = T
     long long ps_lo = W.pass_start[0], ps_hi = W.pass_start[1];  // pass p's slots (scalar)
     // A wave takes `nb` tickets of one counter at a time (chunks c, c + 8, ...; lane l resolves
     // slot l % spt of the batch's chunk l / spt).  One ticket while the chunks hold states to
@@ -584,7 +617,10 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
     const int nb_max = 64 / spt;
     const int lj = lane / spt, lo_slot = lane - lj * spt;
     int nb = 1;
-    long long c = claim_chunk(W, q, nchunks);
+    // wave w starts on chunk w; the counters hand out the chunks after the first `c_first`
+    const long long c_first = (n_waves + 7) & ~7ll;
+    long long c = (long long)blockIdx.x * nw + (threadIdx.x >> 6);
+    if (c >= nchunks) c = -1;
     while (c >= 0) {
         const long long cj = c + 8 * (long long)lj;
         const long long sl = cj * spt + lo_slot;
@@ -596,13 +632,29 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
         int kl = 0;  // the slot's place among its edge's slots of the pass
         int pl = p;
         bool dead = false;
-        if (valid) {
-            long long lo = ps_lo;
-            if (sl < ps_lo || sl >= ps_hi) {  // another pass: walk from the hint
-                if (W.pass_start[pl] > sl) pl = 0;
-                while (pl < MRCC_MAX_PASSES && W.pass_start[pl + 1] <= sl) ++pl;
-                lo = W.pass_start[pl];
+        long long lo = ps_lo;
+        if (__ballot(valid && (sl < ps_lo || sl >= ps_hi))) {  // some slot of another pass
+            // 64 passes at a time: lane j reads pass wb + j's first slot (one round trip), each lane
+            // searches the window for its slot's pass
+            int wb = c * spt < ps_lo ? 0 : p;  // the wave moved to another counter: from the start
+            bool found = !valid;
+            for (;;) {
+                const long long tab = W.pass_start[min(wb + lane, n_pass)];  // [n_pass] = T
+                int j = 0;
+#pragma unroll
+                for (int h = 32; h >= 1; h >>= 1)
+                    if (__shfl(tab, j + h, 64) <= sl) j += h;
+                const long long t0 = __shfl(tab, j, 64);
+                if (!found && (j < 63 || wb + 63 >= n_pass)) {
+                    found = true;
+                    pl = wb + j;
+                    lo = t0;
+                }
+                if (__all(found)) break;
+                wb += 63;
             }
+        }
+        if (valid) {
             const long long off = sl - lo;
             const long long r = off >> lgG;
             const int k = (int)(off & ((1 << lgG) - 1));
@@ -626,7 +678,9 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
                         w.full = full;
                         w.first = B.incl ? 0 : 1;
                         w.err = 0;
-                        i = edge_state_index(w, local, B.incl);
+                        // one slot per pass: the states of a whole edge in the binary order (any
+                        // order gives the verdict; this one reaches the middle of a long edge first)
+                        i = full && lgG == 0 ? w.first + bfs_index(Mv, local) : edge_state_index(w, local, B.incl);
                         if (i >= 0) {
                             e = ee;
                             N = Nv;
@@ -688,7 +742,7 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
         const int nb_next = jn >= 0 ? 1 : (2 * nb < nb_max ? 2 * nb : nb_max);
         const int x = (home + q) & 7;
         unsigned long long tk = 0;
-        if (lane == 0) tk = atomicAdd(W.ticket + 32 * x, (unsigned long long)nb_next);
+        if (lane == 0 && c_first < nchunks) tk = atomicAdd(W.ticket + 32 * x, (unsigned long long)nb_next);
         while (jn >= 0) {
             const int jc = jn, ej = en, ij = in_, mj = mn;
             const double aj = an, dj = dn;
@@ -721,11 +775,12 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
         }
         const unsigned long long k = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(tk >> 32)) << 32) |
                                      (unsigned)__builtin_amdgcn_readfirstlane((unsigned)tk);
-        c = (long long)x + 8 * (long long)k;
+        if (c_first >= nchunks) break;  // no chunk beyond the waves' first ones
+        c = c_first + x + 8 * (long long)k;
         nb = nb_next;
         if (c >= nchunks) {  // counter x is exhausted: continue on the others
-            ++q;
-            c = claim_chunk(W, q, nchunks);
+            c = steal_chunk(W, home, q, nchunks - c_first);
+            if (c >= 0) c += c_first;
             nb = 1;
         }
     }
@@ -758,6 +813,10 @@ __global__ void __launch_bounds__(256) k_arm_direct(ArmK V, EdgeBatchView B, con
                                                     int wpe, int init_out,
                                                     unsigned long long* stats) {
     extern __shared__ double lds_arm[];
+    if (n_dev) {
+        n_list = *n_dev;
+        if (n_list == 0) return;  // no long edges: before the scene is staged
+    }
     arm_stage_scene(lds_arm, V);
     const ArmLds Wl = arm_lds(lds_arm, V);
     const ArmRegs R = arm_regs(V, Wl);
@@ -765,7 +824,6 @@ __global__ void __launch_bounds__(256) k_arm_direct(ArmK V, EdgeBatchView B, con
     unsigned long long n_eval = 0;
     unsigned rechecks = 0;
     ArmCountT<true> cnt = {0, 0, 0, 0};
-    if (n_dev) n_list = *n_dev;
     const long long nitems = n_list * wpe;
     const long long w0 = (long long)blockIdx.x * nw + (threadIdx.x >> 6);
     for (long long it = w0; it < nitems; it += (long long)gridDim.x * nw) {
@@ -833,6 +891,46 @@ __global__ void __launch_bounds__(256, 3) k_arm_configs(ArmK V, const double* qv
         const bool c = arm_state_collides<GRASP, CHAIN, false>(V, Wl, R, q, mode, mask, rechecks, cnt, false,
                                                                first, t0);
         if (lane == 0) out[r] = c ? 0 : 1;
+    }
+}
+
+// The configurations that the screen left (out[r] = 1): a wave takes `chunk` (<= 64) consecutive
+// rows at a time and evaluates those in turn; the next one's row is loaded ahead.
+template <bool GRASP, bool CHAIN>
+__global__ void __launch_bounds__(GRASP ? 64 * MRCC_PERSISTENT_GRASP_NW : 256, GRASP ? 3 : 4)
+    k_arm_configs_rest(ArmK V, const double* qv, int n, long long rs,
+                                                                         long long ds, const int* modes, unsigned mask,
+                                                                         unsigned char* out, int chunk) {
+    extern __shared__ double lds_arm[];
+    arm_stage_scene(lds_arm, V);
+    const ArmLds Wl = arm_lds(lds_arm, V);
+    const ArmRegs R = arm_regs(V, Wl);
+    const int nw = blockDim.x >> 6, lane = wave_lane();
+    NoCount rechecks;
+    ArmCountT<false> cnt;
+    const long long nchunks = ((long long)n + chunk - 1) / chunk;
+    unsigned recent = 0;  // outcomes of the wave's last states (1: collision)
+    for (long long c = (long long)blockIdx.x * nw + (threadIdx.x >> 6); c < nchunks; c += (long long)gridDim.x * nw) {
+        const int r = (int)(c * chunk) + lane;
+        const bool left = lane < chunk && r < n && out[r] != 0;
+        const int md = left && modes ? modes[r] : 0;
+        unsigned long long m = __ballot(left);
+        auto load = [&](unsigned long long mm) -> double {
+            const long long row = c * chunk + __builtin_ctzll(mm);
+            return lane < V.D ? qv[row * rs + (long long)lane * ds] : 0.0;
+        };
+        double qn = m ? load(m) : 0.0;
+        while (m) {
+            const int j = __builtin_ctzll(m);
+            m &= m - 1ull;
+            const double q = qn;
+            if (m) qn = load(m);
+            const bool hit = arm_state_collides<GRASP, CHAIN, false>(V, Wl, R, q, __builtin_amdgcn_readlane(md, j), mask,
+                                                                     rechecks, cnt,
+                                                                     __builtin_popcount(recent & 0xffffu) >= 8);
+            recent = (recent << 1) | (hit ? 1u : 0u);
+            if (hit && lane == 0) out[c * chunk + j] = 0;
+        }
     }
 }
 
@@ -1215,6 +1313,7 @@ void launch_plan_build(const SceneRec& sc, const EdgeBatchView& B, const PlanWor
     int gs = grid_for(B.n, 256 * SCATTER_EPT);
     if (gs > 1024) gs = 1024;
     k_plan_prep<<<gp, 256, 0, st>>>(B, W, sc.D, lgG, want_dir, lg_lpe, sc.kind == KIND_ARMS ? sc.arm.nm : 0);
+    if (arm_screen_applies(sc, B.n, MRCC_SCREEN_MIN_EDGES)) launch_screen_edges(sc, B, W, lgG, st);
     k_plan_scan<<<1, 1024, 0, st>>>(W, lgG);
     k_plan_scatter<<<gs, 256, 0, st>>>(W, B.n);
 }
@@ -1349,6 +1448,26 @@ void launch_configs(const SceneRec& sc, const double* q, long long n, long long 
             break;
         }
         case KIND_ARMS: {
+            if (arm_screen_applies(sc, n, MRCC_SCREEN_MIN_CONFIGS)) {
+                launch_screen_configs(sc, q, n, rs, ds, modes, mask, out, st);
+                const int nw = sc.arm_nw_pers;
+                const long long waves = (long long)sc.arm_blocks_pers * nw;
+                int chunk = 1;  // at least 4 chunks per resident wave, at most a wave's lanes
+                while (chunk < 64 && n > 4 * waves * chunk) chunk *= 2;
+                const long long nchunks = (n + chunk - 1) / chunk;
+                const int blocks = (int)(((nchunks < waves ? nchunks : waves) + nw - 1) / nw);
+#define MRCC_ARM_REST(G, C) k_arm_configs_rest<G, C><<<blocks, 64 * nw, sc.arm_lds_pers, st>>>(sc.armk, q, (int)n, rs, ds, modes, mask, out, chunk)
+                if (sc.arm.chain) {
+                    if (sc.arm_has_grasp) MRCC_ARM_REST(true, true);
+                    else MRCC_ARM_REST(false, true);
+                } else if (sc.arm_has_grasp) {
+                    MRCC_ARM_REST(true, false);
+                } else {
+                    MRCC_ARM_REST(false, false);
+                }
+#undef MRCC_ARM_REST
+                break;
+            }
             // one wave per configuration up to 4 * max_grid waves
             long long g = n < (long long)max_grid * 4 ? n : (long long)max_grid * 4;
             if (g < 1) g = 1;

@@ -324,8 +324,37 @@ int build_arm_device(SceneRec* sc, const ArmHost& H) {
     if (nm <= MRCC_MODES_LDS_MAX) put(lay.o_mact, H.m_active.data(), 4 * (size_t)nm);
     put(lay.o_sets, lpair_sets.data(), 4 * lpair_sets.size());
     if (NP <= ARM_PAIRS_LDS_MAX) put(lay.o_pairs, lpairs2.data(), 4 * lpairs2.size());
+    // the clearance kernels' binary32 image, laid out as clr_layout
+    const ClrLayout cl = clr_layout(L, na, nb, S, NP, nclu, H.is_chain);
+    std::vector<unsigned char> cimg(cl.bytes, 0);
+    {
+        auto f4 = [&](int off, double x, double y, double z, double w) {
+            const float v[4] = {(float)x, (float)y, (float)z, (float)w};
+            memcpy(cimg.data() + off, v, 16);
+        };
+        for (int l = 0; l < L; ++l) {
+            const double* j = dh4.data() + (H.is_chain ? 12 : 4) * (size_t)l;
+            for (int r = 0; r < (H.is_chain ? 3 : 1); ++r)
+                f4(cl.o_joint + 16 * ((H.is_chain ? 3 : 1) * l + r), j[4 * r], j[4 * r + 1], j[4 * r + 2], j[4 * r + 3]);
+            f4(cl.o_lbc + 16 * l, link_bc[3 * l], link_bc[3 * l + 1], link_bc[3 * l + 2], link_R[l]);
+            const int fc = link_first[l] | ((link_first[l + 1] - link_first[l]) << 16);
+            memcpy(cimg.data() + cl.o_fc + 4 * l, &fc, 4);
+        }
+        for (int a = 0; a < na; ++a)
+            for (int r = 0; r < 3; ++r) {
+                const double* b = H.base.data() + 12 * a;
+                f4(cl.o_base + 16 * (3 * a + r), b[3 * r], b[3 * r + 1], b[3 * r + 2], b[9 + r]);
+            }
+        for (int t = 0; t < S; ++t) {
+            f4(cl.o_sph + 16 * t, H.sph[4 * t], H.sph[4 * t + 1], H.sph[4 * t + 2], sph_r32[t]);
+            memcpy(cimg.data() + cl.o_slink + 4 * t, &sph_link[t], 4);
+        }
+        if (nclu > 0) memcpy(cimg.data() + cl.o_box, box32.data(), 4 * box32.size());
+        if (nclu > 0) memcpy(cimg.data() + cl.o_clu, clu32.data(), 32 * (size_t)nclu);
+        if (NP > 0 && NP <= ARM_PAIRS_LDS_MAX) memcpy(cimg.data() + cl.o_pairs, lpairs2.data(), 4 * lpairs2.size());
+    }
     Packer P;
-    size_t o_img = P.add(img);
+    size_t o_img = P.add(img), o_cimg = P.add(cimg);
     size_t o_lbc = P.add(link_bc), o_lR = P.add(link_R), o_lp = P.add(lpairs2), o_lpc = P.add(lpair_sets);
     size_t o_base = P.add(H.base), o_dh = P.add(dh4), o_lf = P.add(link_first), o_sl = P.add(sph_link),
            o_slo = P.add(sph_lo), o_s64 = P.add(H.sph), o_sr = P.add(sph_r32), o_b32 = P.add(box32),
@@ -418,6 +447,22 @@ int build_arm_device(SceneRec* sc, const ArmHost& H) {
         K.o_boxch64 = (int)o_bch64; K.o_sph64 = (int)o_s64; K.o_sphlo = (int)o_slo; K.o_pairs = (int)o_lp;
         K.o_mact = (int)o_ma; K.o_mgrasp = (int)o_mg; K.o_mrel = (int)o_mr; K.o_mhalf = (int)o_mh;
         K.o_travel = (int)o_tr;
+    }
+    {
+        ClrK& K = sc->clr;
+        memset(&K, 0, sizeof(K));
+        K.na = na; K.dof = dof; K.D = V.D; K.L = L; K.S = S; K.nb = nb; K.NP = NP; K.nclu = nclu;
+        K.chain = V.chain;
+        K.prism = V.prism;
+        for (int k = 0; k < 3; ++k) {
+            K.bb_lo[k] = V.bb_lo[k];
+            K.bb_hi[k] = V.bb_hi[k];
+        }
+        K.img = at<float4>(d, o_cimg);
+        K.img_bytes = cl.bytes;
+        K.box32 = at<float4>(d, o_b32);
+        K.lpairs2 = V.lpairs2;
+        K.sph_lo = V.sph_lo;
     }
     // waves per workgroup: the most resident waves per CU (160 KiB of LDS) within 64 KiB per
     // workgroup; the scene is staged once per workgroup

@@ -3,125 +3,144 @@
 //   cost(q) = sum over the checked pair set of max(0, m + r_i + r_j - |c_i - c_j|)^2
 //           + sum over spheres x boxes of max(0, m + r_i - dist(c_i, box))^2
 // with the pair set of the boolean check (links >= 2 apart in one arm, all links of different
-// arms), culled exactly with the links' bounding spheres.  One waypoint per wavefront.  The
-// backward recomputes the forward kinematics, gathers the force on every sphere centre
-// (d cost / d c) in LDS and maps it to the joints with
-// d c / d q_k = z_{k-1} x (c - o_{k-1}) (revolute joints) or z_{k-1} (prismatic chain joints) for
-// spheres on links >= k of the same arm.
+// arms), culled exactly with the links' bounding spheres.  The backward recomputes the forward
+// kinematics, sums the force of every term and its moment (d cost / d c and c x that) per link in
+// LDS, and maps them to the joints with d c / d q_k = z_{k-1} x (c - o_{k-1}) (revolute joints) or
+// z_{k-1} (prismatic chain joints) for spheres on links >= k of the same arm.
+//
+// Bound by instruction issue and LDS latency (the inputs are 4 D bytes a waypoint).  One waypoint per
+// wave at a time, its kinematics in pairs of waypoints; a workgroup of several waves stages the
+// scene's binary32 tables in LDS once and walks the batch.
 #include "engine.hpp"
 
 namespace {
 
+#define CLR_MAX_NW 8  // waves per workgroup
+
 struct ClrLds {
-    float* cs;     // [D]
-    float* sn;     // [D]
-    float* X;      // [L*12]
-    float4* sph;   // [S]
-    float* F;      // [S*3] forces (backward)
-    float* red;    // [64]
+    // per wave
+    float4* X;     // [2][L*3] rows (R0 R1 R2 t) of every link frame, two waypoints
+    float2* cs;    // [2*D] cosine, sine of every joint (kinematics; shares memory with sph)
+    float4* sph;   // [S] sphere centres, radii
     float4* lk;    // [L] link bounding spheres (x, y, z, R)
-    int* cand;     // [64] candidates of one culling round
     float* tf;     // [L*6] per link: sum of c x f and sum of f over its spheres (backward)
+    int* cand;     // [64] candidates of one culling round
     int* cand2;    // [64] second-level candidates (link, box) of the clustered box test
+    // per workgroup (the scene)
+    const float4* joint;  // [L] d a cos(alpha) sin(alpha), or [L*3] rows of C (chain joints)
+    const float4* base;   // [na*3] rows
+    const float4* sphL;   // [S] centre in the link frame, radius
+    const float4* lbc;    // [L] bounding-sphere centre in the link frame, radius
+    const int* fc;        // [L] first sphere | count << 16
+    const int* slink;     // [S] link of the sphere
+    const float4* box;    // [nb*2] lo, hi (LDS; scenes with box clusters only)
+    const float4* clu;    // [nclu*2] lo xyz | first box, hi xyz | box count
+    const int2* pairs;    // [NP] (NP <= ARM_PAIRS_LDS_MAX)
 };
 
-__device__ inline ClrLds clr_lds(void* base, const ArmView& V) {
+inline __host__ __device__ int clr_sph_bytes(int D, int S) { return 16 * (S > D ? S : D); }
+inline __host__ __device__ int clr_wave_bytes(int D, int L, int S) {
+    return 96 * L + clr_sph_bytes(D, S) + 16 * L + ((24 * L + 15) & ~15) + 512;
+}
+
+__device__ inline ClrLds clr_lds(unsigned char* b, const ClrK& V) {
+    const ClrLayout o = clr_layout(V.L, V.na, V.nb, V.S, V.NP, V.nclu, V.chain);
     ClrLds W;
-    float* f = (float*)base;
-    W.cs = f;
-    W.sn = f + V.D;
-    W.X = f + 2 * V.D;
-    W.sph = (float4*)(((uintptr_t)(W.X + 12 * V.L) + 15) & ~uintptr_t(15));
-    W.F = (float*)(W.sph + V.S);
-    W.red = W.F + 3 * V.S;
-    W.lk = (float4*)(((uintptr_t)(W.red + 64) + 15) & ~uintptr_t(15));
-    W.cand = (int*)(W.lk + V.L);
-    W.tf = (float*)(W.cand + 64);
-    W.cand2 = (int*)(W.tf + 6 * V.L);
+    W.joint = (const float4*)(b + o.o_joint);
+    W.base = (const float4*)(b + o.o_base);
+    W.sphL = (const float4*)(b + o.o_sph);
+    W.lbc = (const float4*)(b + o.o_lbc);
+    W.fc = (const int*)(b + o.o_fc);
+    W.slink = (const int*)(b + o.o_slink);
+    W.box = (const float4*)(b + o.o_box);
+    W.clu = (const float4*)(b + o.o_clu);
+    W.pairs = (const int2*)(b + o.o_pairs);
+    unsigned char* w = b + o.bytes + (threadIdx.x >> 6) * clr_wave_bytes(V.D, V.L, V.S);
+    W.X = (float4*)w;
+    w += 96 * V.L;
+    W.sph = (float4*)w;
+    W.cs = (float2*)w;
+    w += clr_sph_bytes(V.D, V.S);
+    W.lk = (float4*)w;
+    w += 16 * V.L;
+    W.tf = (float*)w;
+    w += (24 * V.L + 15) & ~15;
+    W.cand = (int*)w;
+    W.cand2 = W.cand + 64;
     return W;
 }
 
-// value of lane (lane & ~3) + J of the lane's quad (DPP quad_perm broadcast; the quad's lanes active)
-template <int J>
-__device__ inline float quad_bcast_f32(float v) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), J * 0x55, 0xf, 0xf, false));
-}
-
-// forward kinematics in binary32 and sphere centres into LDS
-__device__ inline void clr_fk(const ArmView& V, const ClrLds& W, const float* q) {
-    const int lane = threadIdx.x;
-    if (lane < V.D) {
+// Forward kinematics of `nw` (1 or 2) waypoints: the rows of every link frame into W.X.  Lane
+// (waypoint, arm, row) carries a row through its arm's joints (rows are independent of each other).
+template <bool CHAIN>
+__device__ inline void clr_fk(const ClrK& V, const ClrLds& W, const float* q, int nw) {
+    const int lane = wave_lane();
+    for (int t = lane; t < nw * V.D; t += 64) {
         float s, c;
-        sincosf(q[lane], &s, &c);
-        const bool pr = (V.prism >> lane) & 1ull;  // prismatic: Tz(q) C = Rz(0) C + q e_z
-        W.cs[lane] = pr ? 1.f : c;
-        W.sn[lane] = pr ? 0.f : s;
+        sincosf(q[t], &s, &c);
+        const int k = t < V.D ? t : t - V.D;
+        const bool pr = CHAIN && ((V.prism >> k) & 1ull);  // prismatic: Tz(q) C = Rz(0) C + q e_z
+        W.cs[t] = pr ? make_float2(1.f, 0.f) : make_float2(c, s);
     }
-    __syncthreads();
-    // lane (arm a, row r, column c) carries entry (r, c) of its arm's transform through the chain,
-    // arms 5 at a time (60 lanes); the quad of a row shares the row's new entries (DPP broadcasts)
-    {
-        const int c = lane & 3, rr = (lane >> 2) % 3, ag = lane / 12;
-        for (int a0 = 0; a0 < V.na; a0 += 5) {
-            const int a = a0 + ag;
-            if (ag < 5 && a < V.na) {
-                const double* B = V.base + 12 * a;
-                float R0 = (float)B[3 * rr], R1 = (float)B[3 * rr + 1], R2 = (float)B[3 * rr + 2], t = (float)B[9 + rr];
-                for (int k = 0; k < V.dof; ++k) {
-                    const int l = a * V.dof + k;
-                    const float cs = W.cs[l], sn = W.sn[l];
-                    float A0, A1, A2;  // column c of the joint's step A (3 x 4)
-                    if (V.chain) {  // A = Rz(q) C (revolute), Tz(q) C (prismatic)
-                        const double* C = V.dh + 12 * l;
-                        const float c0 = (float)C[c], c1 = (float)C[4 + c];
-                        A0 = cs * c0 - sn * c1;
-                        A1 = sn * c0 + cs * c1;
-                        A2 = (float)C[8 + c];
-                        if (c == 3 && ((V.prism >> l) & 1ull)) A2 += q[l];
-                    } else {
-                        const double* pd = V.dh + 4 * l;
-                        const float d = (float)pd[0], al = (float)pd[1], ca = (float)pd[2], sa = (float)pd[3];
-                        A0 = c == 0 ? cs : (c == 1 ? -sn * ca : (c == 2 ? sn * sa : al * cs));
-                        A1 = c == 0 ? sn : (c == 1 ? cs * ca : (c == 2 ? -cs * sa : al * sn));
-                        A2 = c == 0 ? 0.f : (c == 1 ? sa : (c == 2 ? ca : d));
-                    }
-                    const float y = R0 * A0 + R1 * A1 + R2 * A2 + (c == 3 ? t : 0.f);
-                    W.X[12 * l + (c < 3 ? 3 * rr + c : 9 + rr)] = y;
-                    R0 = quad_bcast_f32<0>(y);
-                    R1 = quad_bcast_f32<1>(y);
-                    R2 = quad_bcast_f32<2>(y);
-                    t = quad_bcast_f32<3>(y);
-                }
+    wave_sync();
+    const int rows = 3 * V.na;  // <= 24
+    if (lane < nw * rows) {
+        const int w = lane >= rows ? 1 : 0, ar = lane - w * rows, a = ar / 3, r = ar - 3 * a;
+        const float4 b = W.base[ar];
+        float R0 = b.x, R1 = b.y, R2 = b.z, t = b.w;
+        const int l0 = a * V.dof;
+        for (int k = 0; k < V.dof; ++k) {
+            const int l = l0 + k;
+            const float2 cs = W.cs[w * V.D + l];
+            float y0, y1, y2, y3;
+            if constexpr (CHAIN) {  // A = Rz(q) C (revolute), Tz(q) C (prismatic)
+                const float4 c0 = W.joint[3 * l], c1 = W.joint[3 * l + 1], c2 = W.joint[3 * l + 2];
+                const float u = R0 * cs.x + R1 * cs.y, v = R1 * cs.x - R0 * cs.y;
+                const float q3 = ((V.prism >> l) & 1ull) ? q[w * V.D + l] : 0.f;
+                y0 = u * c0.x + v * c1.x + R2 * c2.x;
+                y1 = u * c0.y + v * c1.y + R2 * c2.y;
+                y2 = u * c0.z + v * c1.z + R2 * c2.z;
+                y3 = u * c0.w + v * c1.w + R2 * (c2.w + q3) + t;
+            } else {  // A = Rz(q) Tz(d) Tx(a) Rx(alpha)
+                const float4 p = W.joint[l];
+                const float u = R0 * cs.x + R1 * cs.y, v = R1 * cs.x - R0 * cs.y;
+                y0 = u;
+                y1 = v * p.z + R2 * p.w;
+                y2 = R2 * p.z - v * p.w;
+                y3 = u * p.y + R2 * p.x + t;
             }
+            W.X[(w * V.L + l) * 3 + r] = make_float4(y0, y1, y2, y3);
+            R0 = y0;
+            R1 = y1;
+            R2 = y2;
+            t = y3;
         }
     }
-    __syncthreads();
-    for (int s = lane; s < V.S; s += 64) {
-        const float* X = W.X + 12 * V.sph_link[s];
-        const double* l = V.sph64 + 4 * s;
-        const float l0 = (float)l[0], l1 = (float)l[1], l2 = (float)l[2];
-        W.sph[s] = make_float4(X[0] * l0 + X[1] * l1 + X[2] * l2 + X[9], X[3] * l0 + X[4] * l1 + X[5] * l2 + X[10],
-                               X[6] * l0 + X[7] * l1 + X[8] * l2 + X[11], V.sph_r32[s]);
-    }
-    __syncthreads();
+    wave_sync();
+}
+
+__device__ inline float4 clr_point(const float4* X, float4 l) {
+    const float4 a = X[0], b = X[1], c = X[2];
+    return make_float4(a.x * l.x + a.y * l.y + a.z * l.z + a.w, b.x * l.x + b.y * l.y + b.z * l.z + b.w,
+                       c.x * l.x + c.y * l.y + c.z * l.z + c.w, l.w);
 }
 
 // Slack of the link-level cull (metres): covers the binary32 rounding of the link and sphere
 // centres (micrometres) with a wide margin.
 #define CLR_CULL_EPS 1e-4f
 
-// One penetration term: cost += pen^2 for pen = R - d > 0, and the force on the first sphere
-// (fx, fy, fz += g e, g = -2 pen / d) when `grad`.  The square root only for pairs within reach:
-// d < R implies e2 < R^2 (1 + 2^-21), so the bound passes every pair with pen > 0.
-__device__ inline bool clr_term(float ex, float ey, float ez, float R, bool grad, float& cost, float& gx,
-                                float& gy, float& gz) {
+// One penetration term: cost += pen^2 for pen = R - d > 0, and with GRAD the force g e on the first
+// sphere (g = -2 pen / d).  The square root only for pairs within reach: d < R implies
+// e2 < R^2 (1 + 2^-21), so the bound passes every pair with pen > 0.
+template <bool GRAD>
+__device__ inline bool clr_term(float ex, float ey, float ez, float R, float& cost, float& gx, float& gy, float& gz) {
     const float e2 = ex * ex + ey * ey + ez * ez;
     if (!(e2 <= R * R * 1.0001f)) return false;
     const float d = sqrtf(e2);
     const float pen = R - d;
     if (!(pen > 0.f)) return false;
     cost += pen * pen;
-    if (!grad || !(d > 0.f)) return false;
+    if (!GRAD || !(d > 0.f)) return false;
     const float g = -2.f * pen / d;
     gx = g * ex;
     gy = g * ey;
@@ -129,319 +148,301 @@ __device__ inline bool clr_term(float ex, float ey, float ez, float R, bool grad
     return true;
 }
 
+// adds the force g at the point c to the link's sums: moment c x g, force g
+__device__ inline void clr_add(float* tf, float4 c, float gx, float gy, float gz) {
+    atomicAdd(tf, c.y * gz - c.z * gy);
+    atomicAdd(tf + 1, c.z * gx - c.x * gz);
+    atomicAdd(tf + 2, c.x * gy - c.y * gx);
+    atomicAdd(tf + 3, gx);
+    atomicAdd(tf + 4, gy);
+    atomicAdd(tf + 5, gz);
+}
+
+// squared distance from c to the box [lo, hi], and its vector
+__device__ inline float3 clr_box_e(float4 c, float4 lo, float4 hi) {
+    return make_float3(c.x - fminf(fmaxf(c.x, lo.x), hi.x), c.y - fminf(fmaxf(c.y, lo.y), hi.y),
+                       c.z - fminf(fmaxf(c.z, lo.z), hi.z));
+}
+__device__ inline float clr_box_e2(float4 c, float4 lo, float4 hi) {
+    const float3 e = clr_box_e(c, lo, hi);
+    return e.x * e.x + e.y * e.y + e.z * e.z;
+}
+
+// sum over the wave's lanes, in lane 63 (DPP: rows of 16 lanes, then across the rows)
+__device__ inline float wave_sum_f32(float v) {
+    auto add = [&](auto ctrl, int rows) {
+        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, false));
+        (void)rows;
+    };
+    add(std::integral_constant<int, 0x111>{}, 0);  // row_shr 1
+    add(std::integral_constant<int, 0x112>{}, 0);  // row_shr 2
+    add(std::integral_constant<int, 0x114>{}, 0);  // row_shr 4
+    add(std::integral_constant<int, 0x118>{}, 0);  // row_shr 8: lane 15 of each row holds the row's sum
+    return readlane_f(v, 15) + readlane_f(v, 31) + (readlane_f(v, 47) + readlane_f(v, 63));
+}
+
 // The full pair set without culling (the scene's broad phase off): lane = sphere i, every partner
-// j >= sph_lo[i] and every box in turn.  Accumulates the cost; when `grad`, also the forces in W.F
-// (zeroed here).
-__device__ inline float clr_pairs_all(const ArmView& V, const ClrLds& W, float m, bool grad) {
-    const int lane = threadIdx.x;
+// j >= sph_lo[i] and every box in turn.  Returns the lane's share of the cost.
+template <bool GRAD>
+__device__ inline float clr_pairs_all(const ClrK& V, const ClrLds& W, float m) {
+    const int lane = wave_lane();
     const int S = V.S;
-    if (grad) {
-        for (int t = lane; t < 3 * S; t += 64) W.F[t] = 0.f;
-        __syncthreads();
-    }
     float cost = 0.f;
     for (int base = 0; base < S; base += 64) {
         const int i = base + lane;
         const bool act = i < S;
         const float4 ci = W.sph[act ? i : 0];
         float fx = 0.f, fy = 0.f, fz = 0.f;
-        // spheres vs boxes
         for (int b = 0; b < V.nb; ++b) {
-            const float* bx = V.box32 + 8 * b;
-            const float ex = ci.x - fminf(fmaxf(ci.x, bx[0]), bx[4]);
-            const float ey = ci.y - fminf(fmaxf(ci.y, bx[1]), bx[5]);
-            const float ez = ci.z - fminf(fmaxf(ci.z, bx[2]), bx[6]);
-            const float e2 = ex * ex + ey * ey + ez * ez;
-            const float R = m + ci.w;
-            // the square root only for pairs within reach: d < R implies e2 < R^2 (1 + 2^-21),
-            // so the bound below passes every pair with pen > 0, whose terms are unchanged
-            if (!(act && e2 <= R * R * 1.0001f)) continue;
-            const float d = sqrtf(e2);
-            const float pen = R - d;
-            if (pen > 0.f) {
-                cost += pen * pen;
-                if (grad && d > 0.f) {
-                    const float g = -2.f * pen / d;
-                    fx += g * ex;
-                    fy += g * ey;
-                    fz += g * ez;
-                }
+            const float3 e = clr_box_e(ci, V.box32[2 * b], V.box32[2 * b + 1]);
+            float gx, gy, gz;
+            if (act && clr_term<GRAD>(e.x, e.y, e.z, m + ci.w, cost, gx, gy, gz)) {
+                fx += gx;
+                fy += gy;
+                fz += gz;
             }
         }
-        // sphere pairs
         const int lo = act ? V.sph_lo[i] : 0x7fffffff;
         for (int j = V.sph_lo[base]; j < S; ++j) {
             const float4 cj = W.sph[j];
-            const float ex = ci.x - cj.x, ey = ci.y - cj.y, ez = ci.z - cj.z;
-            const float e2 = ex * ex + ey * ey + ez * ez;
-            const float R = m + ci.w + cj.w;
-            if (!(j >= lo && e2 <= R * R * 1.0001f)) continue;  // as above
-            const float d = sqrtf(e2);
-            const float pen = R - d;
-            if (pen > 0.f) {
-                cost += pen * pen;
-                if (grad && d > 0.f) {
-                    const float g = -2.f * pen / d;
-                    fx += g * ex;
-                    fy += g * ey;
-                    fz += g * ez;
-                    atomicAdd(&W.F[3 * j], -g * ex);
-                    atomicAdd(&W.F[3 * j + 1], -g * ey);
-                    atomicAdd(&W.F[3 * j + 2], -g * ez);
-                }
+            float gx, gy, gz;
+            if (j >= lo && clr_term<GRAD>(ci.x - cj.x, ci.y - cj.y, ci.z - cj.z, m + ci.w + cj.w, cost, gx, gy, gz)) {
+                fx += gx;
+                fy += gy;
+                fz += gz;
+                clr_add(W.tf + 6 * W.slink[j], cj, -gx, -gy, -gz);
             }
         }
-        if (grad && act) {
-            atomicAdd(&W.F[3 * i], fx);
-            atomicAdd(&W.F[3 * i + 1], fy);
-            atomicAdd(&W.F[3 * i + 2], fz);
-        }
+        if (GRAD && act) clr_add(W.tf + 6 * W.slink[i], ci, fx, fy, fz);
     }
-    // wave sum
-    W.red[lane] = cost;
-    __syncthreads();
-    for (int off = 32; off > 0; off >>= 1) {
-        if (lane < off) W.red[lane] += W.red[lane + off];
-        __syncthreads();
-    }
-    const float total = W.red[0];
-    __syncthreads();
-    return total;
+    return cost;
 }
 
-// Accumulates the cost of the pair set; when `grad`, also the forces in W.F (zeroed here).
+// The lane's share of the cost of the pair set; with GRAD also the links' forces and moments in W.tf.
 // Terms are nonzero only for pairs within reach, so both parts are culled with the links'
 // bounding spheres first (the triangle inequality: a sphere of link A lies within R_A - r of A's
 // centre, so no pair of two links farther apart than m + R_A + R_B, and no sphere of a link
 // farther than m + R_A from a box, penetrates); the surviving (link, box) and (link, link)
 // candidates are expanded to their spheres, 8 x 8 lanes at a time.  With the scene's broad phase
 // off (V.broadphase = 0) the full pair set is walked instead (clr_pairs_all).
-__device__ inline float clr_pairs(const ArmView& V, const ClrLds& W, float m, bool grad) {
-    if (!V.broadphase) return clr_pairs_all(V, W, m, grad);
-    const int lane = threadIdx.x;
-    const int S = V.S, L = V.L;
-    if (grad)
-        for (int t = lane; t < 3 * S; t += 64) W.F[t] = 0.f;
-    for (int l = lane; l < L; l += 64) {
-        const float* X = W.X + 12 * l;
-        const double* b = V.link_bc64 + 3 * l;
-        const float b0 = (float)b[0], b1 = (float)b[1], b2 = (float)b[2];
-        W.lk[l] = make_float4(X[0] * b0 + X[1] * b1 + X[2] * b2 + X[9], X[3] * b0 + X[4] * b1 + X[5] * b2 + X[10],
-                              X[6] * b0 + X[7] * b1 + X[8] * b2 + X[11], V.link_R32[l]);
-    }
-    __syncthreads();
+template <bool GRAD>
+__device__ inline float clr_pairs(const ClrK& V, const ClrLds& W, float m) {
+    if (!V.broadphase) return clr_pairs_all<GRAD>(V, W, m);
+    const int lane = wave_lane();
+    const int L = V.L;
     float cost = 0.f;
-    const unsigned long long below = (1ull << lane) - 1ull;
     // the spheres of (link, box) candidate `cd` (lane k of its group of 8 takes the link's sphere k)
-    auto sphere_box = [&](int cd, int k) {
+    auto sphere_box = [&](int cd, int k, const float4* box) {
         const int l = cd & 255, b = cd >> 8;
-        const int s = V.link_first[l] + k;
-        if (s >= V.link_first[l + 1]) return;
-        const float4 ci = W.sph[s];
-        const float* bx = V.box32 + 8 * b;
+        const int fc = W.fc[l];
+        if (k >= (fc >> 16)) return;
+        const float4 ci = W.sph[(fc & 0xffff) + k];
+        const float3 e = clr_box_e(ci, box[2 * b], box[2 * b + 1]);
         float gx, gy, gz;
-        if (clr_term(ci.x - fminf(fmaxf(ci.x, bx[0]), bx[4]), ci.y - fminf(fmaxf(ci.y, bx[1]), bx[5]),
-                     ci.z - fminf(fmaxf(ci.z, bx[2]), bx[6]), m + ci.w, grad, cost, gx, gy, gz)) {
-            atomicAdd(&W.F[3 * s], gx);
-            atomicAdd(&W.F[3 * s + 1], gy);
-            atomicAdd(&W.F[3 * s + 2], gz);
-        }
+        if (clr_term<GRAD>(e.x, e.y, e.z, m + ci.w, cost, gx, gy, gz)) clr_add(W.tf + 6 * l, ci, gx, gy, gz);
     };
-    // squared distance from the link sphere's centre to a box [lo, hi]
-    auto box_e2 = [](float4 c, const float* lo, const float* hi) {
-        const float ex = c.x - fminf(fmaxf(c.x, lo[0]), hi[0]);
-        const float ey = c.y - fminf(fmaxf(c.y, lo[1]), hi[1]);
-        const float ez = c.z - fminf(fmaxf(c.z, lo[2]), hi[2]);
-        return ex * ex + ey * ey + ez * ez;
-    };
-    // 1. spheres vs boxes.  Scenes with box clusters (at most 8 boxes each): (link, cluster) pairs
-    //    lane-parallel, the boxes of the candidate clusters 8 lanes per pair, then the spheres of
-    //    the candidate (link, box) pairs 8 lanes per pair; otherwise (link, box) pairs directly.
-    if (V.nclu > 0) {
-        const int nlc = L * V.nclu;
-        for (int t0 = 0; t0 < nlc; t0 += 64) {
-            const int t = t0 + lane;
-            bool cand = false;
-            int code = 0;
-            if (t < nlc) {
-                const int l = t / V.nclu, c = t - l * V.nclu;
-                const float4 lk = W.lk[l];
-                const float R = m + lk.w + CLR_CULL_EPS;
-                cand = V.link_first[l + 1] > V.link_first[l] &&
-                       box_e2(lk, V.clu32 + 8 * c, V.clu32 + 8 * c + 4) <= R * R;
-                code = l | (c << 8);
-            }
+    // 1. spheres vs boxes: links against the box around all obstacles, then, in scenes with box
+    //    clusters (at most 16, of at most 8 boxes), (link, cluster) pairs lane-parallel, the boxes of
+    //    the candidate clusters 8 lanes per pair, the spheres of the candidate (link, box) pairs 8
+    //    lanes per pair; otherwise each link against 64 boxes at a time
+    bool lsurv = false;
+    if (lane < L && (W.fc[lane] >> 16) > 0) {
+        const float4 c = W.lk[lane];
+        const float R = m + c.w + CLR_CULL_EPS;
+        lsurv = clr_box_e2(c, make_float4(V.bb_lo[0], V.bb_lo[1], V.bb_lo[2], 0.f),
+                           make_float4(V.bb_hi[0], V.bb_hi[1], V.bb_hi[2], 0.f)) <= R * R && V.nb > 0;
+    }
+    const unsigned long long smask = __ballot(lsurv);
+    if (V.nclu > 0 && smask) {
+        if (lsurv) W.cand2[lanes_below(smask)] = lane;
+        wave_sync();
+        const int nsv = __popcll(smask);
+        const int lgKG = V.nclu <= 8 ? 3 : 4;  // lanes per link: 8 or 16
+        const int per = 64 >> lgKG;
+        for (int k0 = 0; k0 < nsv; k0 += per) {
+            const int k = k0 + (lane >> lgKG), cc = lane & ((1 << lgKG) - 1);
+            const bool in = k < nsv && cc < V.nclu;
+            const int l = W.cand2[in ? k : k0];
+            const float4 lk = W.lk[l];
+            const float R = m + lk.w + CLR_CULL_EPS;
+            const int ci = in ? cc : 0;
+            const bool cand = in && clr_box_e2(lk, W.clu[2 * ci], W.clu[2 * ci + 1]) <= R * R;
             const unsigned long long mk = __ballot(cand);
             if (mk == 0ull) continue;  // wave-uniform
-            if (cand) W.cand[__popcll(mk & below)] = code;
-            __syncthreads();
+            if (cand) W.cand[lanes_below(mk)] = l | (cc << 8);
+            wave_sync();
             const int nA = __popcll(mk);
             for (int a0 = 0; a0 < nA; a0 += 8) {  // 8 (link, cluster) candidates x 8 boxes
                 const int g = lane >> 3, j = lane & 7;
                 const bool ga = a0 + g < nA;
                 const int c2 = W.cand[ga ? a0 + g : a0];
-                const int l = c2 & 255, cl = c2 >> 8;
-                const int first = __float_as_int(V.clu32[8 * cl + 3]), count = __float_as_int(V.clu32[8 * cl + 7]);
+                const int l2 = c2 & 255, cl = c2 >> 8;
+                const int first = __float_as_int(W.clu[2 * cl].w), count = __float_as_int(W.clu[2 * cl + 1].w);
                 const bool act = ga && j < count;
-                const int b = first + (act ? j : 0);
-                const float4 lk = W.lk[l];
-                const float R = m + lk.w + CLR_CULL_EPS;
-                const bool bc = act && box_e2(lk, V.box32 + 8 * b, V.box32 + 8 * b + 4) <= R * R;
-                const unsigned long long bm = __ballot(bc);
-                if (bm == 0ull) continue;  // wave-uniform
-                if (bc) W.cand2[__popcll(bm & below)] = l | (b << 8);
-                __syncthreads();
-                const int nB = __popcll(bm);
-                for (int c0 = 0; c0 < nB; c0 += 8)  // 8 (link, box) candidates x 8 spheres
-                    if (c0 + (lane >> 3) < nB) sphere_box(W.cand2[c0 + (lane >> 3)], lane & 7);
-                __syncthreads();  // W.cand2 is rewritten by the next group
+                const int b = act ? first + j : 0;
+                const float4 lk2 = W.lk[l2];
+                const float R2 = m + lk2.w + CLR_CULL_EPS;
+                const bool bc = act && clr_box_e2(lk2, W.box[2 * b], W.box[2 * b + 1]) <= R2 * R2;
+                unsigned long long bm = __ballot(bc);
+                const int code = l2 | (b << 8);
+                while (bm) {  // 8 (link, box) candidates x 8 spheres: lane group g takes the g-th set lane
+                    int src = -1;
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) {
+                        const int z = bm ? __builtin_ctzll(bm) : -1;
+                        bm &= bm - 1ull;
+                        src = g == t ? z : src;
+                    }
+                    const int cd = __shfl(code, src < 0 ? 0 : src, 64);
+                    if (src >= 0) sphere_box(cd, j, W.box);
+                }
             }
-            __syncthreads();  // W.cand is rewritten by the next round
+            wave_sync();  // W.cand is rewritten by the next round
         }
-    } else {
-        const int nlb = L * V.nb;
-        for (int t0 = 0; t0 < nlb; t0 += 64) {
-            const int t = t0 + lane;
-            bool cand = false;
-            int code = 0;
-            if (t < nlb) {
-                const int l = t / V.nb, b = t - l * V.nb;
-                const float4 lk = W.lk[l];
-                const float R = m + lk.w + CLR_CULL_EPS;
-                cand = V.link_first[l + 1] > V.link_first[l] && box_e2(lk, V.box32 + 8 * b, V.box32 + 8 * b + 4) <= R * R;
-                code = l | (b << 8);
-            }
+    }
+    for (unsigned long long lm = V.nclu > 0 ? 0ull : smask; lm; lm &= lm - 1ull) {
+        const int l = __builtin_ctzll(lm);
+        const float4 lk = W.lk[l];
+        const float R = m + lk.w + CLR_CULL_EPS;
+        for (int b0 = 0; b0 < V.nb; b0 += 64) {
+            const int b = b0 + lane;
+            const int bi = b < V.nb ? b : 0;
+            const bool cand = b < V.nb && clr_box_e2(lk, V.box32[2 * bi], V.box32[2 * bi + 1]) <= R * R;
             const unsigned long long mk = __ballot(cand);
             if (mk == 0ull) continue;  // wave-uniform
-            if (cand) W.cand[__popcll(mk & below)] = code;
-            __syncthreads();
+            if (cand) W.cand[lanes_below(mk)] = l | (b << 8);
+            wave_sync();
             const int n = __popcll(mk);
             for (int c0 = 0; c0 < n; c0 += 8)  // 8 candidates x 8 spheres per round
-                if (c0 + (lane >> 3) < n) sphere_box(W.cand[c0 + (lane >> 3)], lane & 7);
-            __syncthreads();  // W.cand is rewritten by the next round
+                if (c0 + (lane >> 3) < n) sphere_box(W.cand[c0 + (lane >> 3)], lane & 7, V.box32);
+            wave_sync();  // W.cand is rewritten by the next round
         }
     }
     // 2. sphere pairs of the link pairs in the pair set
     for (int p0 = 0; p0 < V.NP; p0 += 64) {
         const int pi = p0 + lane;
-        bool cand = false;
-        int y = 0;
-        if (pi < V.NP) {
-            const int2 pr = V.lpairs2[pi];
-            const float4 A = W.lk[(pr.x >> 8) & 255], B = W.lk[pr.x & 255];
-            const float dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
-            const float R = m + A.w + B.w + CLR_CULL_EPS;
-            cand = dx * dx + dy * dy + dz * dz <= R * R;
-            y = pr.y;
+        const bool in = pi < V.NP;
+        int2 pr;
+        if (V.NP <= ARM_PAIRS_LDS_MAX) {
+            const unsigned long long v = ((lds_cu64*)W.pairs)[in ? pi : p0];
+            pr = make_int2((int)(unsigned)v, (int)(unsigned)(v >> 32));
+        } else {
+            pr = V.lpairs2[in ? pi : p0];
         }
-        const unsigned long long mk = __ballot(cand);
-        if (mk == 0ull) continue;  // wave-uniform
-        if (cand) W.cand[__popcll(mk & below)] = y;
-        __syncthreads();
-        const int n = __popcll(mk);
-        for (int c = 0; c < n; ++c) {  // one link pair per round: lane (i, j) of its 8 x 8 spheres
-            const int yc = W.cand[c];
+        const float4 A = W.lk[(pr.x >> 8) & 255], B = W.lk[pr.x & 255];
+        const float dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
+        const float R = m + A.w + B.w + CLR_CULL_EPS;
+        const bool cand = in && dx * dx + dy * dy + dz * dz <= R * R;
+        unsigned long long mk = __ballot(cand);
+        while (mk) {  // one link pair per round: lane (i, j) of its 8 x 8 spheres
+            const int src = __builtin_ctzll(mk);
+            mk &= mk - 1ull;
+            const int xc = __builtin_amdgcn_readlane(pr.x, src), yc = __builtin_amdgcn_readlane(pr.y, src);
             const int fl = yc & 511, nl = (yc >> 9) & 15, fm = (yc >> 13) & 511, nm = (yc >> 22) & 15;
-            if ((lane >> 3) >= nl || (lane & 7) >= nm) continue;
-            const int i = fl + (lane >> 3), j = fm + (lane & 7);
-            const float4 ci = W.sph[i], cj = W.sph[j];
+            const int i = lane >> 3, j = lane & 7;
+            const bool act = i < nl && j < nm;
+            const float4 ci = W.sph[fl + (act ? i : 0)], cj = W.sph[fm + (act ? j : 0)];
             float gx, gy, gz;
-            if (clr_term(ci.x - cj.x, ci.y - cj.y, ci.z - cj.z, m + ci.w + cj.w, grad, cost, gx, gy, gz)) {
-                atomicAdd(&W.F[3 * i], gx);
-                atomicAdd(&W.F[3 * i + 1], gy);
-                atomicAdd(&W.F[3 * i + 2], gz);
-                atomicAdd(&W.F[3 * j], -gx);
-                atomicAdd(&W.F[3 * j + 1], -gy);
-                atomicAdd(&W.F[3 * j + 2], -gz);
+            if (act && clr_term<GRAD>(ci.x - cj.x, ci.y - cj.y, ci.z - cj.z, m + ci.w + cj.w, cost, gx, gy, gz)) {
+                clr_add(W.tf + 6 * ((xc >> 8) & 255), ci, gx, gy, gz);
+                clr_add(W.tf + 6 * (xc & 255), cj, -gx, -gy, -gz);
             }
         }
-        __syncthreads();
     }
-    // wave sum
-    W.red[lane] = cost;
-    __syncthreads();
-    for (int off = 32; off > 0; off >>= 1) {
-        if (lane < off) W.red[lane] += W.red[lane + off];
-        __syncthreads();
-    }
-    const float total = W.red[0];
-    __syncthreads();
-    return total;
+    return cost;
 }
 
-__global__ void __launch_bounds__(64) k_clearance(ArmView V, const float* q, long long n, float m,
-                                                  const float* grad_cost, float* cost, float* grad_q) {
-    extern __shared__ float lds_clr[];
-    ClrLds W = clr_lds(lds_clr, V);
-    const bool grad = grad_q != nullptr;
-    for (long long r = blockIdx.x; r < n; r += gridDim.x) {
-        const float* qr = q + r * V.D;
-        clr_fk(V, W, qr);
-        const float c = clr_pairs(V, W, m, grad);
-        if (!grad) {
-            if (threadIdx.x == 0) cost[r] = c;
-        } else {
-            __syncthreads();
-            // lane (arm a, joint k): g = z_{k-1} . sum_{s on links >= k} (c_s - o_{k-1}) x f_s
-            //   = z_{k-1} . (T_k - o_{k-1} x F_k), T_k and F_k the sums of c_s x f_s and of f_s
-            //   over the arm's links >= k: per-link sums first (lane per link), then suffix sums
-            const int lane = threadIdx.x;
-            for (int l = lane; l < V.L; l += 64) {
-                float t0 = 0.f, t1 = 0.f, t2 = 0.f, f0 = 0.f, f1 = 0.f, f2 = 0.f;
-                for (int s = V.link_first[l]; s < V.link_first[l + 1]; ++s) {
-                    const float4 c = W.sph[s];
-                    const float a0 = W.F[3 * s], a1 = W.F[3 * s + 1], a2 = W.F[3 * s + 2];
-                    t0 += c.y * a2 - c.z * a1;
-                    t1 += c.z * a0 - c.x * a2;
-                    t2 += c.x * a1 - c.y * a0;
-                    f0 += a0;
-                    f1 += a1;
-                    f2 += a2;
-                }
-                float* tf = W.tf + 6 * l;
-                tf[0] = t0; tf[1] = t1; tf[2] = t2;
-                tf[3] = f0; tf[4] = f1; tf[5] = f2;
-            }
-            __syncthreads();
-            if (lane < V.D) {
-                const int a = lane / V.dof, k = lane % V.dof;
-                float z0, z1, z2, o0, o1, o2;
-                if (k == 0) {
-                    const double* P = V.base + 12 * a;
-                    z0 = (float)P[2]; z1 = (float)P[5]; z2 = (float)P[8];
-                    o0 = (float)P[9]; o1 = (float)P[10]; o2 = (float)P[11];
-                } else {
-                    const float* P = W.X + 12 * (a * V.dof + k - 1);
-                    z0 = P[2]; z1 = P[5]; z2 = P[8];
-                    o0 = P[9]; o1 = P[10]; o2 = P[11];
-                }
-                float T0 = 0.f, T1 = 0.f, T2 = 0.f, F0 = 0.f, F1 = 0.f, F2 = 0.f;
-                for (int l = (a + 1) * V.dof - 1; l >= a * V.dof + k; --l) {
-                    const float* tf = W.tf + 6 * l;
-                    T0 += tf[0]; T1 += tf[1]; T2 += tf[2];
-                    F0 += tf[3]; F1 += tf[4]; F2 += tf[5];
-                }
-                const bool pr = (V.prism >> lane) & 1ull;  // prismatic: d c / d q = z, g = z . F
-                const float g = pr ? z0 * F0 + z1 * F1 + z2 * F2
-                                   : z0 * (T0 - (o1 * F2 - o2 * F1)) + z1 * (T1 - (o2 * F0 - o0 * F2)) +
-                                         z2 * (T2 - (o0 * F1 - o1 * F0));
-                grad_q[r * V.D + lane] = grad_cost[r] * g;
-            }
-        }
-        __syncthreads();
+template <bool GRAD, bool CHAIN>
+__global__ void __launch_bounds__(64 * CLR_MAX_NW, 4) k_clearance(ClrK V, const float* q, long long n, float m,
+                                                                  const float* grad_cost, float* cost, float* grad_q) {
+    extern __shared__ float4 lds_clr[];
+    {
+        const int n16 = V.img_bytes >> 4;
+        for (int i = threadIdx.x; i < n16; i += blockDim.x) lds_clr[i] = V.img[i];
     }
+    __syncthreads();
+    const ClrLds W = clr_lds((unsigned char*)lds_clr, V);
+    const int lane = wave_lane(), nw = blockDim.x >> 6;
+    const long long waves = (long long)gridDim.x * nw, w0 = (long long)blockIdx.x * nw + (threadIdx.x >> 6);
+    const int per = n > waves ? 2 : 1;  // waypoints per turn: small batches one per wave
+    for (long long r0 = w0 * per; r0 < n; r0 += waves * per) {
+        const int k_end = r0 + per <= n ? per : (int)(n - r0);
+        clr_fk<CHAIN>(V, W, q + r0 * V.D, k_end);
+        for (int k = 0; k < k_end; ++k) {
+            const long long r = r0 + k;
+            const float4* X = W.X + 3 * V.L * k;
+            for (int s = lane; s < V.S; s += 64) W.sph[s] = clr_point(X + 3 * W.slink[s], W.sphL[s]);
+            if (lane < V.L) W.lk[lane] = clr_point(X + 3 * lane, W.lbc[lane]);
+            if (GRAD)
+                for (int t = lane; t < 6 * V.L; t += 64) W.tf[t] = 0.f;
+            wave_sync();
+            const float c = clr_pairs<GRAD>(V, W, m);
+            if (cost) {
+                const float total = wave_sum_f32(c);
+                if (lane == 0) cost[r] = total;
+            }
+            if (GRAD) {
+                wave_sync();
+                // lane (arm a, joint k): g = z_{k-1} . sum_{s on links >= k} (c_s - o_{k-1}) x f_s
+                //   = z_{k-1} . (T_k - o_{k-1} x F_k), T_k and F_k the sums of c_s x f_s and of f_s
+                //   over the arm's links >= k
+                if (lane < V.D) {
+                    const int a = lane / V.dof, kj = lane - a * V.dof;
+                    const float4* P = kj == 0 ? W.base + 3 * a : X + 3 * (lane - 1);
+                    const float4 p0 = P[0], p1 = P[1], p2 = P[2];
+                    const float z0 = p0.z, z1 = p1.z, z2 = p2.z, o0 = p0.w, o1 = p1.w, o2 = p2.w;
+                    float T0 = 0.f, T1 = 0.f, T2 = 0.f, F0 = 0.f, F1 = 0.f, F2 = 0.f;
+                    for (int l = (a + 1) * V.dof - 1; l >= lane; --l) {
+                        const float2* tf = (const float2*)(W.tf + 6 * l);
+                        const float2 u = tf[0], v = tf[1], x = tf[2];
+                        T0 += u.x; T1 += u.y; T2 += v.x;
+                        F0 += v.y; F1 += x.x; F2 += x.y;
+                    }
+                    const bool pr = CHAIN && ((V.prism >> lane) & 1ull);  // prismatic: g = z . F
+                    const float g = pr ? z0 * F0 + z1 * F1 + z2 * F2
+                                       : z0 * (T0 - (o1 * F2 - o2 * F1)) + z1 * (T1 - (o2 * F0 - o0 * F2)) +
+                                             z2 * (T2 - (o0 * F1 - o1 * F0));
+                    grad_q[r * V.D + lane] = grad_cost[r] * g;
+                }
+            }
+            wave_sync();  // the wave's LDS is rewritten for the next waypoint
+        }
+    }
+}
+
+// waves per workgroup and workgroups per CU: the most resident waves in 160 KiB of LDS, 16 at most
+// (4 per SIMD, the kernels' register budget)
+struct ClrShape {
+    int nw, wgs;
+    size_t lds;
+};
+ClrShape clr_shape(const ClrK& K) {
+    ClrShape b = {0, 0, 0};
+    for (int nw = 1; nw <= CLR_MAX_NW; ++nw) {
+        const size_t lds = (size_t)K.img_bytes + (size_t)nw * clr_wave_bytes(K.D, K.L, K.S);
+        if (lds > 163840) break;
+        const int fit = (int)(163840 / lds), wgs = fit < 16 / nw ? fit : 16 / nw;
+        if (wgs * nw > b.nw * b.wgs) b = {nw, wgs, lds};
+    }
+    return b;
 }
 
 }  // namespace
 
-size_t clearance_lds_bytes(const ArmView& V) {
-    return sizeof(float) * (2 * V.D + 12 * V.L) + 16 + sizeof(float4) * V.S + sizeof(float) * 3 * V.S +
-           sizeof(float) * 64 + 16 + sizeof(float4) * V.L + sizeof(int) * 64 + sizeof(float) * 6 * V.L +
-           sizeof(int) * 64;
-}
-
 void launch_clearance(const SceneRec& sc, const float* q, long long n, float margin,
                       const float* grad_cost, float* cost, float* grad_q, hipStream_t st) {
-    long long g = n < 65536 ? n : 65536;
-    k_clearance<<<(int)g, 64, clearance_lds_bytes(sc.arm), st>>>(sc.arm, q, n, margin, grad_cost, cost, grad_q);
+    ClrK K = sc.clr;
+    K.broadphase = sc.arm.broadphase;
+    const ClrShape b = clr_shape(K);
+    const long long waves = (long long)b.nw * b.wgs * mrcc_internal::device_cus();
+    const int blocks = (int)(((n < waves ? n : waves) + b.nw - 1) / b.nw);
+#define MRCC_CLR(G, C) k_clearance<G, C><<<blocks, 64 * b.nw, b.lds, st>>>(K, q, n, margin, grad_cost, cost, grad_q)
+    if (grad_q) {
+        if (K.chain) MRCC_CLR(true, true);
+        else MRCC_CLR(true, false);
+    } else {
+        if (K.chain) MRCC_CLR(false, true);
+        else MRCC_CLR(false, false);
+    }
+#undef MRCC_CLR
 }

@@ -4,6 +4,37 @@
 #include "../../include/mrcc.h"
 #include "evaluators.hpp"
 
+// An arm scene as the clearance kernels see it: scalars and the binary32 tables as one image that a
+// workgroup stages in LDS (clr_layout); tables too large for it are read from global memory.
+struct ClrK {
+    int na, dof, D, L, S, nb, NP, nclu, chain, broadphase;
+    unsigned long long prism;
+    float bb_lo[3], bb_hi[3];
+    const float4* img;
+    int img_bytes;
+    const float4* box32;  // [nb*2] lo, hi
+    const int2* lpairs2;  // [NP]
+    const int* sph_lo;    // [S]
+};
+struct ClrLayout {
+    int o_joint, o_base, o_sph, o_lbc, o_fc, o_slink, o_box, o_clu, o_pairs, bytes;
+};
+__host__ __device__ inline ClrLayout clr_layout(int L, int na, int nb, int S, int NP, int nclu, int chain) {
+    ClrLayout o;
+    int b = 0;
+    o.o_joint = b;  b += 16 * (chain ? 3 : 1) * L;  // d a cos(alpha) sin(alpha), or the rows of C
+    o.o_base = b;   b += 48 * na;                   // rows R0 R1 R2 t
+    o.o_sph = b;    b += 16 * S;                    // centre in the link frame, radius
+    o.o_lbc = b;    b += 16 * L;                    // bounding-sphere centre in the link frame, radius
+    o.o_fc = b;     b += align16(4 * L);            // first sphere | count << 16
+    o.o_slink = b;  b += align16(4 * S);            // link of each sphere
+    o.o_box = b;    b += (nclu > 0 ? 32 * nb : 0);
+    o.o_clu = b;    b += 32 * nclu;
+    o.o_pairs = b;  b += (NP <= ARM_PAIRS_LDS_MAX ? align16(8 * NP) : 0);
+    o.bytes = b;
+    return o;
+}
+
 // A scene as held by the library: the kind, its device view and the device allocation behind it.
 struct SceneRec {
     int kind;
@@ -14,6 +45,7 @@ struct SceneRec {
     PlanarView planar;
     ArmView arm;          // every array of an arm scene (clearance and kinematics kernels)
     ArmK armk;            // the edge and configuration kernels' view of the same scene
+    ClrK clr;             // the clearance kernels' view
     size_t arm_lds;       // dynamic LDS bytes of the arm kernels (arm_nw waves per workgroup)
     size_t arm_lds1;      // dynamic LDS bytes of an arm kernel with one wave per workgroup
     int arm_nw;           // waves per workgroup of the arm kernels

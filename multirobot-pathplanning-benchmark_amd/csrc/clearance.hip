@@ -148,7 +148,14 @@ __device__ inline bool clr_term(float ex, float ey, float ez, float R, float& co
     return true;
 }
 
-// adds the force g at the point c to the link's sums: moment c x g, force g
+// Force and moment sums of the links, lane (arm a, joint k) = 8 a + k holding link (a, k).  Summed in
+// registers by lane shifts: LDS atomics of the lanes of one candidate all go to the same two links,
+// one after the other (262,144 waypoints: 694 us with them).
+struct ClrSums {
+    float T0, T1, T2, F0, F1, F2;
+};
+
+// adds the force g at the point c to the link's sums in LDS (the walk over the full pair set)
 __device__ inline void clr_add(float* tf, float4 c, float gx, float gy, float gz) {
     atomicAdd(tf, c.y * gz - c.z * gy);
     atomicAdd(tf + 1, c.z * gx - c.x * gz);
@@ -156,6 +163,21 @@ __device__ inline void clr_add(float* tf, float4 c, float gx, float gy, float gz
     atomicAdd(tf + 3, gx);
     atomicAdd(tf + 4, gy);
     atomicAdd(tf + 5, gz);
+}
+
+template <int CTRL, int ROWS = 0xf>
+__device__ inline float dpp_add(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+}
+// sum over the lane's group of 8, in the group's last lane (row_shr 1, 2, 4; lanes whose source lies
+// in the group before take it too: their value is not used)
+__device__ inline float group8_sum(float v) { return dpp_add<0x114>(dpp_add<0x112>(dpp_add<0x111>(v))); }
+// sum over the wave, wave-uniform (rows of 16, then row_bcast 15 and 31 across the rows)
+__device__ inline float wave_sum_f32(float v) {
+    v = dpp_add<0x118>(group8_sum(v));
+    v = dpp_add<0x142, 0xa>(v);
+    v = dpp_add<0x143, 0xc>(v);
+    return readlane_f(v, 63);
 }
 
 // squared distance from c to the box [lo, hi], and its vector
@@ -168,17 +190,16 @@ __device__ inline float clr_box_e2(float4 c, float4 lo, float4 hi) {
     return e.x * e.x + e.y * e.y + e.z * e.z;
 }
 
-// sum over the wave's lanes, in lane 63 (DPP: rows of 16 lanes, then across the rows)
-__device__ inline float wave_sum_f32(float v) {
-    auto add = [&](auto ctrl, int rows) {
-        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, false));
-        (void)rows;
-    };
-    add(std::integral_constant<int, 0x111>{}, 0);  // row_shr 1
-    add(std::integral_constant<int, 0x112>{}, 0);  // row_shr 2
-    add(std::integral_constant<int, 0x114>{}, 0);  // row_shr 4
-    add(std::integral_constant<int, 0x118>{}, 0);  // row_shr 8: lane 15 of each row holds the row's sum
-    return readlane_f(v, 15) + readlane_f(v, 31) + (readlane_f(v, 47) + readlane_f(v, 63));
+// sum of the lane's value and those of the lanes after it in its group of 8 (DPP row_shl; the last
+// lanes of a group take nothing from the next group)
+__device__ inline float clr_suffix8(float v) {
+    const int k = threadIdx.x & 7;
+    float u = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x101, 0xf, 0xf, false));
+    v += k < 7 ? u : 0.f;
+    u = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x102, 0xf, 0xf, false));
+    v += k < 6 ? u : 0.f;
+    u = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x104, 0xf, 0xf, false));
+    return v + (k < 4 ? u : 0.f);
 }
 
 // The full pair set without culling (the scene's broad phase off): lane = sphere i, every partner
@@ -226,20 +247,38 @@ __device__ inline float clr_pairs_all(const ClrK& V, const ClrLds& W, float m) {
 // candidates are expanded to their spheres, 8 x 8 lanes at a time.  With the scene's broad phase
 // off (V.broadphase = 0) the full pair set is walked instead (clr_pairs_all).
 template <bool GRAD>
-__device__ inline float clr_pairs(const ClrK& V, const ClrLds& W, float m) {
-    if (!V.broadphase) return clr_pairs_all<GRAD>(V, W, m);
+__device__ inline float clr_pairs(const ClrK& V, const ClrLds& W, float m, int my_link, ClrSums& S) {
     const int lane = wave_lane();
     const int L = V.L;
     float cost = 0.f;
     // the spheres of (link, box) candidate `cd` (lane k of its group of 8 takes the link's sphere k)
-    auto sphere_box = [&](int cd, int k, const float4* box) {
+    auto sphere_box = [&](bool act, int cd, int k, const float4* box) {
         const int l = cd & 255, b = cd >> 8;
         const int fc = W.fc[l];
-        if (k >= (fc >> 16)) return;
-        const float4 ci = W.sph[(fc & 0xffff) + k];
+        act = act && k < (fc >> 16);
+        const float4 ci = W.sph[(fc & 0xffff) + (act ? k : 0)];
         const float3 e = clr_box_e(ci, box[2 * b], box[2 * b + 1]);
-        float gx, gy, gz;
-        if (clr_term<GRAD>(e.x, e.y, e.z, m + ci.w, cost, gx, gy, gz)) clr_add(W.tf + 6 * l, ci, gx, gy, gz);
+        float gx = 0.f, gy = 0.f, gz = 0.f;
+        const bool f = act && clr_term<GRAD>(e.x, e.y, e.z, m + ci.w, cost, gx, gy, gz);
+        if constexpr (GRAD) {
+            unsigned long long mk = __ballot(f);
+            if (mk == 0ull) return;  // wave-uniform
+            if (!f) gx = gy = gz = 0.f;
+            const float t0 = group8_sum(ci.y * gz - ci.z * gy), t1 = group8_sum(ci.z * gx - ci.x * gz),
+                        t2 = group8_sum(ci.x * gy - ci.y * gx), f0 = group8_sum(gx), f1 = group8_sum(gy),
+                        f2 = group8_sum(gz);
+            while (mk) {  // the groups with a force
+                const int g = __builtin_ctzll(mk) >> 3, last = 8 * g + 7;
+                mk &= ~(255ull << (8 * g));
+                const float w = __builtin_amdgcn_readlane(l, last) == my_link ? 1.f : 0.f;
+                S.T0 += w * readlane_f(t0, last);
+                S.T1 += w * readlane_f(t1, last);
+                S.T2 += w * readlane_f(t2, last);
+                S.F0 += w * readlane_f(f0, last);
+                S.F1 += w * readlane_f(f1, last);
+                S.F2 += w * readlane_f(f2, last);
+            }
+        }
     };
     // 1. spheres vs boxes: links against the box around all obstacles, then, in scenes with box
     //    clusters (at most 16, of at most 8 boxes), (link, cluster) pairs lane-parallel, the boxes of
@@ -294,7 +333,7 @@ __device__ inline float clr_pairs(const ClrK& V, const ClrLds& W, float m) {
                         src = g == t ? z : src;
                     }
                     const int cd = __shfl(code, src < 0 ? 0 : src, 64);
-                    if (src >= 0) sphere_box(cd, j, W.box);
+                    sphere_box(src >= 0, src >= 0 ? cd : 0, j, W.box);
                 }
             }
             wave_sync();  // W.cand is rewritten by the next round
@@ -313,8 +352,10 @@ __device__ inline float clr_pairs(const ClrK& V, const ClrLds& W, float m) {
             if (cand) W.cand[lanes_below(mk)] = l | (b << 8);
             wave_sync();
             const int n = __popcll(mk);
-            for (int c0 = 0; c0 < n; c0 += 8)  // 8 candidates x 8 spheres per round
-                if (c0 + (lane >> 3) < n) sphere_box(W.cand[c0 + (lane >> 3)], lane & 7, V.box32);
+            for (int c0 = 0; c0 < n; c0 += 8) {  // 8 candidates x 8 spheres per round
+                const int k = c0 + (lane >> 3);
+                sphere_box(k < n, W.cand[k < n ? k : c0], lane & 7, V.box32);
+            }
             wave_sync();  // W.cand is rewritten by the next round
         }
     }
@@ -342,10 +383,21 @@ __device__ inline float clr_pairs(const ClrK& V, const ClrLds& W, float m) {
             const int i = lane >> 3, j = lane & 7;
             const bool act = i < nl && j < nm;
             const float4 ci = W.sph[fl + (act ? i : 0)], cj = W.sph[fm + (act ? j : 0)];
-            float gx, gy, gz;
-            if (act && clr_term<GRAD>(ci.x - cj.x, ci.y - cj.y, ci.z - cj.z, m + ci.w + cj.w, cost, gx, gy, gz)) {
-                clr_add(W.tf + 6 * ((xc >> 8) & 255), ci, gx, gy, gz);
-                clr_add(W.tf + 6 * (xc & 255), cj, -gx, -gy, -gz);
+            float gx = 0.f, gy = 0.f, gz = 0.f;
+            const bool f = act && clr_term<GRAD>(ci.x - cj.x, ci.y - cj.y, ci.z - cj.z, m + ci.w + cj.w, cost, gx, gy, gz);
+            if constexpr (GRAD) {
+                if (__ballot(f)) {
+                    if (!f) gx = gy = gz = 0.f;
+                    // the opposite force on the second link; c_i x g = c_j x g, since the force acts
+                    // along the line of the centres
+                    const float w = ((xc >> 8) & 255) == my_link ? 1.f : ((xc & 255) == my_link ? -1.f : 0.f);
+                    S.T0 += w * wave_sum_f32(ci.y * gz - ci.z * gy);
+                    S.T1 += w * wave_sum_f32(ci.z * gx - ci.x * gz);
+                    S.T2 += w * wave_sum_f32(ci.x * gy - ci.y * gx);
+                    S.F0 += w * wave_sum_f32(gx);
+                    S.F1 += w * wave_sum_f32(gy);
+                    S.F2 += w * wave_sum_f32(gz);
+                }
             }
         }
     }
@@ -371,38 +423,47 @@ __global__ void __launch_bounds__(64 * CLR_MAX_NW, 4) k_clearance(ClrK V, const 
         for (int k = 0; k < k_end; ++k) {
             const long long r = r0 + k;
             const float4* X = W.X + 3 * V.L * k;
+            const float gw = GRAD ? grad_cost[r] : 0.f;  // in flight during the pairs
             for (int s = lane; s < V.S; s += 64) W.sph[s] = clr_point(X + 3 * W.slink[s], W.sphL[s]);
             if (lane < V.L) W.lk[lane] = clr_point(X + 3 * lane, W.lbc[lane]);
-            if (GRAD)
-                for (int t = lane; t < 6 * V.L; t += 64) W.tf[t] = 0.f;
-            wave_sync();
-            const float c = clr_pairs<GRAD>(V, W, m);
+            // lane (arm a, joint kj), 8 lanes per arm
+            const int a = lane >> 3, kj = lane & 7;
+            const bool in = a < V.na && kj < V.dof;
+            const int l = in ? a * V.dof + kj : 0;
+            ClrSums S = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            float c;
+            if (V.broadphase) {
+                wave_sync();
+                c = clr_pairs<GRAD>(V, W, m, in ? l : -1, S);
+            } else {
+                if (GRAD)
+                    for (int t = lane; t < 6 * V.L; t += 64) W.tf[t] = 0.f;
+                wave_sync();
+                c = clr_pairs_all<GRAD>(V, W, m);
+                wave_sync();
+                const float* tf = W.tf + 6 * l;
+                if (GRAD && in) S = {tf[0], tf[1], tf[2], tf[3], tf[4], tf[5]};
+            }
             if (cost) {
                 const float total = wave_sum_f32(c);
                 if (lane == 0) cost[r] = total;
             }
             if (GRAD) {
-                wave_sync();
-                // lane (arm a, joint k): g = z_{k-1} . sum_{s on links >= k} (c_s - o_{k-1}) x f_s
-                //   = z_{k-1} . (T_k - o_{k-1} x F_k), T_k and F_k the sums of c_s x f_s and of f_s
-                //   over the arm's links >= k
-                if (lane < V.D) {
-                    const int a = lane / V.dof, kj = lane - a * V.dof;
-                    const float4* P = kj == 0 ? W.base + 3 * a : X + 3 * (lane - 1);
-                    const float4 p0 = P[0], p1 = P[1], p2 = P[2];
-                    const float z0 = p0.z, z1 = p1.z, z2 = p2.z, o0 = p0.w, o1 = p1.w, o2 = p2.w;
-                    float T0 = 0.f, T1 = 0.f, T2 = 0.f, F0 = 0.f, F1 = 0.f, F2 = 0.f;
-                    for (int l = (a + 1) * V.dof - 1; l >= lane; --l) {
-                        const float2* tf = (const float2*)(W.tf + 6 * l);
-                        const float2 u = tf[0], v = tf[1], x = tf[2];
-                        T0 += u.x; T1 += u.y; T2 += v.x;
-                        F0 += v.y; F1 += x.x; F2 += x.y;
-                    }
-                    const bool pr = CHAIN && ((V.prism >> lane) & 1ull);  // prismatic: g = z . F
+                // g of joint k = z_{k-1} . sum over spheres on links >= k
+                // of (c_s - o_{k-1}) x f_s = z_{k-1} . (T_k - o_{k-1} x F_k), T_k and F_k the sums of
+                // c_s x f_s and of f_s over the arm's links >= k (suffix sums by lane shifts)
+                const float T0 = clr_suffix8(S.T0), T1 = clr_suffix8(S.T1), T2 = clr_suffix8(S.T2),
+                            F0 = clr_suffix8(S.F0), F1 = clr_suffix8(S.F1), F2 = clr_suffix8(S.F2);
+                if (in) {
+                    const float4* P = kj == 0 ? W.base + 3 * a : X + 3 * (l - 1);
+                    const float2* P2 = (const float2*)P;  // (R0 R1) (R2 t) per row
+                    const float2 p0 = P2[1], p1 = P2[3], p2 = P2[5];
+                    const float z0 = p0.x, z1 = p1.x, z2 = p2.x, o0 = p0.y, o1 = p1.y, o2 = p2.y;
+                    const bool pr = CHAIN && ((V.prism >> l) & 1ull);  // prismatic: g = z . F
                     const float g = pr ? z0 * F0 + z1 * F1 + z2 * F2
                                        : z0 * (T0 - (o1 * F2 - o2 * F1)) + z1 * (T1 - (o2 * F0 - o0 * F2)) +
                                              z2 * (T2 - (o0 * F1 - o1 * F0));
-                    grad_q[r * V.D + lane] = grad_cost[r] * g;
+                    grad_q[r * V.D + l] = gw * g;
                 }
             }
             wave_sync();  // the wave's LDS is rewritten for the next waypoint

@@ -272,6 +272,14 @@ int mrcc_clearance_forward(const mrcc_scene* scene, const float* q, int64_t n, i
 int mrcc_clearance_backward(const mrcc_scene* scene, const float* q, int64_t n, int32_t dim, float margin,
                             const float* grad_cost, float* grad_q, void* stream);
 
+/* Both in one pass: cost[r] and dcost_dq[r][k] = d cost[r] / d q[r][k] (mrcc_clearance_backward with
+ * grad_cost = 1), for callers that will want the gradient of this cost. */
+int mrcc_clearance_forward_grad(const mrcc_scene* scene, const float* q, int64_t n, int32_t dim, float margin,
+                                float* cost, float* dcost_dq, void* stream);
+/* out[r][k] = w[r] * x[r][k] (device float, rows contiguous of dim): the chain rule from dcost_dq to
+ * the gradient of a function of the costs. */
+int mrcc_scale_rows(const float* x, const float* w, int64_t n, int32_t dim, float* out, void* stream);
+
 /* ---- configuration-pair costs and distances (device) ------------------------------------- */
 /* The planners' metric functions (core/configuration.py):
  *   batch_config_cost / _batch_config_cost_impl  :437-510 (config_cost :352-363)

@@ -1,7 +1,10 @@
 """Differentiable clearance cost of arm scenes and the gradient path-repair step.
 
 ``clearance_cost(scene, q, margin)`` is a ``torch.autograd.Function`` over libmrcc's forward
-(``mrcc_clearance_forward``) and hand-written backward (``mrcc_clearance_backward``, FK recomputed):
+(``mrcc_clearance_forward``) and hand-written gradient.  When ``q`` needs a gradient, cost and
+d cost / d q come from one pass (``mrcc_clearance_forward_grad``) and the backward scales the rows
+(``mrcc_scale_rows``); ``mrcc_clearance_backward`` is the separate backward of the C interface, which
+recomputes the kinematics:
   cost(q) = sum max(0, m + r_i + r_j - |c_i - c_j|)^2 + sum max(0, m + r_i - dist(c_i, box))^2
 over the pair set of the boolean check, in binary32.
 
@@ -38,30 +41,33 @@ class _ClearanceFn:
 
             class ClearanceCost(torch.autograd.Function):
                 @staticmethod
-                def forward(ctx, q, scene, margin):
+                def forward(ctx, q, scene, margin, need_grad):
                     q = q.contiguous()
-                    n = q.shape[0]
+                    n, D = q.shape
                     cost = torch.empty(n, dtype=torch.float32, device=q.device)
                     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-                    check(lib().mrcc_clearance_forward(scene.handle, ctypes.c_void_p(q.data_ptr()), n, q.shape[1],
-                                                       ctypes.c_float(margin), ctypes.c_void_p(cost.data_ptr()),
-                                                       st))
-                    ctx.save_for_backward(q)
                     ctx.scene = scene
-                    ctx.margin = margin
+                    if not need_grad:
+                        check(lib().mrcc_clearance_forward(scene.handle, q.data_ptr(), n, D, margin, cost.data_ptr(),
+                                                           st))
+                        return cost
+                    # cost and gradient share the kinematics and the pairs in reach: one pass for both
+                    dq = torch.empty_like(q)
+                    check(lib().mrcc_clearance_forward_grad(scene.handle, q.data_ptr(), n, D, margin, cost.data_ptr(),
+                                                            dq.data_ptr(), st))
+                    ctx.save_for_backward(q, dq)
                     return cost
 
                 @staticmethod
+                @torch.autograd.function.once_differentiable
                 def backward(ctx, grad_cost):
-                    (q,) = ctx.saved_tensors
+                    q, dq = ctx.saved_tensors
                     g = grad_cost.contiguous().to(torch.float32)
                     grad_q = torch.empty_like(q)
                     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-                    check(lib().mrcc_clearance_backward(ctx.scene.handle, ctypes.c_void_p(q.data_ptr()), q.shape[0],
-                                                        q.shape[1], ctypes.c_float(ctx.margin),
-                                                        ctypes.c_void_p(g.data_ptr()),
-                                                        ctypes.c_void_p(grad_q.data_ptr()), st))
-                    return grad_q, None, None
+                    check(lib().mrcc_scale_rows(dq.data_ptr(), g.data_ptr(), q.shape[0], q.shape[1],
+                                                grad_q.data_ptr(), st))
+                    return grad_q, None, None, None
 
             cls.cls = ClearanceCost
         return cls.cls
@@ -76,7 +82,8 @@ def clearance_cost(scene, q, margin: float = 0.02):
         raise ValueError(f"clearance_cost: rows of {q.shape[-1]} coordinates, the scene has D = {scene.D}")
     shape = q.shape[:-1]
     flat = q.reshape(-1, q.shape[-1])
-    return _ClearanceFn.get().apply(flat, scene, float(margin)).reshape(shape)
+    need_grad = torch.is_grad_enabled() and flat.requires_grad
+    return _ClearanceFn.get().apply(flat, scene, float(margin), need_grad).reshape(shape)
 
 
 def validate_paths(env, paths: np.ndarray, modes=None) -> np.ndarray:

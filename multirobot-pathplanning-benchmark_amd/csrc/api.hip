@@ -1586,6 +1586,29 @@ int mrcc_clearance_backward(const mrcc_scene* scene, const float* q, int64_t n, 
     return MRCC_OK;
 }
 
+int mrcc_clearance_forward_grad(const mrcc_scene* scene, const float* q, int64_t n, int32_t dim, float margin,
+                                float* cost, float* dcost_dq, void* stream) {
+    CHECK_INJECT();
+    if (!scene || (!q && n) || (!cost && n) || (!dcost_dq && n)) return fail(MRCC_ERR_INVALID, "null argument");
+    const SceneRec* sc = rec_of(scene);
+    if (sc->kind != KIND_ARMS) return fail(MRCC_ERR_UNSUPPORTED, "clearance needs an arm scene");
+    if (dim != sc->D) return fail(MRCC_ERR_INVALID, "rows of %d coordinates, the scene has D = %d", dim, sc->D);
+    if (n <= 0) return MRCC_OK;
+    launch_clearance(*sc, q, n, margin, nullptr, cost, dcost_dq, (hipStream_t)stream);
+    HIP_OK(hipGetLastError());
+    return MRCC_OK;
+}
+
+int mrcc_scale_rows(const float* x, const float* w, int64_t n, int32_t dim, float* out, void* stream) {
+    CHECK_INJECT();
+    if (n < 0 || dim < 1) return fail(MRCC_ERR_INVALID, "n < 0 or dim < 1");
+    if (n == 0) return MRCC_OK;
+    if (!x || !w || !out) return fail(MRCC_ERR_INVALID, "null argument");
+    launch_scale_rows(x, w, n, dim, out, (hipStream_t)stream);
+    HIP_OK(hipGetLastError());
+    return MRCC_OK;
+}
+
 int mrcc_config_cost(const double* p, int64_t p_row_stride, const double* q, int64_t q_row_stride,
                      int64_t n, int32_t dim, const int32_t* slices, int32_t n_slices, int32_t metric,
                      int32_t reduction, double w, double* out, void* stream) {

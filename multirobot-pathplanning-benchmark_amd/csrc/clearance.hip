@@ -74,6 +74,7 @@ __device__ inline ClrLds clr_lds(unsigned char* b, const ClrK& V) {
 // (waypoint, arm, row) carries a row through its arm's joints (rows are independent of each other).
 template <bool CHAIN>
 __device__ inline void clr_fk(const ClrK& V, const ClrLds& W, const float* q, int nw) {
+#pragma clang fp contract(off)
     const int lane = wave_lane();
     for (int t = lane; t < nw * V.D; t += 64) {
         float s, c;
@@ -95,19 +96,19 @@ __device__ inline void clr_fk(const ClrK& V, const ClrLds& W, const float* q, in
             float y0, y1, y2, y3;
             if constexpr (CHAIN) {  // A = Rz(q) C (revolute), Tz(q) C (prismatic)
                 const float4 c0 = W.joint[3 * l], c1 = W.joint[3 * l + 1], c2 = W.joint[3 * l + 2];
-                const float u = R0 * cs.x + R1 * cs.y, v = R1 * cs.x - R0 * cs.y;
+                const float u = fmaf(R1, cs.y, R0 * cs.x), v = fmaf(-R0, cs.y, R1 * cs.x);
                 const float q3 = ((V.prism >> l) & 1ull) ? q[w * V.D + l] : 0.f;
-                y0 = u * c0.x + v * c1.x + R2 * c2.x;
-                y1 = u * c0.y + v * c1.y + R2 * c2.y;
-                y2 = u * c0.z + v * c1.z + R2 * c2.z;
-                y3 = u * c0.w + v * c1.w + R2 * (c2.w + q3) + t;
+                y0 = fmaf(R2, c2.x, fmaf(v, c1.x, u * c0.x));
+                y1 = fmaf(R2, c2.y, fmaf(v, c1.y, u * c0.y));
+                y2 = fmaf(R2, c2.z, fmaf(v, c1.z, u * c0.z));
+                y3 = fmaf(R2, c2.w + q3, fmaf(v, c1.w, fmaf(u, c0.w, t)));
             } else {  // A = Rz(q) Tz(d) Tx(a) Rx(alpha)
                 const float4 p = W.joint[l];
-                const float u = R0 * cs.x + R1 * cs.y, v = R1 * cs.x - R0 * cs.y;
+                const float u = fmaf(R1, cs.y, R0 * cs.x), v = fmaf(-R0, cs.y, R1 * cs.x);
                 y0 = u;
-                y1 = v * p.z + R2 * p.w;
-                y2 = R2 * p.z - v * p.w;
-                y3 = u * p.y + R2 * p.x + t;
+                y1 = fmaf(R2, p.w, v * p.z);
+                y2 = fmaf(-v, p.w, R2 * p.z);
+                y3 = fmaf(R2, p.x, fmaf(u, p.y, t));
             }
             W.X[(w * V.L + l) * 3 + r] = make_float4(y0, y1, y2, y3);
             R0 = y0;
@@ -119,11 +120,13 @@ __device__ inline void clr_fk(const ClrK& V, const ClrLds& W, const float* q, in
     wave_sync();
 }
 
+// Fused operations are written out here and in the terms: the kernels with and without the gradient
+// then round the same, and a cost does not depend on whether its gradient is wanted.
+__device__ inline float clr_row(float4 a, float4 l) { return fmaf(a.z, l.z, fmaf(a.y, l.y, fmaf(a.x, l.x, a.w))); }
 __device__ inline float4 clr_point(const float4* X, float4 l) {
-    const float4 a = X[0], b = X[1], c = X[2];
-    return make_float4(a.x * l.x + a.y * l.y + a.z * l.z + a.w, b.x * l.x + b.y * l.y + b.z * l.z + b.w,
-                       c.x * l.x + c.y * l.y + c.z * l.z + c.w, l.w);
+    return make_float4(clr_row(X[0], l), clr_row(X[1], l), clr_row(X[2], l), l.w);
 }
+__device__ inline float clr_sq(float ex, float ey, float ez) { return fmaf(ez, ez, fmaf(ey, ey, ex * ex)); }
 
 // Slack of the link-level cull (metres): covers the binary32 rounding of the link and sphere
 // centres (micrometres) with a wide margin.
@@ -134,12 +137,12 @@ __device__ inline float4 clr_point(const float4* X, float4 l) {
 // e2 < R^2 (1 + 2^-21), so the bound passes every pair with pen > 0.
 template <bool GRAD>
 __device__ inline bool clr_term(float ex, float ey, float ez, float R, float& cost, float& gx, float& gy, float& gz) {
-    const float e2 = ex * ex + ey * ey + ez * ez;
+    const float e2 = clr_sq(ex, ey, ez);
     if (!(e2 <= R * R * 1.0001f)) return false;
     const float d = sqrtf(e2);
     const float pen = R - d;
     if (!(pen > 0.f)) return false;
-    cost += pen * pen;
+    cost = fmaf(pen, pen, cost);
     if (!GRAD || !(d > 0.f)) return false;
     const float g = -2.f * pen / d;
     gx = g * ex;
@@ -165,19 +168,20 @@ __device__ inline void clr_add(float* tf, float4 c, float gx, float gy, float gz
     atomicAdd(tf + 5, gz);
 }
 
-template <int CTRL, int ROWS = 0xf>
+// v + the value of the lane a row shift away (0 beyond the row of 16: one add with a DPP operand)
+template <int CTRL>
 __device__ inline float dpp_add(float v) {
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
 // sum over the lane's group of 8, in the group's last lane (row_shr 1, 2, 4; lanes whose source lies
 // in the group before take it too: their value is not used)
 __device__ inline float group8_sum(float v) { return dpp_add<0x114>(dpp_add<0x112>(dpp_add<0x111>(v))); }
-// sum over the wave, wave-uniform (rows of 16, then row_bcast 15 and 31 across the rows)
+// sum over the lane's row of 16, in the row's last lane
+__device__ inline float row16_sum(float v) { return dpp_add<0x118>(group8_sum(v)); }
+// sum over the wave, wave-uniform
 __device__ inline float wave_sum_f32(float v) {
-    v = dpp_add<0x118>(group8_sum(v));
-    v = dpp_add<0x142, 0xa>(v);
-    v = dpp_add<0x143, 0xc>(v);
-    return readlane_f(v, 63);
+    v = row16_sum(v);
+    return readlane_f(v, 15) + readlane_f(v, 31) + (readlane_f(v, 47) + readlane_f(v, 63));
 }
 
 // squared distance from c to the box [lo, hi], and its vector
@@ -187,19 +191,17 @@ __device__ inline float3 clr_box_e(float4 c, float4 lo, float4 hi) {
 }
 __device__ inline float clr_box_e2(float4 c, float4 lo, float4 hi) {
     const float3 e = clr_box_e(c, lo, hi);
-    return e.x * e.x + e.y * e.y + e.z * e.z;
+    return clr_sq(e.x, e.y, e.z);
 }
 
 // sum of the lane's value and those of the lanes after it in its group of 8 (DPP row_shl; the last
 // lanes of a group take nothing from the next group)
 __device__ inline float clr_suffix8(float v) {
     const int k = threadIdx.x & 7;
-    float u = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x101, 0xf, 0xf, false));
-    v += k < 7 ? u : 0.f;
-    u = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x102, 0xf, 0xf, false));
-    v += k < 6 ? u : 0.f;
-    u = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x104, 0xf, 0xf, false));
-    return v + (k < 4 ? u : 0.f);
+    const float a = dpp_add<0x101>(v), b = k < 7 ? a : v;
+    const float c = dpp_add<0x102>(b), d = k < 6 ? c : b;
+    const float e = dpp_add<0x104>(d);
+    return k < 4 ? e : d;
 }
 
 // The full pair set without culling (the scene's broad phase off): lane = sphere i, every partner
@@ -373,7 +375,7 @@ __device__ inline float clr_pairs(const ClrK& V, const ClrLds& W, float m, int m
         const float4 A = W.lk[(pr.x >> 8) & 255], B = W.lk[pr.x & 255];
         const float dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
         const float R = m + A.w + B.w + CLR_CULL_EPS;
-        const bool cand = in && dx * dx + dy * dy + dz * dz <= R * R;
+        const bool cand = in && clr_sq(dx, dy, dz) <= R * R;
         unsigned long long mk = __ballot(cand);
         while (mk) {  // one link pair per round: lane (i, j) of its 8 x 8 spheres
             const int src = __builtin_ctzll(mk);
@@ -386,17 +388,25 @@ __device__ inline float clr_pairs(const ClrK& V, const ClrLds& W, float m, int m
             float gx = 0.f, gy = 0.f, gz = 0.f;
             const bool f = act && clr_term<GRAD>(ci.x - cj.x, ci.y - cj.y, ci.z - cj.z, m + ci.w + cj.w, cost, gx, gy, gz);
             if constexpr (GRAD) {
-                if (__ballot(f)) {
+                unsigned long long hm = __ballot(f);
+                if (hm) {
                     if (!f) gx = gy = gz = 0.f;
                     // the opposite force on the second link; c_i x g = c_j x g, since the force acts
                     // along the line of the centres
                     const float w = ((xc >> 8) & 255) == my_link ? 1.f : ((xc & 255) == my_link ? -1.f : 0.f);
-                    S.T0 += w * wave_sum_f32(ci.y * gz - ci.z * gy);
-                    S.T1 += w * wave_sum_f32(ci.z * gx - ci.x * gz);
-                    S.T2 += w * wave_sum_f32(ci.x * gy - ci.y * gx);
-                    S.F0 += w * wave_sum_f32(gx);
-                    S.F1 += w * wave_sum_f32(gy);
-                    S.F2 += w * wave_sum_f32(gz);
+                    const float t0 = row16_sum(ci.y * gz - ci.z * gy), t1 = row16_sum(ci.z * gx - ci.x * gz),
+                                t2 = row16_sum(ci.x * gy - ci.y * gx), f0 = row16_sum(gx), f1 = row16_sum(gy),
+                                f2 = row16_sum(gz);
+                    do {  // the rows of 16 lanes with a force
+                        const int row = __builtin_ctzll(hm) >> 4, last = 16 * row + 15;
+                        hm &= ~(65535ull << (16 * row));
+                        S.T0 += w * readlane_f(t0, last);
+                        S.T1 += w * readlane_f(t1, last);
+                        S.T2 += w * readlane_f(t2, last);
+                        S.F0 += w * readlane_f(f0, last);
+                        S.F1 += w * readlane_f(f1, last);
+                        S.F2 += w * readlane_f(f2, last);
+                    } while (hm);
                 }
             }
         }
@@ -423,7 +433,7 @@ __global__ void __launch_bounds__(64 * CLR_MAX_NW, 4) k_clearance(ClrK V, const 
         for (int k = 0; k < k_end; ++k) {
             const long long r = r0 + k;
             const float4* X = W.X + 3 * V.L * k;
-            const float gw = GRAD ? grad_cost[r] : 0.f;  // in flight during the pairs
+            const float gw = GRAD && grad_cost ? grad_cost[r] : 1.f;  // in flight during the pairs
             for (int s = lane; s < V.S; s += 64) W.sph[s] = clr_point(X + 3 * W.slink[s], W.sphL[s]);
             if (lane < V.L) W.lk[lane] = clr_point(X + 3 * lane, W.lbc[lane]);
             // lane (arm a, joint kj), 8 lanes per arm
@@ -488,7 +498,32 @@ ClrShape clr_shape(const ClrK& K) {
     return b;
 }
 
+// out[r][k] = w[r] x[r][k]: the chain rule of a cost whose gradient is already there.  Bound by
+// memory: 16-byte accesses where the rows are a multiple of 4 wide and the tensors aligned.
+template <bool VEC>
+__global__ void __launch_bounds__(256) k_scale_rows(const float* x, const float* w, long long n, int D, float* out) {
+    const long long total = n * D / (VEC ? 4 : 1), step = (long long)gridDim.x * blockDim.x;
+    for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += step) {
+        if constexpr (VEC) {
+            const float c = w[4 * t / D];
+            const float4 v = ((const float4*)x)[t];
+            ((float4*)out)[t] = make_float4(c * v.x, c * v.y, c * v.z, c * v.w);
+        } else {
+            out[t] = w[t / D] * x[t];
+        }
+    }
+}
+
 }  // namespace
+
+void launch_scale_rows(const float* x, const float* w, long long n, int D, float* out, hipStream_t st) {
+    const bool vec = (D & 3) == 0 && (((uintptr_t)x | (uintptr_t)out) & 15) == 0;
+    const long long total = n * D / (vec ? 4 : 1), cap = 16ll * mrcc_internal::device_cus();
+    const long long blocks = (total + 255) / 256;
+    const int g = (int)(blocks < cap ? blocks : cap);
+    if (vec) k_scale_rows<true><<<g, 256, 0, st>>>(x, w, n, D, out);
+    else k_scale_rows<false><<<g, 256, 0, st>>>(x, w, n, D, out);
+}
 
 void launch_clearance(const SceneRec& sc, const float* q, long long n, float margin,
                       const float* grad_cost, float* cost, float* grad_q, hipStream_t st) {

@@ -109,6 +109,7 @@ void launch_arm_fk(const SceneRec& sc, const double* q, long long n, long long r
 void launch_sincos(const double* x, long long n, double* s, double* c, hipStream_t st);
 void launch_clearance(const SceneRec& sc, const float* q, long long n, float margin,
                       const float* grad_cost, float* cost, float* grad_q, hipStream_t st);
+void launch_scale_rows(const float* x, const float* w, long long n, int D, float* out, hipStream_t st);
 
 // configuration-pair costs (cost.hip): row r of the result reduces d = P[r*ps + k] - Q[r*qs + k]
 // (k < D) over the slices [sl[2i], sl[2i+1])

@@ -93,10 +93,47 @@ struct Packer {
 template <class T>
 const T* at(void* base, size_t off) { return (const T*)((unsigned char*)base + off); }
 
-int upload(SceneRec* sc, Packer& P) {
-    HIP_OK(hipMalloc(&sc->dev_mem, P.buf.size()));
+// Uploads the packed tables; `extra` bytes after them (from `*o_extra` on) are left for the device.
+int upload(SceneRec* sc, Packer& P, size_t extra = 0, size_t* o_extra = nullptr) {
+    const size_t off = (P.buf.size() + 255) & ~size_t(255);
+    if (o_extra) *o_extra = off;
+    HIP_OK(hipMalloc(&sc->dev_mem, off + extra));
     HIP_OK(hipMemcpy(sc->dev_mem, P.buf.data(), P.buf.size(), hipMemcpyHostToDevice));
-    sc->dev_bytes = P.buf.size();
+    sc->dev_bytes = off + extra;
+    return MRCC_OK;
+}
+
+// Cells per axis of a plane scene's cell table.  Smaller cells leave fewer obstacles open, and
+// the table (16 bytes a cell and robot: 1 MiB for four robots) has to stay in an XCD's 4 MiB L2.
+#define MRCC_CELLS 128
+
+// Corner and scale of the cell table over obstacles in [lo, hi] for robots reaching `reach` from
+// their centre; no table (n = 0) without obstacles, beyond 65,535 of them (16-bit indices) and
+// beyond MRCC_CELL_EXTENT metres, where binary32 coordinates are too coarse for it.
+#define MRCC_CELL_EXTENT 1.0e5
+CellGrid cell_grid(const double* lo, const double* hi, double reach, long long n_obs, bool ok) {
+    CellGrid C;
+    memset(&C, 0, sizeof(C));
+    if (!ok || n_obs < 1 || n_obs > 65535) return C;
+    double far = reach;
+    for (int k = 0; k < 2; ++k) far = std::max(far, std::max(fabs(lo[k]), fabs(hi[k])));
+    if (!(far < MRCC_CELL_EXTENT)) return C;
+    const double pad = reach + 0.01 * (reach + std::max(hi[0] - lo[0], hi[1] - lo[1])) + 4.0 * cell_slack(far, 0.0);
+    C.x0 = (float)(lo[0] - pad);
+    C.y0 = (float)(lo[1] - pad);
+    C.ix = (float)(MRCC_CELLS / (hi[0] + pad - (double)C.x0));
+    C.iy = (float)(MRCC_CELLS / (hi[1] + pad - (double)C.y0));
+    C.n = MRCC_CELLS;
+    return C;
+}
+size_t cell_bytes(const CellGrid& C, int robots) { return (size_t)robots * C.n * C.n * sizeof(uint4); }
+
+// Builds the table of a scene whose view is complete (on the null stream, and waits for it).
+int build_cells(const SceneRec* sc) {
+    if ((sc->kind == KIND_DISKS ? sc->disk.grid.n : sc->planar.grid.n) == 0) return MRCC_OK;
+    launch_cells(*sc, nullptr);
+    HIP_OK(hipGetLastError());
+    HIP_OK(hipStreamSynchronize(nullptr));
     return MRCC_OK;
 }
 
@@ -768,8 +805,28 @@ int mrcc_scene_create_disks(int n_robots, int robot_dim, const double* robot_rad
     size_t o_r = P.add(r32), o_rrT32 = P.add(rrT32), o_rrT64 = P.add(rrT64), o_sc32 = P.add(sc32),
            o_sc64 = P.add(sc64), o_srT32 = P.add(srT32), o_srT64 = P.add(srT64), o_lo32 = P.add(lo32),
            o_hi32 = P.add(hi32), o_lo64 = P.add(lo64), o_hi64 = P.add(hi64), o_rp32 = P.add(rp2_32),
-           o_rp64 = P.add(rp2_64);
-    int rc = upload(sc, P);
+           o_rp64 = P.add(rp2_64), o_cells = 0;
+    double clo[2] = {1e300, 1e300}, chi[2] = {-1e300, -1e300}, reach = 0.0;
+    bool plane = rd == 2;  // non-negative sizes, finite
+    for (int i = 0; i < nr && plane; ++i) {
+        plane = std::isfinite(robot_radius[i]) && robot_radius[i] >= 0.0;
+        reach = std::max(reach, robot_radius[i]);
+    }
+    for (int o = 0; o < ns && plane; ++o)
+        for (int k = 0; k < 2; ++k) {
+            const double c = sphere_center[2 * o + k], r = sphere_radius[o];
+            plane = plane && std::isfinite(c) && std::isfinite(r) && r >= 0.0;
+            clo[k] = std::min(clo[k], c - r);
+            chi[k] = std::max(chi[k], c + r);
+        }
+    for (int o = 0; o < nq && plane; ++o)
+        for (int k = 0; k < 2; ++k) {
+            plane = plane && std::isfinite(lo64[2 * o + k]) && std::isfinite(hi64[2 * o + k]) && lo64[2 * o + k] <= hi64[2 * o + k];
+            clo[k] = std::min(clo[k], lo64[2 * o + k]);
+            chi[k] = std::max(chi[k], hi64[2 * o + k]);
+        }
+    sc->disk.grid = cell_grid(clo, chi, reach, (long long)ns + nq, plane);
+    int rc = upload(sc, P, cell_bytes(sc->disk.grid, nr), &o_cells);
     if (rc != MRCC_OK) {
         delete box;
         return rc;
@@ -791,6 +848,13 @@ int mrcc_scene_create_disks(int n_robots, int robot_dim, const double* robot_rad
     V.hi64 = at<double>(d, o_hi64);
     V.rp2_32 = at<float>(d, o_rp32);
     V.rp2_64 = at<double>(d, o_rp64);
+    V.grid.rec = at<uint4>(d, o_cells);
+    rc = build_cells(sc);
+    if (rc != MRCC_OK) {
+        (void)hipFree(sc->dev_mem);
+        delete box;
+        return rc;
+    }
     *out = (mrcc_scene*)box;
     return MRCC_OK;
 }
@@ -835,8 +899,25 @@ int mrcc_scene_create_planar_boxes(int n_robots, const double* robot_half_extent
     sc->n_robots = nr;
     (void)hipGetDevice(&sc->device);
     Packer P;
-    size_t o_rh32 = P.add(rh32), o_rh64 = P.add(rh64), o_ob32 = P.add(ob32), o_ob64 = P.add(ob64);
-    int rc = upload(sc, P);
+    size_t o_rh32 = P.add(rh32), o_rh64 = P.add(rh64), o_ob32 = P.add(ob32), o_ob64 = P.add(ob64), o_cells = 0;
+    double clo[2] = {1e300, 1e300}, chi[2] = {-1e300, -1e300}, reach = 0.0;
+    bool plane = true;  // non-negative sizes, finite, unit axes
+    for (int i = 0; i < nr && plane; ++i) {
+        plane = std::isfinite(rh64[2 * i]) && std::isfinite(rh64[2 * i + 1]) && rh64[2 * i] >= 0.0 && rh64[2 * i + 1] >= 0.0;
+        reach = std::max(reach, std::hypot(rh64[2 * i], rh64[2 * i + 1]));
+    }
+    for (int o = 0; o < no && plane; ++o) {
+        const double* b = ob64.data() + 8 * o;
+        for (int k = 0; k < 8; ++k) plane = plane && std::isfinite(b[k]);
+        plane = plane && b[6] >= 0.0 && b[7] >= 0.0 && fabs(obstacle_pose[3 * o + 2]) <= CELL_MAX_YAW;
+        for (int k = 0; k < 2; ++k) {
+            const double e = fabs(b[2 + k]) * b[6] + fabs(b[4 + k]) * b[7];
+            clo[k] = std::min(clo[k], b[k] - e);
+            chi[k] = std::max(chi[k], b[k] + e);
+        }
+    }
+    sc->planar.grid = cell_grid(clo, chi, reach, no, plane);
+    int rc = upload(sc, P, cell_bytes(sc->planar.grid, nr), &o_cells);
     if (rc != MRCC_OK) {
         delete box;
         return rc;
@@ -849,6 +930,13 @@ int mrcc_scene_create_planar_boxes(int n_robots, const double* robot_half_extent
     V.rh64 = at<double>(d, o_rh64);
     V.ob32 = at<float>(d, o_ob32);
     V.ob64 = at<double>(d, o_ob64);
+    V.grid.rec = at<uint4>(d, o_cells);
+    rc = build_cells(sc);
+    if (rc != MRCC_OK) {
+        (void)hipFree(sc->dev_mem);
+        delete box;
+        return rc;
+    }
     *out = (mrcc_scene*)box;
     return MRCC_OK;
 }

@@ -1,0 +1,82 @@
+// cells.hip — the cell table of plane scenes (CellGrid), built on the device when a scene is made.
+#include "engine.hpp"
+
+namespace {
+
+// One thread per (robot, cell): every obstacle's distance to the cell's centre against the robot's
+// circumscribed and inscribed radii, widened by the cell's half diagonal and the slack.
+// Triangle inequality: a centre within `hd` of the cell's centre is at d - hd .. d + hd from the
+// obstacle; beyond the circumscribed radius nothing overlaps (and a separating axis of the two boxes
+// exceeds the gap over sqrt 2), within the inscribed radius the overlap is certain.
+// 128 x 128 cells: 10 us (2 disks, 20 rectangles), 30 us (4 boxes, 100 obstacles), once per scene.
+__device__ inline void cell_fill(CellGrid C, double hd, double slack, int i, double r_in, double r_out, int n_obs,
+                                 int t, const DiskView* D, const PlanarView* P) {
+    const int cy = t / C.n, cx = t - cy * C.n;
+    const double x = (double)C.x0 + (cx + 0.5) / (double)C.ix, y = (double)C.y0 + (cy + 0.5) / (double)C.iy;
+    unsigned short h[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    unsigned n = 0;
+    for (int o = 0; o < n_obs; ++o) {
+        double d2, lo = r_in, hi = r_out;  // squared distance
+        if (P) {
+            const double* b = P->ob64 + 8 * o;
+            const double tx = x - b[0], ty = y - b[1];
+            const double ex = fmax(fabs(tx * b[2] + ty * b[3]) - b[6], 0.0);
+            const double ey = fmax(fabs(tx * b[4] + ty * b[5]) - b[7], 0.0);
+            d2 = ex * ex + ey * ey;
+        } else if (o < D->ns) {
+            const double tx = x - D->sc64[2 * o], ty = y - D->sc64[2 * o + 1];
+            d2 = tx * tx + ty * ty;
+            lo = hi = sqrt(D->srT64[i * D->ns + o]);  // the sum of the radii, to rounding
+        } else {
+            const int k = o - D->ns;
+            const double ex = fmax(fmax(D->lo64[2 * k] - x, x - D->hi64[2 * k]), 0.0);
+            const double ey = fmax(fmax(D->lo64[2 * k + 1] - y, y - D->hi64[2 * k + 1]), 0.0);
+            d2 = ex * ex + ey * ey;
+        }
+        const double far = hi + slack + hd, near = lo - slack - hd;
+        if (d2 > far * far) continue;
+        if (near > 0.0 && d2 < near * near) {
+            n = CELL_HIT;
+            break;
+        }
+        ++n;
+#pragma unroll
+        for (int k = 1; k <= CELL_LIST; ++k)
+            if ((int)n == k) h[k] = (unsigned short)o;
+    }
+    if (n != CELL_HIT && n > CELL_LIST) n = CELL_MANY;
+    uint4 r;
+    r.x = n | ((unsigned)h[1] << 16);
+    r.y = h[2] | ((unsigned)h[3] << 16);
+    r.z = h[4] | ((unsigned)h[5] << 16);
+    r.w = h[6] | ((unsigned)h[7] << 16);
+    ((uint4*)C.rec)[(size_t)i * C.n * C.n + t] = r;
+}
+
+__global__ void __launch_bounds__(256) k_cells_disk(DiskView S, double hd, double slack) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
+    if (t >= S.grid.n * S.grid.n) return;
+    const double r = sqrt(S.rp2_64[i]);
+    cell_fill(S.grid, hd, slack, i, r, r, S.ns + S.nrect, t, &S, nullptr);
+}
+
+__global__ void __launch_bounds__(256) k_cells_planar(PlanarView S, double hd, double slack) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
+    if (t >= S.grid.n * S.grid.n) return;
+    const double a = S.rh64[2 * i], b = S.rh64[2 * i + 1];
+    cell_fill(S.grid, hd, slack, i, fmin(a, b), sqrt(a * a + b * b), S.no, t, nullptr, &S);
+}
+
+}  // namespace
+
+// Fills the table that sc's view points to (grid.rec, corner and scale set).
+void launch_cells(const SceneRec& sc, hipStream_t st) {
+    const CellGrid& C = sc.kind == KIND_DISKS ? sc.disk.grid : sc.planar.grid;
+    const double wx = 1.0 / (double)C.ix, wy = 1.0 / (double)C.iy;
+    const double hd = 0.5 * sqrt(wx * wx + wy * wy);
+    const double ext = std::max(std::max(fabs((double)C.x0), fabs((double)C.y0)), C.n * std::max(wx, wy));
+    const double slack = cell_slack(ext, std::max(wx, wy));
+    const dim3 grid((C.n * C.n + 255) / 256, sc.n_robots);
+    if (sc.kind == KIND_DISKS) k_cells_disk<<<grid, 256, 0, st>>>(sc.disk, hd, slack);
+    else k_cells_planar<<<grid, 256, 0, st>>>(sc.planar, hd, slack);
+}

@@ -385,6 +385,22 @@ __host__ __device__ inline int edge_state_index(const EdgeWin& w, int local, int
 
 // --------------------------------------------------------------------------------------------
 // device views of the scenes (plain pointers into one library-owned device allocation)
+
+// Cell table of a plane scene (disks in the plane, planar boxes): for every robot and every cell of
+// an n x n grid over the obstacles, what a robot whose centre lies in the cell can touch.  A record
+// is 8 halfwords: the count and up to 7 obstacle indices that may or may not touch, or CELL_HIT
+// (some obstacle overlaps the robot wherever in the cell its centre is, at any yaw) or CELL_MANY
+// (more than 7: every obstacle is tested).  Outside the grid nothing is in reach.
+struct CellGrid {
+    const uint4* rec;  // [robots * n * n]
+    float x0, y0;      // corner
+    float ix, iy;      // cells per metre
+    int n;             // cells per axis; 0: no table
+};
+#define CELL_HIT 0xffffu
+#define CELL_MANY 0xfffeu
+#define CELL_LIST 7
+
 struct DiskView {
     int nr, rd, D, ns, nrect;
     float Bscene;
@@ -395,6 +411,7 @@ struct DiskView {
     const float* lo32; const float* hi32;     // [nrect*rd]
     const double* lo64; const double* hi64;
     const float* rp2_32; const double* rp2_64;  // [nr] r**2
+    CellGrid grid;                            // rd = 2 (obstacles: spheres, then rectangles)
 };
 
 struct PlanarView {
@@ -402,6 +419,7 @@ struct PlanarView {
     float Bscene;
     const float* rh32; const double* rh64;  // [nr*2]
     const float* ob32; const double* ob64;  // [no*8] x y ux uy vx vy h0 h1
+    CellGrid grid;
 };
 
 struct ArmView {

@@ -4,6 +4,8 @@
 #include "../../include/mrcc.h"
 #include "evaluators.hpp"
 
+#include <algorithm>
+
 // An arm scene as the clearance kernels see it: scalars and the binary32 tables as one image that a
 // workgroup stages in LDS (clr_layout); tables too large for it are read from global memory.
 struct ClrK {
@@ -84,6 +86,8 @@ void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork&
 void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, long long n_list,
                    const long long* n_dev, int wpe, int init_out, int max_grid,
                    unsigned long long* stats, hipStream_t st);
+// cells.hip: fills the cell table of a plane scene
+void launch_cells(const SceneRec& sc, hipStream_t st);
 void launch_fill_u8(unsigned char* p, long long n, unsigned char v, hipStream_t st);
 // plain per-call form: edge 0 of B in one workgroup (k_arm_edge / k_lane_edge)
 void launch_edge1(const SceneRec& sc, const EdgeBatchView& B, hipStream_t st);

@@ -404,6 +404,205 @@ __device__ inline bool planar_collides(const PlanarView& S, const double* q, uns
 }
 
 // --------------------------------------------------------------------------------------------
+// Plane scenes by cell table (CellGrid): a state's robots look their cells up (one 16-byte load
+// each, all in flight together) instead of testing every obstacle, and only the few obstacles that
+// the table leaves open are tested, by the same binary32 tests and binary64 rechecks.  The table's
+// answers hold with a slack far above the rounding of the lookup (cell_slack), so the verdict is
+// that of the full test.  Every obstacle against every robot of every state bounded the batches
+// (100 obstacles x 4 robots: 400 separating-axis tests a state, k_lane_persistent 423 us on 262,144
+// edges; 20 rectangles x 2 disks, 10,000 edges of ~290 states: 135 us); by table 176 and 100 us.
+// The per-call kernels, whose lanes share a state's obstacles out, keep the full test.  `q(k)` gives coordinate k in binary64; LOOK: only what the table alone
+// decides (true: collision).
+#define CELL_MAX_YAW 0x1p20
+__host__ __device__ inline double cell_slack(double B, double cell) { return 0x1p-14 * (1.0 + B) + 0x1p-8 * cell; }
+
+__device__ inline uint4 cell_record(const CellGrid& C, int robot, float x, float y) {
+    const float fx = (x - C.x0) * C.ix, fy = (y - C.y0) * C.iy;
+    const float fn = (float)C.n;
+    uint4 r = make_uint4(C.n ? 0 : CELL_MANY, 0, 0, 0);
+    if (fx >= 0.0f && fx < fn && fy >= 0.0f && fy < fn)
+        r = C.rec[((size_t)robot * C.n + (int)fy) * C.n + (int)fx];
+    return r;
+}
+__device__ inline void cell_next(uint4& r) {  // drops the first halfword
+    r.x = __builtin_amdgcn_alignbit(r.y, r.x, 16);
+    r.y = __builtin_amdgcn_alignbit(r.z, r.y, 16);
+    r.z = __builtin_amdgcn_alignbit(r.w, r.z, 16);
+    r.w >>= 16;
+}
+// calls test(o) for the obstacles of a record (all `n_all` of them for CELL_MANY) until one is true
+template <class F>
+__device__ inline bool cell_any(uint4 r, int n_all, F test) {
+    const unsigned c = r.x & 0xffffu;
+    const bool many = c == CELL_MANY;
+    const int m = many ? n_all : (int)c;
+    for (int k = 0; k < m; ++k) {
+        cell_next(r);
+        if (test(many ? k : (int)(r.x & 0xffffu))) return true;
+    }
+    return false;
+}
+
+// planar boxes, nr <= NRB robots
+template <int NRB, bool LOOK, class Q>
+__device__ inline bool planar_state(const PlanarView& S, const Q& q, unsigned mask, unsigned& rechecks) {
+    const int nr = S.nr;
+    float x[NRB], y[NRB];
+    uint4 rec[NRB];
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < NRB; ++i) {
+        if (i >= nr) break;
+        const double qx = q(3 * i), qy = q(3 * i + 1), qt = q(3 * i + 2);
+        if constexpr (!LOOK)
+            finite = finite && __builtin_isfinite(qx) && __builtin_isfinite(qy) && __builtin_isfinite(qt);
+        x[i] = (float)qx;
+        y[i] = (float)qy;
+        rec[i] = ((mask >> i) & 1u) ? cell_record(S.grid, i, x[i], y[i]) : make_uint4(0, 0, 0, 0);
+        // the table takes the axes for unit vectors, which sincos_f64 gives up to |yaw| = 2^20
+        if (!(__builtin_fabs(qt) <= CELL_MAX_YAW) && ((mask >> i) & 1u)) rec[i].x = CELL_MANY;
+    }
+    if (!finite) return true;
+    bool hit = false;
+#pragma unroll
+    for (int i = 0; i < NRB; ++i) {
+        if (i >= nr) break;
+        hit = hit || (rec[i].x & 0xffffu) == CELL_HIT;
+    }
+    if (LOOK || hit) return hit;
+    float c[NRB], s[NRB];
+    float B = S.Bscene;
+#pragma unroll
+    for (int i = 0; i < NRB; ++i) {
+        if (i >= nr) break;
+        const SinCos t = sincos_f64(q(3 * i + 2));
+        c[i] = (float)t.c;
+        s[i] = (float)t.s;
+        B = fmaxf(B, fmaxf(fabsf(x[i]), fabsf(y[i])));
+    }
+    const float M = planar_margin(B);
+#pragma unroll
+    for (int i = 0; i < NRB; ++i) {
+        if (i >= nr) break;
+        const float hi0 = S.rh32[2 * i], hi1 = S.rh32[2 * i + 1];
+#pragma unroll
+        for (int j = i + 1; j < NRB; ++j) {
+            if (j >= nr) break;
+            if (!((mask >> i) & 1u) || !((mask >> j) & 1u)) continue;
+            const float v = obb2_sep_f32(x[i], y[i], c[i], s[i], hi0, hi1, x[j], y[j], c[j], s[j], S.rh32[2 * j],
+                                         S.rh32[2 * j + 1]);
+            if (v <= M) {
+                if (v < -M) return true;
+                ++rechecks;
+                if (planar_rr_f64(S, q(3 * i), q(3 * i + 1), q(3 * i + 2), i, q(3 * j), q(3 * j + 1), q(3 * j + 2), j))
+                    return true;
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NRB; ++i) {
+        if (i >= nr) break;
+        const float h0 = S.rh32[2 * i], h1 = S.rh32[2 * i + 1];
+        if (cell_any(rec[i], S.no, [&](int o) {
+                const float4 a = *(const float4*)(S.ob32 + 8 * o);
+                const float2 h = *(const float2*)(S.ob32 + 8 * o + 6);
+                const float v = obb2_sep_f32(x[i], y[i], c[i], s[i], h0, h1, a.x, a.y, a.z, a.w, h.x, h.y);
+                if (!(v <= M)) return false;
+                if (v < -M) return true;
+                ++rechecks;
+                return planar_ro_f64(S, q(3 * i), q(3 * i + 1), q(3 * i + 2), i, o);
+            }))
+            return true;
+    }
+    return false;
+}
+
+// disks in the plane, nr <= NRB robots
+template <int NRB, bool LOOK, class Q>
+__device__ inline bool disk2_state(const DiskView& S, const Q& q, unsigned mask, unsigned& rechecks) {
+    const int nr = S.nr;
+    float x[NRB], y[NRB];
+    uint4 rec[NRB];
+    float B = S.Bscene;
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < NRB; ++i) {
+        if (i >= nr) break;
+        const double qx = q(2 * i), qy = q(2 * i + 1);
+        finite = finite && __builtin_isfinite(qx) && __builtin_isfinite(qy);
+        x[i] = (float)qx;
+        y[i] = (float)qy;
+        B = fmaxf(B, fmaxf(fabsf(x[i]), fabsf(y[i])));
+        rec[i] = ((mask >> i) & 1u) ? cell_record(S.grid, i, x[i], y[i]) : make_uint4(0, 0, 0, 0);
+    }
+    if (!LOOK && !finite) {  // the literal binary64 evaluation
+#pragma unroll
+        for (int i = 0; i < NRB; ++i) {
+            if (i >= nr) break;
+            if (!((mask >> i) & 1u)) continue;
+#pragma unroll
+            for (int j = i + 1; j < NRB; ++j) {
+                if (j >= nr) break;
+                if (((mask >> j) & 1u) && disk_rr2_f64(S, q(2 * i), q(2 * i + 1), q(2 * j), q(2 * j + 1), i, j)) return true;
+            }
+            for (int o = 0; o < S.ns; ++o)
+                if (disk_rs2_f64(S, q(2 * i), q(2 * i + 1), i, o)) return true;
+            for (int o = 0; o < S.nrect; ++o)
+                if (disk_rect2_f64(S, q(2 * i), q(2 * i + 1), i, o)) return true;
+        }
+        return false;
+    }
+    bool hit = false;
+#pragma unroll
+    for (int i = 0; i < NRB; ++i) {
+        if (i >= nr) break;
+        hit = hit || (rec[i].x & 0xffffu) == CELL_HIT;
+    }
+    if (LOOK || hit) return hit;
+    const float M = disk_margin(B, 2);
+#pragma unroll
+    for (int i = 0; i < NRB; ++i) {
+        if (i >= nr) break;
+#pragma unroll
+        for (int j = i + 1; j < NRB; ++j) {
+            if (j >= nr) break;
+            if (!((mask >> i) & 1u) || !((mask >> j) & 1u)) continue;
+            const float dx = x[i] - x[j], dy = y[i] - y[j];
+            const float d2 = fmaf(dy, dy, dx * dx), T = S.rrT32[i * nr + j];
+            if (d2 < T + M) {
+                if (d2 < T - M) return true;
+                ++rechecks;
+                if (disk_rr2_f64(S, q(2 * i), q(2 * i + 1), q(2 * j), q(2 * j + 1), i, j)) return true;
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NRB; ++i) {
+        if (i >= nr) break;
+        if (cell_any(rec[i], S.ns + S.nrect, [&](int o) {
+                if (o < S.ns) {
+                    const float dx = S.sc32[2 * o] - x[i], dy = S.sc32[2 * o + 1] - y[i];
+                    const float d2 = fmaf(dy, dy, dx * dx), T = S.srT32[i * S.ns + o];
+                    if (!(d2 < T + M)) return false;
+                    if (d2 < T - M) return true;
+                    ++rechecks;
+                    return disk_rs2_f64(S, q(2 * i), q(2 * i + 1), i, o);
+                }
+                const int r = o - S.ns;
+                const float ex = fminf(fmaxf(x[i], S.lo32[2 * r]), S.hi32[2 * r]) - x[i];
+                const float ey = fminf(fmaxf(y[i], S.lo32[2 * r + 1]), S.hi32[2 * r + 1]) - y[i];
+                const float d2 = fmaf(ey, ey, ex * ex), T = S.rp2_32[i];
+                if (!(d2 <= T + M)) return false;
+                if (d2 < T - M) return true;
+                ++rechecks;
+                return disk_rect2_f64(S, q(2 * i), q(2 * i + 1), i, r);
+            }))
+            return true;
+    }
+    return false;
+}
+
+// --------------------------------------------------------------------------------------------
 // arms: one state per wavefront; workgroups of 1, 2 or 4 waves.
 //
 // LDS of a workgroup = one static region (the scene, staged once per kernel by the whole

@@ -390,46 +390,39 @@ __device__ inline EdgeWin win_of(const PlanWork& W, int e, int incl) {
 
 // ============================================================================================
 // lane-per-state kinds
-template <class View, int T1, int T2>
-__device__ inline bool lane_collides(const View& S, const double* q, unsigned mask, unsigned& rc);
-
-// register length of the per-lane state: exact for the specialised shapes
+// Disks in the plane: <DiskView, 2, NRB>, at most NRB robots; planar boxes: <PlanarView, NRB, 0>,
+// likewise; other disks: <DiskView, 0, 0>.
+// register length of the per-lane state
 template <class View, int T1, int T2>
 struct LaneDim {
-    static constexpr int value = MRCC_MAX_D;
+    static constexpr int value = T1 ? T1 * T2 : MRCC_DISK_MAX_RD * 4;
 };
-template <>
-struct LaneDim<DiskView, 2, 2> {
-    static constexpr int value = 4;
-};
-template <>
-struct LaneDim<PlanarView, 4, 0> {
-    static constexpr int value = 12;
-};
-template <>
-struct LaneDim<PlanarView, 0, 0> {
-    static constexpr int value = 3 * MRCC_PLANAR_MAX_ROBOTS;
-};
-template <>
-struct LaneDim<DiskView, 0, 0> {
-    static constexpr int value = MRCC_DISK_MAX_RD * 4;
+template <int T1>
+struct LaneDim<PlanarView, T1, 0> {
+    static constexpr int value = 3 * (T1 ? T1 : MRCC_PLANAR_MAX_ROBOTS);
 };
 
-template <>
-__device__ inline bool lane_collides<DiskView, 2, 2>(const DiskView& S, const double* q, unsigned mask, unsigned& rc) {
-    return disk_collides<2, 2>(S, q, mask, rc);
+template <class View, int T1, int T2>
+__device__ inline bool lane_collides(const View& S, const double* q, unsigned mask, unsigned& rc) {
+    auto at = [&](int k) { return q[k]; };
+    if constexpr (std::is_same<View, PlanarView>::value) return planar_state<T1, false>(S, at, mask, rc);
+    else if constexpr (T1 == 2) return disk2_state<T2, false>(S, at, mask, rc);
+    else return disk_collides<0, 0>(S, q, mask, rc);
 }
-template <>
-__device__ inline bool lane_collides<DiskView, 0, 0>(const DiskView& S, const double* q, unsigned mask, unsigned& rc) {
-    return disk_collides<0, 0>(S, q, mask, rc);
-}
-template <>
-__device__ inline bool lane_collides<PlanarView, 4, 0>(const PlanarView& S, const double* q, unsigned mask, unsigned& rc) {
-    return planar_collides<4>(S, q, mask, rc);
-}
-template <>
-__device__ inline bool lane_collides<PlanarView, 0, 0>(const PlanarView& S, const double* q, unsigned mask, unsigned& rc) {
-    return planar_collides<0>(S, q, mask, rc);
+
+// calls F(view, T1, T2) with the smallest bounds that hold the scene
+template <class F>
+static void lane_dispatch(const SceneRec& sc, F f) {
+    using std::integral_constant;
+    if (sc.kind == KIND_DISKS) {
+        if (sc.disk.rd == 2 && sc.disk.nr <= 2) f(sc.disk, integral_constant<int, 2>(), integral_constant<int, 2>());
+        else if (sc.disk.rd == 2 && sc.disk.nr <= 4) f(sc.disk, integral_constant<int, 2>(), integral_constant<int, 4>());
+        else f(sc.disk, integral_constant<int, 0>(), integral_constant<int, 0>());
+    } else {
+        if (sc.planar.nr <= 4) f(sc.planar, integral_constant<int, 4>(), integral_constant<int, 0>());
+        else if (sc.planar.nr <= 8) f(sc.planar, integral_constant<int, 8>(), integral_constant<int, 0>());
+        else f(sc.planar, integral_constant<int, MRCC_PLANAR_MAX_ROBOTS>(), integral_constant<int, 0>());
+    }
 }
 
 template <class View, int T1, int T2>
@@ -1322,16 +1315,10 @@ void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork&
                      int spt, int grid, hipStream_t st) {
     switch (sc.kind) {
         case KIND_DISKS:
-            if (sc.disk.rd == 2 && sc.disk.nr == 2)
-                k_lane_persistent<DiskView, 2, 2><<<grid, 256, 0, st>>>(sc.disk, B, W, lgG, spt);
-            else
-                k_lane_persistent<DiskView, 0, 0><<<grid, 256, 0, st>>>(sc.disk, B, W, lgG, spt);
-            break;
         case KIND_PLANAR:
-            if (sc.planar.nr == 4)
-                k_lane_persistent<PlanarView, 4, 0><<<grid, 256, 0, st>>>(sc.planar, B, W, lgG, spt);
-            else
-                k_lane_persistent<PlanarView, 0, 0><<<grid, 256, 0, st>>>(sc.planar, B, W, lgG, spt);
+            lane_dispatch(sc, [&](auto view, auto t1, auto t2) {
+                k_lane_persistent<decltype(view), t1, t2><<<grid, 256, 0, st>>>(view, B, W, lgG, spt);
+            });
             break;
         case KIND_ARMS: {
             // grid counts waves; workgroups of arm_nw_pers waves, no more of them than can be resident
@@ -1393,16 +1380,10 @@ void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, 
     if (grid < 1) grid = 1;
     switch (sc.kind) {
         case KIND_DISKS:
-            if (sc.disk.rd == 2 && sc.disk.nr == 2)
-                k_lane_direct<DiskView, 2, 2><<<grid, 64, 0, st>>>(sc.disk, B, list, n_list, n_dev, wpe, init_out, stats);
-            else
-                k_lane_direct<DiskView, 0, 0><<<grid, 64, 0, st>>>(sc.disk, B, list, n_list, n_dev, wpe, init_out, stats);
-            break;
         case KIND_PLANAR:
-            if (sc.planar.nr == 4)
-                k_lane_direct<PlanarView, 4, 0><<<grid, 64, 0, st>>>(sc.planar, B, list, n_list, n_dev, wpe, init_out, stats);
-            else
-                k_lane_direct<PlanarView, 0, 0><<<grid, 64, 0, st>>>(sc.planar, B, list, n_list, n_dev, wpe, init_out, stats);
+            lane_dispatch(sc, [&](auto view, auto t1, auto t2) {
+                k_lane_direct<decltype(view), t1, t2><<<grid, 64, 0, st>>>(view, B, list, n_list, n_dev, wpe, init_out, stats);
+            });
             break;
         case KIND_ARMS: {
             // `grid` waves (at most one per work item), in workgroups of arm_nw waves, or of
@@ -1429,22 +1410,13 @@ void launch_configs(const SceneRec& sc, const double* q, long long n, long long 
                     const int* modes, unsigned mask, unsigned char* out, int max_grid,
                     hipStream_t st) {
     switch (sc.kind) {
-        case KIND_DISKS: {
-            int g = grid_for(n, 256);
-            if (g > max_grid) g = max_grid;
-            if (sc.disk.rd == 2 && sc.disk.nr == 2)
-                k_lane_configs<DiskView, 2, 2><<<g, 256, 0, st>>>(sc.disk, q, n, rs, ds, mask, out);
-            else
-                k_lane_configs<DiskView, 0, 0><<<g, 256, 0, st>>>(sc.disk, q, n, rs, ds, mask, out);
-            break;
-        }
+        case KIND_DISKS:
         case KIND_PLANAR: {
             int g = grid_for(n, 256);
             if (g > max_grid) g = max_grid;
-            if (sc.planar.nr == 4)
-                k_lane_configs<PlanarView, 4, 0><<<g, 256, 0, st>>>(sc.planar, q, n, rs, ds, mask, out);
-            else
-                k_lane_configs<PlanarView, 0, 0><<<g, 256, 0, st>>>(sc.planar, q, n, rs, ds, mask, out);
+            lane_dispatch(sc, [&](auto view, auto t1, auto t2) {
+                k_lane_configs<decltype(view), t1, t2><<<g, 256, 0, st>>>(view, q, n, rs, ds, mask, out);
+            });
             break;
         }
         case KIND_ARMS: {

@@ -166,7 +166,8 @@ typedef struct mrcc_edge_batch {
 
 /* Execution shape of the batched edge check (chosen by the autotuner when NULL / zero). */
 typedef struct mrcc_tune {
-    int32_t slots_per_pass;    /* states of one edge issued per pass (coarse-to-fine order) */
+    int32_t slots_per_pass;    /* states of one edge issued per pass (coarse-to-fine order); 0: the
+                                  library's choice (plane scenes then run without the queue) */
     int32_t slots_per_ticket;  /* queue slots a wave claims per atomic ticket (arm scenes:
                                   <= 64, one lane resolves one slot) */
     int32_t waves_per_cu;      /* persistent grid = waves_per_cu * CUs */

@@ -22,8 +22,9 @@ from .backend import EdgePlan, make_tune
 CACHE = os.environ.get("MRCC_AUTOTUNE_CACHE", os.path.join(os.path.expanduser("~"), ".cache", "mrcc_autotune.json"))
 
 DIRECT = dict(persistent=0, sorted=0)  # the single launch: no queue, one workgroup per edge
+DEFAULT = dict(slots_per_pass=0, slots_per_ticket=0, waves_per_cu=0)  # the library's own choice
 LANE_GRID = [dict(slots_per_pass=g, slots_per_ticket=t, waves_per_cu=w)
-             for g in (4, 8, 16, 32) for t in (1, 2, 4) for w in (8, 16)] + [DIRECT]
+             for g in (4, 8, 16, 32) for t in (1, 2, 4) for w in (8, 16)] + [DIRECT, DEFAULT]
 ARM_GRID = [dict(slots_per_pass=g, slots_per_ticket=t, waves_per_cu=w)
             for g in (1, 2, 4, 8) for t in (8, 16, 32) for w in (12, 16)] + [DIRECT]
 
@@ -31,6 +32,8 @@ ARM_GRID = [dict(slots_per_pass=g, slots_per_ticket=t, waves_per_cu=w)
 def candidate_name(cand: dict) -> str:
     if not cand.get("persistent", 1):
         return "direct"
+    if not cand["slots_per_pass"]:
+        return "default"
     return "G{slots_per_pass}/t{slots_per_ticket}/w{waves_per_cu}".format(**cand)
 
 

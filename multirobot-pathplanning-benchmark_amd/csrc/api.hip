@@ -623,7 +623,9 @@ int tune_defaults(const SceneRec* sc, const mrcc_tune* tune, mrcc_tune* t) {
     memset(t, 0, sizeof(*t));
     if (tune) *t = *tune;
     const bool arms = sc->kind == KIND_ARMS;
-    if (t->slots_per_pass <= 0) t->slots_per_pass = arms ? 1 : 8;
+    // plane scenes with a cell table take the queue when its shape is asked for, or its statistics
+    if (t->slots_per_pass <= 0)
+        t->slots_per_pass = arms ? 1 : (lane_looks_apply(*sc) && !t->collect_stats ? 0 : 8);
     if (t->slots_per_ticket <= 0) t->slots_per_ticket = arms ? 16 : 4;
     if (t->waves_per_cu <= 0) t->waves_per_cu = 16;
     if (!tune) {
@@ -636,6 +638,10 @@ int tune_defaults(const SceneRec* sc, const mrcc_tune* tune, mrcc_tune* t) {
     if (arms && t->slots_per_ticket > 64)  // one lane resolves one slot of a claimed chunk
         return ::fail(MRCC_ERR_INVALID, "arm scenes: slots_per_ticket <= 64");
     return MRCC_OK;
+}
+
+int plan_lgG(const mrcc_tune& t) {
+    return t.slots_per_pass > 0 ? __builtin_ctz((unsigned)t.slots_per_pass) : MRCC_NO_QUEUE;
 }
 
 int plan_grid(const SceneRec* sc, const mrcc_tune& t) {
@@ -665,12 +671,18 @@ size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W) {
         W->ticket = (unsigned long long*)(base + o_tick);
         W->stats = (unsigned long long*)(base + o_stats);
         W->dir = (double*)(base + o_dir);
+        W->items = (int2*)(base + o_rec);  // 20 n + 256 Ki bytes
+        W->items_cap = (long long)((o_meta - o_rec) / sizeof(int2));
     }
     return top;
 }
 
 void launch_plan_sequence(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, int spt,
-                          int grid, hipStream_t st) {
+                          int grid, hipStream_t st, bool shared) {
+    if (lgG == MRCC_NO_QUEUE) {
+        launch_lane_looks(sc, B, W, shared, st);
+        return;
+    }
     launch_plan_build(sc, B, W, lgG, st);
     launch_plan_run(sc, B, W, lgG, spt, grid, st);
     launch_long_edges(sc, B, W, st);
@@ -704,7 +716,11 @@ static void plan_launch_sequence(mrcc_edge_plan* p, hipStream_t st) {
     const bool ev = p->ev[0] != nullptr;
     if (ev) (void)hipEventRecord(p->ev[0], st);
     if (p->tune.persistent && !ev) {
-        mrcc_internal::launch_plan_sequence(*p->sc, p->B, p->W, p->lgG, p->tune.slots_per_ticket, p->grid, st);
+        mrcc_internal::launch_plan_sequence(*p->sc, p->B, p->W, p->lgG, p->tune.slots_per_ticket, p->grid, st, false);
+    } else if (p->tune.persistent && p->lgG == MRCC_NO_QUEUE) {
+        (void)hipEventRecord(p->ev[1], st);
+        launch_lane_looks(*p->sc, p->B, p->W, false, st);
+        (void)hipEventRecord(p->ev[2], st);
     } else if (p->tune.persistent) {
         launch_plan_build(*p->sc, p->B, p->W, p->lgG, st);
         (void)hipEventRecord(p->ev[1], st);
@@ -1126,7 +1142,7 @@ int mrcc_edge_plan_create(const mrcc_scene* scene, const mrcc_edge_batch* batch,
     p->sc = sc;
     p->B = view_of(batch);
     p->tune = t;
-    p->lgG = __builtin_ctz((unsigned)t.slots_per_pass);
+    p->lgG = mrcc_internal::plan_lgG(t);
     p->grid = mrcc_internal::plan_grid(sc, t);
     // workspace
     const size_t work_bytes = mrcc_internal::plan_layout(batch->n_edges, sc->D, nullptr, nullptr);

@@ -567,4 +567,7 @@ struct PlanWork {
     unsigned long long* ticket;  // [8 * 32]: one chunk counter per XCD, 256 bytes apart
     unsigned long long* stats;  // [8]
     double* dir;       // [n*D] (lane-per-state kinds) or null
+    // lane_looks.hip uses meta in its own way and this list, in the place of erec .. pass_start
+    int2* items;       // (edge, part) of long edges
+    long long items_cap;
 };

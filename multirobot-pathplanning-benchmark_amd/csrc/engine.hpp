@@ -86,6 +86,11 @@ void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork&
 void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, long long n_list,
                    const long long* n_dev, int wpe, int init_out, int max_grid,
                    unsigned long long* stats, hipStream_t st);
+// lane_looks.hip: edge batches of plane scenes with a cell table, two launches, no queue; W.meta is
+// zero before the workspace's first run (`reset`: cleared here, for workspaces used otherwise too)
+bool lane_looks_apply(const SceneRec& sc);
+void launch_lane_looks(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, bool reset, hipStream_t st);
+#define MRCC_NO_QUEUE (-1)  // lgG of such a run
 // cells.hip: fills the cell table of a plane scene
 void launch_cells(const SceneRec& sc, hipStream_t st);
 void launch_fill_u8(unsigned char* p, long long n, unsigned char v, hipStream_t st);
@@ -148,8 +153,10 @@ int plan_grid(const SceneRec* sc, const mrcc_tune& t);
 size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W);
 void launch_long_edges(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, hipStream_t st);
 // queue build, persistent kernel and long-edge fallback on stream st
+// (lgG = MRCC_NO_QUEUE: the two launches of lane_looks.hip; `shared`: the workspace serves other runs too)
 void launch_plan_sequence(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, int spt,
-                          int grid, hipStream_t st);
+                          int grid, hipStream_t st, bool shared);
+int plan_lgG(const mrcc_tune& t);
 }  // namespace mrcc_internal
 
 // noalloc.hip: looks up the current device's scratch array (called by mrcc_init)

@@ -1,0 +1,83 @@
+// lanes.hpp — what the edge kernels share: rows, interpolation, verdict bytes, and the choice of
+// the lane-per-state evaluator.
+#pragma once
+
+#include "engine.hpp"
+
+using namespace mrcc;
+
+__device__ inline void stat_add(unsigned long long* stats, int idx, unsigned long long v) {
+    if (stats && v) atomicAdd(stats + idx, v);
+}
+
+// row pointers of edge e
+__device__ inline const double* row1(const EdgeBatchView& B, long long e) {
+    long long r = B.idx1 ? (long long)B.idx1[e] : e;
+    return B.q1 + r * B.rs;
+}
+__device__ inline const double* row1(const ArmQueue& B, long long e) {
+    long long r = B.idx1 ? (long long)B.idx1[e] : e;
+    return B.q1 + r * B.rs;
+}
+__device__ inline const double* row2(const EdgeBatchView& B, long long e) {
+    long long r = B.idx2 ? (long long)B.idx2[e] : e;
+    return B.q2 + r * B.rs;
+}
+
+// interpolated state (abstract_env.py:341, :348): q1 + ((q2 - q1) / (N - 1)) * i, unfused
+__device__ inline double interp_f64(double a, double b, int N, int i) {
+#pragma clang fp contract(off)
+    double dir = (b - a) / (double)(N - 1);
+    return a + dir * (double)i;
+}
+__device__ inline double interp_dir_f64(double a, double dir, int i) {
+#pragma clang fp contract(off)
+    return a + dir * (double)i;
+}
+
+// binary64 interpolation step of one coordinate, (b - a) / (N - 1), as interp_f64 forms it
+__device__ inline double interp_step_f64(double a, double b, int N) {
+#pragma clang fp contract(off)
+    return (b - a) / (double)(N - 1);
+}
+
+// The verdict byte of an edge in the persistent kernels, as every XCD sees it: another wave
+// writes an edge's 0 when one of its states collides, and the later slots of the edge are skipped
+// when they read it.  Each XCD has its own L2 and plain accesses may stay in it (a plain read can
+// return an XCD's stale copy until the kernel ends); agent-scope accesses reach the level that all
+// XCDs share.  (The direct kernels keep plain accesses: there the agent-scope ones measured slower,
+// 47 -> 248 us for a list of 30 arm edges with 64 waves per edge.)
+__device__ inline bool edge_dead(const unsigned char* out, int e) {
+    return __hip_atomic_load(out + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+}
+__device__ inline void edge_kill(unsigned char* out, int e) {
+    __hip_atomic_store(out + e, (unsigned char)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Disks in the plane: <DiskView, 2, NRB>, at most NRB robots; planar boxes: <PlanarView, NRB, 0>,
+// likewise; other disks: <DiskView, 0, 0>.
+// register length of the per-lane state
+template <class View, int T1, int T2>
+struct LaneDim {
+    static constexpr int value = T1 ? T1 * T2 : MRCC_DISK_MAX_RD * 4;
+};
+template <int T1>
+struct LaneDim<PlanarView, T1, 0> {
+    static constexpr int value = 3 * (T1 ? T1 : MRCC_PLANAR_MAX_ROBOTS);
+};
+
+// calls F(view, T1, T2) with the smallest bounds that hold the scene
+template <class F>
+static void lane_dispatch(const SceneRec& sc, F f) {
+    using std::integral_constant;
+    if (sc.kind == KIND_DISKS) {
+        if (sc.disk.rd == 2 && sc.disk.nr <= 2) f(sc.disk, integral_constant<int, 2>(), integral_constant<int, 2>());
+        else if (sc.disk.rd == 2 && sc.disk.nr <= 4) f(sc.disk, integral_constant<int, 2>(), integral_constant<int, 4>());
+        else f(sc.disk, integral_constant<int, 0>(), integral_constant<int, 0>());
+    } else {
+        if (sc.planar.nr <= 4) f(sc.planar, integral_constant<int, 4>(), integral_constant<int, 0>());
+        else if (sc.planar.nr <= 8) f(sc.planar, integral_constant<int, 8>(), integral_constant<int, 0>());
+        else f(sc.planar, integral_constant<int, MRCC_PLANAR_MAX_ROBOTS>(), integral_constant<int, 0>());
+    }
+}
+

@@ -91,8 +91,8 @@ extern "C" int mrcc_check_edges_noalloc(const mrcc_scene* scene, const mrcc_edge
     W.stats = nullptr;
     if (batch->n_edges > 0) {
         const EdgeBatchView B = mrcc_internal::batch_view(batch);
-        mrcc_internal::launch_plan_sequence(*sc, B, W, __builtin_ctz((unsigned)t.slots_per_pass), t.slots_per_ticket,
-                                            mrcc_internal::plan_grid(sc, t), st);
+        mrcc_internal::launch_plan_sequence(*sc, B, W, mrcc_internal::plan_lgG(t), t.slots_per_ticket,
+                                            mrcc_internal::plan_grid(sc, t), st, true);
     }
     if (n_invalid) k_store_count<<<1, 64, 0, st>>>(batch->n_edges > 0 ? W.meta + 2 : nullptr, n_invalid);
     hipError_t e = hipGetLastError();

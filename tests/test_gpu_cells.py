@@ -65,3 +65,53 @@ def test_scenes_without_a_table():
     desc.obstacle_half[3] *= -1.0
     desc.obstacle_pose[4, 0] = 3e5
     _check(desc, q, a, b)
+
+
+def _batch(rng, desc, n):
+    a = rng.uniform(desc.limits[0], desc.limits[1], size=(n, desc.dim))
+    step = np.exp(rng.normal(np.log(0.3), 1.2, (n, 1)))
+    return a, a + step * rng.uniform(-1, 1, a.shape)
+
+
+# edges per wave 1, 2, 4, 8, 16 change at multiples of 4,000; the last wave is partly filled
+@pytest.mark.parametrize("n", [1, 63, 7999, 8000, 16001, 32003, 64005])
+@pytest.mark.parametrize("kind,nr", [("disks", 2), ("disks", 3), ("planar", 2), ("planar", 5)])
+def test_batches(n, kind, nr):
+    rng = np.random.default_rng(n + nr)
+    desc = (scenes.planar_disks(rng=rng, n_robots=nr, n_rects=6) if kind == "disks" else
+            scenes.planar_boxes(rng=rng, n_robots=nr, n_obstacles=12))
+    sc, o = backend().Scene(desc), O.Scene(desc)
+    a, b = _batch(rng, desc, n)
+    if n > 100:
+        a[5, 1], b[6] = np.nan, a[6]
+    assert np.array_equal(gpu_edges(sc, a, b, 0.01), o.check_edges(a, b, 0.01))
+    N = rng.integers(2, 90, n).astype(np.int32)
+    S = (rng.uniform(size=n) * N * 0.5).astype(np.int32)
+    M = np.where(rng.uniform(size=n) < 0.3, -1, S + rng.integers(0, 40, n)).astype(np.int32)
+    for incl in (False, True):
+        assert np.array_equal(gpu_edges(sc, a, b, 0.05, N=N, N_start=S, N_max=M, incl=incl),
+                              o.check_edges(a, b, 0.05, N=N, N_start=S, N_max=M, include_endpoints=incl))
+
+
+# 1,024 states: the most that a wave takes on its own; 200 edges of 60,000: more items than the list
+# holds; 3 of 3,000,000: the largest share of the list
+@pytest.mark.parametrize("n,states", [(9, 1026), (9, 1027), (40, 20000), (200, 60000), (3, 3000000)])
+def test_long_edges(n, states):
+    rng = np.random.default_rng(states)
+    desc = scenes.disks_scene([0.1, 0.05], 2, np.array([[-2.0] * 4, [2.0] * 4]),
+                              spheres=[(np.array([0.3, 0.2]), 0.1)], rects=[(np.array([-0.9, 0.5]), np.array([0.2, 0.3]))])
+    sc, o = backend().Scene(desc), O.Scene(desc)
+    a = rng.uniform(-2, 2, (n, 4))
+    b = a.copy()
+    b[:, 0] = a[:, 0] + 0.5
+    b[:, 1:] += 0.2 * rng.uniform(-1, 1, (n, 3))
+    N = np.full(n, states, np.int32)
+    N[::4] = 50
+    ref = o.check_edges(a, b, 0.01, N=N)
+    ta, tb, tN = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda(), torch.from_numpy(N).cuda()
+    out = torch.empty(n, dtype=torch.uint8, device="cuda")
+    plan = backend().EdgePlan(sc, sc.edge_batch(ta, tb, out, 0.01, N=tN), keep=(ta, tb, tN, out))
+    for _ in range(4):  # the counters go from run to run
+        out.fill_(9)
+        plan.run()
+        assert np.array_equal(out.cpu().numpy().astype(bool), ref)

@@ -162,6 +162,23 @@ __host__ __device__ inline void chain_step_f64(double* X, const double* C, SinCo
     for (int k = 0; k < 12; ++k) X[k] = Y[k];
 }
 
+// one row (R0 R1 R2 | t) of X <- X * A of a chain joint: chain_step_f64's operations
+__host__ __device__ inline void chain_row_f64(double& R0, double& R1, double& R2, double& t, const double* C,
+                                              double cs, double sn, bool prismatic, double q) {
+#pragma clang fp contract(off)
+    double y[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const ChainCoef k = chain_coef_f64(cs, sn, C[c], C[4 + c]);
+        const double a2 = c == 3 ? chain_a23_f64(C, prismatic, q) : C[8 + c];
+        y[c] = (R0 * k.a0 + R1 * k.a1) + R2 * a2;
+    }
+    R0 = y[0];
+    R1 = y[1];
+    R2 = y[2];
+    t = y[3] + t;
+}
+
 // one row of G = X * Rel (compose_f64)
 __host__ __device__ inline void compose_row_f64(double R0, double R1, double R2, double t,
                                                 const double* Rel, double* g) {

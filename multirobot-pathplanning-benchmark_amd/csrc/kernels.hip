@@ -1173,30 +1173,69 @@ __global__ void __launch_bounds__(NT) k_lane_edge(View S0, EdgeBatchView B) {
     if (threadIdx.x == 0) B.out[0] = (w.err || s_hit) ? 0 : 1;
 }
 
-// binary64 forward kinematics of every link, out[r][L][12]
-__global__ void k_arm_fk(ArmView V, const double* qv, long long n, long long rs, long long ds,
-                         double* out) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+// Binary64 forward kinematics of every link, out[r][L][12].  HBM-bound (291 MB for 100,000 rows of
+// 28 joints, 92% of it written).  A quad of lanes per (row, arm) t: lanes 0..2 carry a row of the
+// frame each, the joints' sines and cosines are shared out over the quad.  The frames of t are the
+// contiguous run out[(t dof + k) 12], k < dof, and a wave's 16 runs are one: they are gathered in LDS
+// and leave as whole lines.  A lane per (row, arm) storing its frames as they came wrote 8 bytes at a
+// time, 672 apart (100-132 us); one joint at a time through LDS still left lines half written
+// when they were evicted (61 us into a buffer that the 256 MB cache holds, 122 us otherwise).
+// V2: `out` is 16-byte aligned, else 8-byte stores.
+#define FK_NW 2
+#define FK_ITEMS 16
+template <bool V2>
+__global__ void __launch_bounds__(64 * FK_NW) k_arm_fk(ArmView V, const double* qv, long long n, long long rs,
+                                                       long long ds, double* out) {
+    using Word = typename std::conditional<V2, double2, double>::type;
+    extern __shared__ double2 s_fk[];
+    const int lane = wave_lane(), dof = V.dof, wid = threadIdx.x >> 6;
+    double* mine = (double*)s_fk + (size_t)wid * FK_ITEMS * 12 * dof;
+    const long long t0 = ((long long)blockIdx.x * FK_NW + wid) * FK_ITEMS;
+    const long long left = n * V.na - t0;
+    if (left <= 0) return;  // no workgroup barrier below
+    const int items = left < FK_ITEMS ? (int)left : FK_ITEMS;
+    const int i = lane >> 2, sub = lane & 3;
+    const long long t = t0 + (i < items ? i : items - 1);
     const long long r = t / V.na;
-    const int a = (int)(t % V.na);
-    if (r >= n) return;
-    double X[12];
-    for (int k = 0; k < 12; ++k) X[k] = V.base[12 * a + k];
-    for (int k = 0; k < V.dof; ++k) {
-        const int l = a * V.dof + k;
-        const double q = qv[r * rs + (long long)l * ds];
-        if (V.chain) {
-            const bool pr = (V.prism >> l) & 1ull;
-            SinCos j = sincos_f64(q);
-            if (pr) j.s = 0.0, j.c = 1.0;
-            chain_step_f64(X, V.dh + 12 * l, j, pr, q);
-        } else {
-            const SinCos j = sincos_f64(q);
-            const double* p = V.dh + 4 * l;
-            dh_step_f64(X, p[0], p[1], p[2], p[3], j);
-        }
-        for (int c = 0; c < 12; ++c) out[(r * V.L + l) * 12 + c] = X[c];
+    const int a = (int)(t - r * V.na);
+    const int row = sub < 3 ? sub : 2;
+    double q[2];
+    SinCos sc[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k = sub + 4 * h, l = a * dof + k;
+        q[h] = k < dof ? qv[r * rs + (long long)l * ds] : 0.0;
     }
+    double R0 = V.base[12 * a + 3 * row], R1 = V.base[12 * a + 3 * row + 1], R2 = V.base[12 * a + 3 * row + 2],
+           T = V.base[12 * a + 9 + row];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) sc[h] = sincos_f64(q[h]);
+#pragma unroll
+    for (int k = 0; k < MRCC_MAX_DOF; ++k) {
+        if (k >= dof) break;
+        const int l = a * dof + k;
+        double sn = quad_bcast_f64(sc[k >> 2].s, k & 3), cs = quad_bcast_f64(sc[k >> 2].c, k & 3);
+        if (V.chain) {
+            const double qk = quad_bcast_f64(q[k >> 2], k & 3);
+            const bool pr = (V.prism >> l) & 1ull;
+            if (pr) sn = 0.0, cs = 1.0;
+            chain_row_f64(R0, R1, R2, T, V.dh + 12 * l, cs, sn, pr, qk);
+        } else {
+            dh_row_f64(R0, R1, R2, T, V.dh + 4 * l, cs, sn);
+        }
+        if (sub < 3) {
+            double* f = mine + (i * dof + k) * 12;
+            f[3 * row] = R0;
+            f[3 * row + 1] = R1;
+            f[3 * row + 2] = R2;
+            f[9 + row] = T;
+        }
+    }
+    wave_sync();
+    const int words = items * dof * (V2 ? 6 : 12);
+    const Word* src = (const Word*)mine;
+    Word* dst = (Word*)(out + t0 * dof * 12);
+    for (int u = lane; u < words; u += 64) dst[u] = src[u];
 }
 
 __global__ void k_sincos(const double* x, long long n, double* s, double* c) {
@@ -1476,7 +1515,10 @@ void launch_edge1(const SceneRec& sc, const EdgeBatchView& B, hipStream_t st) {
 void launch_arm_fk(const SceneRec& sc, const double* q, long long n, long long rs, long long ds,
                    double* out, hipStream_t st) {
     long long t = n * sc.arm.na;
-    k_arm_fk<<<grid_for(t, 128), 128, 0, st>>>(sc.arm, q, n, rs, ds, out);
+    const int blocks = grid_for(t, FK_ITEMS * FK_NW);
+    const size_t lds = sizeof(double) * 12 * FK_ITEMS * FK_NW * sc.arm.dof;  // at most 24 KiB
+    if (((uintptr_t)out & 15) == 0) k_arm_fk<true><<<blocks, 64 * FK_NW, lds, st>>>(sc.arm, q, n, rs, ds, out);
+    else k_arm_fk<false><<<blocks, 64 * FK_NW, lds, st>>>(sc.arm, q, n, rs, ds, out);
 }
 
 __global__ void k_set_flag(unsigned char* flag) {

@@ -659,7 +659,8 @@ size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W) {
     };
     const size_t o_rec = sz(16 * n), o_order = sz(4 * n), o_hist = sz(4 * (MRCC_MAX_PASSES + 1)),
                  o_cur = sz(4 * (MRCC_MAX_PASSES + 1)), o_ps = sz(8 * (MRCC_MAX_PASSES + 1)), o_meta = sz(8 * 8),
-                 o_long = sz(4 * n), o_tick = sz(8 * 32 * 8), o_stats = sz(8 * 8), o_dir = sz(8 * (size_t)n * D);
+                 o_spare = sz(4 * n), o_tick = sz(8 * 32 * 8), o_stats = sz(8 * 8), o_dir = sz(8 * (size_t)n * D);
+    (void)o_spare;  // keeps the size that the no-allocation entry point's limit is stated by
     if (W) {
         W->erec = (int4*)(base + o_rec);
         W->order = (int*)(base + o_order);
@@ -667,7 +668,6 @@ size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W) {
         W->cursor = (int*)(base + o_cur);
         W->pass_start = (long long*)(base + o_ps);
         W->meta = (long long*)(base + o_meta);
-        W->long_list = (int*)(base + o_long);
         W->ticket = (unsigned long long*)(base + o_tick);
         W->stats = (unsigned long long*)(base + o_stats);
         W->dir = (double*)(base + o_dir);
@@ -678,23 +678,15 @@ size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W) {
 }
 
 void launch_plan_sequence(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, int spt,
-                          int grid, hipStream_t st, bool shared) {
+                          int grid, hipStream_t st, bool clear) {
     if (lgG == MRCC_NO_QUEUE) {
-        launch_lane_looks(sc, B, W, shared, st);
+        launch_lane_looks(sc, B, W, clear, st);
         return;
     }
-    launch_plan_build(sc, B, W, lgG, st);
+    launch_plan_build(sc, B, W, lgG, clear, st);
     launch_plan_run(sc, B, W, lgG, spt, grid, st);
-    launch_long_edges(sc, B, W, st);
 }
 
-// Edges with more passes than the queue holds: disk and planar scenes one workgroup per edge, arm
-// scenes every resident wave on one edge after another (16,385 states or more, one per wave and
-// turn).
-void launch_long_edges(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, hipStream_t st) {
-    const int waves = (sc.kind == KIND_ARMS ? 16 : 4) * ::device_cus();
-    launch_direct(sc, B, W.long_list, 0, W.meta + 3, sc.kind == KIND_ARMS ? waves : 1, 0, waves, W.stats, st);
-}
 }  // namespace mrcc_internal
 
 struct mrcc_edge_plan {
@@ -710,26 +702,28 @@ struct mrcc_edge_plan {
     hipStream_t cap_stream;
     hipEvent_t ev[4];  // time_kernels: start, queue built, main kernel done, end
     int timed_runs;
+    bool dirty;  // a launch of a run failed: the workspace is cleared before the next one
 };
 
 static void plan_launch_sequence(mrcc_edge_plan* p, hipStream_t st) {
     const bool ev = p->ev[0] != nullptr;
+    const bool clear = p->dirty || p->W.stats;  // statistics are those of the last run
     if (ev) (void)hipEventRecord(p->ev[0], st);
     if (p->tune.persistent && !ev) {
-        mrcc_internal::launch_plan_sequence(*p->sc, p->B, p->W, p->lgG, p->tune.slots_per_ticket, p->grid, st, false);
+        mrcc_internal::launch_plan_sequence(*p->sc, p->B, p->W, p->lgG, p->tune.slots_per_ticket, p->grid, st,
+                                            clear);
     } else if (p->tune.persistent && p->lgG == MRCC_NO_QUEUE) {
         (void)hipEventRecord(p->ev[1], st);
-        launch_lane_looks(*p->sc, p->B, p->W, false, st);
+        launch_lane_looks(*p->sc, p->B, p->W, clear, st);
         (void)hipEventRecord(p->ev[2], st);
     } else if (p->tune.persistent) {
-        launch_plan_build(*p->sc, p->B, p->W, p->lgG, st);
+        launch_plan_build(*p->sc, p->B, p->W, p->lgG, clear, st);
         (void)hipEventRecord(p->ev[1], st);
         launch_plan_run(*p->sc, p->B, p->W, p->lgG, p->tune.slots_per_ticket, p->grid, st);
         (void)hipEventRecord(p->ev[2], st);
-        mrcc_internal::launch_long_edges(*p->sc, p->B, p->W, st);
     } else {
         if (ev) (void)hipEventRecord(p->ev[1], st);
-        launch_direct(*p->sc, p->B, nullptr, p->B.n, nullptr, 1, 1, 1 << 20, p->W.stats, st);
+        launch_direct(*p->sc, p->B, nullptr, p->B.n, 1, 1, 1 << 20, p->W.stats, st);
         if (ev) (void)hipEventRecord(p->ev[2], st);
     }
     if (ev) {
@@ -1152,10 +1146,9 @@ int mrcc_edge_plan_create(const mrcc_scene* scene, const mrcc_edge_batch* batch,
     }
     unsigned char* w = (unsigned char*)p->work_mem;
     mrcc_internal::plan_layout(batch->n_edges, sc->D, w, &p->W);
-    unsigned char* stats_mem = (unsigned char*)p->W.stats;
     if (!t.collect_stats) p->W.stats = nullptr;
-    if (t.collect_stats) HIP_OK(hipMemset(stats_mem, 0, 64));
-    HIP_OK(hipMemset(p->W.meta, 0, 64));
+    launch_plan_clear(p->W, (hipStream_t)stream);
+    HIP_OK(hipGetLastError());
     if (t.time_kernels && !t.use_graph)
         for (int i = 0; i < 4; ++i) HIP_OK(hipEventCreate(&p->ev[i]));
     if (t.use_graph && batch->n_edges > 0) {
@@ -1187,7 +1180,9 @@ int mrcc_edge_plan_run(mrcc_edge_plan* p, void* stream) {
         HIP_OK(hipGraphLaunch(p->exec, st));
     } else {
         plan_launch_sequence(p, st);
-        HIP_OK(hipGetLastError());
+        const hipError_t e = hipGetLastError();
+        p->dirty = e != hipSuccess;
+        HIP_OK(e);
     }
     return MRCC_OK;
 }
@@ -1255,9 +1250,9 @@ int mrcc_check_edges(const mrcc_scene* scene, const mrcc_edge_batch* batch, cons
         if (e != hipSuccess) rc = fail(MRCC_ERR_HIP, "edge batch: %s", hipGetErrorString(e));
     }
     mrcc_edge_plan_destroy(p);
-    if (rc == MRCC_OK && meta[2] > 0)
+    if (rc == MRCC_OK && meta[META_ERRORS] > 0)
         return fail(MRCC_ERR_INVALID, "%lld edges have N_start > N (the reference asserts) or more than %d states",
-                    meta[2], MRCC_MAX_EDGE_STATES);
+                    meta[META_ERRORS], MRCC_MAX_EDGE_STATES);
     return rc;
 }
 
@@ -1544,7 +1539,7 @@ int mrcc_check_edges_host(const mrcc_scene* scene, const double* q1, const doubl
     // ones; no more than the longest edge has states (a wave without one would only stage the scene)
     int wpe = n >= 2048 ? 1 : (int)std::min<int64_t>(64, std::max<int64_t>(1, 2048 / n));
     wpe = std::max(1, std::min(wpe, maxN));
-    launch_direct(*sc, v, nullptr, n, nullptr, wpe, 0, 32 * device_cus(), nullptr, st);
+    launch_direct(*sc, v, nullptr, n, wpe, 0, 32 * device_cus(), nullptr, st);
     HIP_OK(hipGetLastError());
     if (zc) {
         // the flag kernel runs after every wave of the check (stream order) and its write reaches

@@ -558,7 +558,8 @@ struct ArmQueue {
     unsigned long long* ticket;
     const double* dir;
     unsigned long long* stats;
-    const long long* meta;
+    long long* meta;
+    int* hist;
     long long rs;
     int ds, n, md0, incl;
     unsigned mask;
@@ -572,6 +573,15 @@ __host__ __device__ inline int batch_mode(const ArmQueue& B, long long e) {
 __host__ __device__ inline int erec_w0(int4 r) { return r.w & 0x7fffffff; }
 __host__ __device__ inline int erec_full(int4 r) { return (int)((unsigned)r.w >> 31); }
 
+// words of PlanWork.meta
+enum {
+    META_SLOTS = 0,    // queue slots
+    META_PASSES = 1,   // passes
+    META_ERRORS = 2,   // edges in error, of the finished run
+    META_MAX_S = 5,    // largest pass count so far
+    META_ERR_SUM = 6,  // edges in error so far
+};
+
 // workspace of a batched plan
 struct PlanWork {
     int4* erec;        // [n] per-edge record (N, M, S, w0 | full << 31)
@@ -579,8 +589,7 @@ struct PlanWork {
     int* hist;         // [MAX_PASSES+1]
     int* cursor;       // [MAX_PASSES+1]
     long long* pass_start;  // [MAX_PASSES+1] slot offset of each pass (G * sum E)
-    long long* meta;   // [8]: 0 total slots, 1 n_pass, 2 error count, 3 long edges, 5 largest pass count
-    int* long_list;    // [n] edges with more passes than MAX_PASSES
+    long long* meta;   // [8], META_*
     unsigned long long* ticket;  // [8 * 32]: one chunk counter per XCD, 256 bytes apart
     unsigned long long* stats;  // [8]
     double* dir;       // [n*D] (lane-per-state kinds) or null

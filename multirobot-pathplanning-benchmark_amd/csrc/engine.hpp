@@ -79,13 +79,14 @@ struct SceneRec {
     unsigned char* list_dev;
 };
 
-void launch_plan_build(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG,
+// `clear`: the workspace is not as a finished run (or launch_plan_clear) left it
+void launch_plan_build(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, bool clear,
                        hipStream_t st);
+void launch_plan_clear(const PlanWork& W, hipStream_t st);
 void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG,
                      int spt, int grid, hipStream_t st);
 void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, long long n_list,
-                   const long long* n_dev, int wpe, int init_out, int max_grid,
-                   unsigned long long* stats, hipStream_t st);
+                   int wpe, int init_out, int max_grid, unsigned long long* stats, hipStream_t st);
 // lane_looks.hip: edge batches of plane scenes with a cell table, two launches, no queue; W.meta is
 // zero before the workspace's first run (`reset`: cleared here, for workspaces used otherwise too)
 bool lane_looks_apply(const SceneRec& sc);
@@ -151,11 +152,10 @@ int tune_defaults(const SceneRec* sc, const mrcc_tune* tune, mrcc_tune* t);
 int plan_grid(const SceneRec* sc, const mrcc_tune& t);
 // Bytes of a plan's workspace for n_edges edges of D coordinates; with W, lays it out from base.
 size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W);
-void launch_long_edges(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, hipStream_t st);
-// queue build, persistent kernel and long-edge fallback on stream st
-// (lgG = MRCC_NO_QUEUE: the two launches of lane_looks.hip; `shared`: the workspace serves other runs too)
+// queue build and persistent kernel on stream st (lgG = MRCC_NO_QUEUE: the two launches of
+// lane_looks.hip); `clear` as for launch_plan_build
 void launch_plan_sequence(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, int spt,
-                          int grid, hipStream_t st, bool shared);
+                          int grid, hipStream_t st, bool clear);
 int plan_lgG(const mrcc_tune& t);
 }  // namespace mrcc_internal
 

@@ -1,15 +1,19 @@
 // kernels.hip — kernels of the collision engine (gfx950, wave64).
 //
 // Edge batches run as one pass-ordered work queue (see PlanWork):
-//   prep      : one thread per edge: N (abstract_env.py:321-323), window (:325-331), slot count M,
-//               passes S = ceil(M / G), histogram of S
-//   scan      : one block: E_p = #{edges with S > p}, pass offsets PS[p] = G * sum_{p'<p} E_p'
-//   scatter   : counting sort, edges longest-first
+//   prep      : a few lanes per edge: N (abstract_env.py:321-323), window (:325-331), slot count M,
+//               passes S = ceil(M / G) (at most MRCC_MAX_PASSES), histogram of S
+//   scatter   : E_p = #{edges with S > p}, pass offsets PS[p] = G * sum_{p'<p} E_p' (every block sums
+//               the histogram for itself); counting sort, edges longest-first
 //   persistent: waves claim chunks of queue slots from 8 XCD-interleaved counters; slot -> (pass p,
 //               rank r, k);
 //               edge = order[r]; state = k * S_e + p of the edge (coarse-to-fine: pass 0 visits G
 //               evenly spread states of every edge, later passes refine; an edge found in
-//               collision is skipped by all later slots)
+//               collision is skipped by all later slots); where S was cut, the states G S apart too
+// Each kernel clears what the one before it has used up (prep the cursors and tickets, persistent the
+// histogram and the sums), so a workspace needs clearing once and not by a launch of every run
+// (k_plan_init 4.7 us); with the sums in the scatter kernel (a launch of one block before, 4.5 us) and
+// long edges in the queue (a launch for them after, 4.0 us) a run has three launches instead of six.
 // The same state evaluators serve the direct kernels (one workgroup per edge: the plain per-call
 // form and the unsorted single-launch ablation) and the configuration kernels.
 #include "lanes.hpp"
@@ -30,13 +34,23 @@ __device__ inline int edge_N_dev(const EdgeBatchView& B, long long e, int D) {
 
 // ============================================================================================
 // queue construction
+// clears a workspace: before its first run, and before each run where it serves others too
 __global__ void k_plan_init(PlanWork W) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
     for (int b = t; b <= MRCC_MAX_PASSES; b += stride) W.hist[b] = 0;
     if (t < 8) W.meta[t] = 0;
-    if (t < 8) W.ticket[32 * t] = 0;
     if (t < 8 && W.stats) W.stats[t] = 0;
+}
+
+// the persistent kernels' part: what the next run's prep counts up from zero
+__device__ inline void plan_clear(int* hist, long long* meta) {
+    const int n_pass = (int)meta[META_PASSES];
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b <= n_pass; b += gridDim.x * blockDim.x) hist[b] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        meta[META_MAX_S] = 0;
+        meta[META_ERR_SUM] = 0;
+    }
 }
 
 // Pass counts of small edges are histogrammed in LDS first (one global atomic per block and
@@ -62,11 +76,13 @@ __device__ inline void prep_load_rows(const EdgeBatchView& B, long long e, int D
     }
 }
 
-// nm > 0: mode ids outside [0, nm) make the edge an error (verdict 0, counted in meta[2])
+// nm > 0: mode ids outside [0, nm) make the edge an error (verdict 0, counted in META_ERR_SUM)
 __global__ void __launch_bounds__(256) k_plan_prep(EdgeBatchView B, PlanWork W, int D, int lgG,
                                                    int want_dir, int lg_lpe, int nm_modes) {
     __shared__ int h[PLAN_LDS_BINS];
     __shared__ int smax;
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b <= MRCC_MAX_PASSES; b += gridDim.x * blockDim.x) W.cursor[b] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 8) W.ticket[32 * threadIdx.x] = 0;
     for (int i = threadIdx.x; i < PLAN_LDS_BINS; i += blockDim.x) h[i] = 0;
     if (threadIdx.x == 0) smax = 0;
     __syncthreads();
@@ -135,12 +151,8 @@ __global__ void __launch_bounds__(256) k_plan_prep(EdgeBatchView B, PlanWork W, 
         }
         int M = w.M;
         long long S = ((long long)M + (1 << lgG) - 1) >> lgG;
-        if (w.err) atomicAdd((unsigned long long*)&W.meta[2], 1ull);
-        if (S > MRCC_MAX_PASSES) {
-            unsigned long long slot = atomicAdd((unsigned long long*)&W.meta[3], 1ull);
-            W.long_list[slot] = (int)e;
-            S = 0;
-        }
+        if (w.err) atomicAdd((unsigned long long*)&W.meta[META_ERR_SUM], 1ull);
+        if (S > MRCC_MAX_PASSES) S = MRCC_MAX_PASSES;  // each of its slots holds several states
         W.erec[e] = make_int4(N, M, (int)S, w.w0 | (w.full << 31));
         B.out[e] = w.err ? 0 : 1;
         if (S < PLAN_LDS_BINS) atomicAdd(&h[S], 1);
@@ -156,12 +168,12 @@ __global__ void __launch_bounds__(256) k_plan_prep(EdgeBatchView B, PlanWork W, 
     __syncthreads();
     for (int i = threadIdx.x; i < PLAN_LDS_BINS; i += blockDim.x)
         if (h[i]) atomicAdd(&W.hist[i], h[i]);
-    if (threadIdx.x == 0 && smax > 0) atomicMax((unsigned long long*)&W.meta[5], (unsigned long long)smax);
+    if (threadIdx.x == 0 && smax > 0) atomicMax((unsigned long long*)&W.meta[META_MAX_S], (unsigned long long)smax);
 }
 
-// Inclusive prefix sum over the threads of a 1024-thread block: shuffles within each wave, then
-// the 16 wave totals through LDS (two barriers).
-__device__ inline long long block_prefix_1024(long long v, long long* wsum) {
+// Inclusive prefix sum over the 256 threads of a block (shuffles within each wave, then the wave
+// totals through LDS); *total: the sum over the block.
+__device__ inline long long block_prefix_256(long long v, long long* wsum, long long* total) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -170,90 +182,93 @@ __device__ inline long long block_prefix_1024(long long v, long long* wsum) {
     }
     if (lane == 63) wsum[wid] = v;
     __syncthreads();
-    long long off = 0;
-    for (int w = 0; w < wid; ++w) off += wsum[w];
+    long long off = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        if (w < wid) off += wsum[w];
+        all += wsum[w];
+    }
+    *total = all;
     __syncthreads();  // wsum is reused by the next call
     return v + off;
 }
 
-// One block of 1024 threads: E_p = number of edges with more than p passes (suffix sums of the
-// pass histogram) and the slot offset of each pass (prefix sums of E_p).  Only passes below the
-// largest pass count (written by the prep kernel) are scanned; slot lookups never read further.
-__global__ void __launch_bounds__(1024) k_plan_scan(PlanWork W, int lgG) {
-    constexpr int PER_MAX = MRCC_MAX_PASSES / 1024;
-    __shared__ long long wsum[16];
-    const int t = threadIdx.x;
-    const int maxS = (int)W.meta[5];             // largest pass count, <= MRCC_MAX_PASSES
-    const int nb = maxS + 1;                     // passes 0..maxS (E_maxS = 0)
-    const int per = (nb + 1023) / 1024;          // <= PER_MAX + 1
-    // thread t owns passes [t*per, (t+1)*per) of [0, nb), in reverse order for the suffix sums
-    long long loc[PER_MAX + 1];
-    long long s = 0;
-    for (int i = per - 1; i >= 0; --i) {
-        const int p = t * per + i;
-        s += (p < maxS) ? (long long)W.hist[p + 1] : 0;
-        loc[i] = s;  // sum_{b in (p, (t+1)*per]}
-    }
-    // suffix sums over threads: the total minus the prefix sum
-    const long long rs = block_prefix_1024(s, wsum);  // sum of s over threads <= t
-    __shared__ long long total_s;
-    if (t == 1023) total_s = rs;
-    __syncthreads();
-    const long long after = total_s - rs;             // sum of s over threads > t
-    long long esum = 0;
-    for (int i = 0; i < per; ++i) {
-        const int p = t * per + i;
-        if (p >= nb) break;
-        const long long E = loc[i] + after;
-        loc[i] = E;
-        esum += E;
-        W.cursor[p] = (int)E;  // descending-order start of bucket p
-    }
-    // exclusive prefix of E over p
-    long long run = block_prefix_1024(esum, wsum) - esum;
-    for (int i = 0; i < per; ++i) {
-        const int p = t * per + i;
-        if (p >= nb) break;
-        W.pass_start[p] = run << lgG;
-        run += loc[i];
-    }
-    // pass_start[maxS] (written above, E_maxS = 0) is the slot count; lookups never read beyond
-    if (t == 1023) {
-        W.meta[1] = maxS;
-        W.meta[0] = run << lgG;
-    }
-}
-
-// Tiles of 256 x SCATTER_EPT edges: edges of a small pass count are ranked within the tile in
-// LDS; the tile then reserves one range of the count's bucket with one global atomic.
+// Pass counts in windows of PLAN_LDS_BINS (nearly always one): every block sums the histogram,
+// E_p = edges with more than p passes = first place of the edges of p passes in the descending order;
+// block 0 also writes the slot offset of each pass (prefix sums of E_p).  Tiles of
+// 256 x SCATTER_EPT edges: a tile's edges of the window are ranked in LDS, then the tile reserves
+// one range of each count's bucket with one global atomic.
 #define SCATTER_EPT 4
 
-__global__ void __launch_bounds__(256) k_plan_scatter(PlanWork W, long long n) {
+__global__ void __launch_bounds__(256) k_plan_scatter(PlanWork W, long long n, int lgG) {
+    constexpr int BPT = PLAN_LDS_BINS / 256;
+    __shared__ int first[PLAN_LDS_BINS];
     __shared__ int cnt[PLAN_LDS_BINS];
     __shared__ int base[PLAN_LDS_BINS];
-    const long long tile_edges = (long long)blockDim.x * SCATTER_EPT;
-    for (long long t0 = (long long)blockIdx.x * tile_edges; t0 < n; t0 += (long long)gridDim.x * tile_edges) {
-        for (int i = threadIdx.x; i < PLAN_LDS_BINS; i += blockDim.x) cnt[i] = 0;
-        __syncthreads();
-        int S[SCATTER_EPT], r[SCATTER_EPT];
+    __shared__ long long wsum[4];
+    const int t = threadIdx.x;
+    const int maxS = (int)W.meta[META_MAX_S];  // <= MRCC_MAX_PASSES
+    long long s = 0, edges, below = 0, slots = 0;
+    for (int p = 1 + t; p <= maxS; p += 256) s += W.hist[p];
+    block_prefix_256(s, wsum, &edges);  // edges with passes
+    const long long tile_edges = 256 * SCATTER_EPT;
+    for (int w0 = 0; w0 <= maxS; w0 += PLAN_LDS_BINS) {
+        long long h[BPT], E[BPT], sum = 0, all;
 #pragma unroll
-        for (int k = 0; k < SCATTER_EPT; ++k) {
-            const long long e = t0 + (long long)k * blockDim.x + threadIdx.x;
-            S[k] = e < n ? W.erec[e].z : 0;
-            r[k] = (S[k] > 0 && S[k] < PLAN_LDS_BINS) ? atomicAdd(&cnt[S[k]], 1) : 0;
+        for (int j = 0; j < BPT; ++j) {
+            const int p = w0 + BPT * t + j;
+            sum += p > 0 && p <= maxS ? (long long)W.hist[p] : 0;
+            h[j] = sum;
+        }
+        const long long before = below + block_prefix_256(sum, wsum, &all) - sum;
+        below += all;
+        long long esum = 0;
+#pragma unroll
+        for (int j = 0; j < BPT; ++j) {
+            E[j] = edges - (before + h[j]);
+            first[BPT * t + j] = (int)E[j];
+            esum += w0 + BPT * t + j <= maxS ? E[j] : 0;
+        }
+        if (blockIdx.x == 0) {
+            long long at = slots + block_prefix_256(esum, wsum, &all) - esum;
+            slots += all;
+#pragma unroll
+            for (int j = 0; j < BPT; ++j) {
+                const int p = w0 + BPT * t + j;
+                if (p <= maxS) W.pass_start[p] = at << lgG;
+                at += E[j];
+            }
+        }
+        for (long long t0 = (long long)blockIdx.x * tile_edges; t0 < n; t0 += (long long)gridDim.x * tile_edges) {
+            __syncthreads();
+            for (int i = t; i < PLAN_LDS_BINS; i += 256) cnt[i] = 0;
+            __syncthreads();
+            int S[SCATTER_EPT], r[SCATTER_EPT];
+#pragma unroll
+            for (int k = 0; k < SCATTER_EPT; ++k) {
+                const long long e = t0 + (long long)k * 256 + t;
+                const int z = e < n ? W.erec[e].z : 0;
+                S[k] = z > 0 ? z - w0 : -1;
+                r[k] = S[k] >= 0 && S[k] < PLAN_LDS_BINS ? atomicAdd(&cnt[S[k]], 1) : 0;
+            }
+            __syncthreads();
+            for (int i = t; i < PLAN_LDS_BINS; i += 256)
+                if (cnt[i]) base[i] = first[i] + atomicAdd(&W.cursor[w0 + i], cnt[i]);
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < SCATTER_EPT; ++k) {
+                if (S[k] < 0 || S[k] >= PLAN_LDS_BINS) continue;
+                const int pos = base[S[k]] + r[k];
+                if (pos < n) W.order[pos] = (int)(t0 + (long long)k * 256 + t);
+            }
         }
         __syncthreads();
-        for (int i = threadIdx.x; i < PLAN_LDS_BINS; i += blockDim.x)
-            if (cnt[i]) base[i] = atomicAdd(&W.cursor[i], cnt[i]);
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < SCATTER_EPT; ++k) {
-            const long long e = t0 + (long long)k * blockDim.x + threadIdx.x;
-            if (S[k] <= 0) continue;
-            const int pos = S[k] < PLAN_LDS_BINS ? base[S[k]] + r[k] : atomicAdd(&W.cursor[S[k]], 1);
-            W.order[pos] = (int)e;
-        }
-        __syncthreads();
+    }
+    // pass_start[maxS] (E_maxS = 0) is the slot count; lookups never read beyond
+    if (blockIdx.x == 0 && t == 0) {
+        W.meta[META_PASSES] = maxS;
+        W.meta[META_SLOTS] = slots << lgG;
+        W.meta[META_ERRORS] = W.meta[META_ERR_SUM];
     }
 }
 
@@ -359,7 +374,8 @@ __global__ void __launch_bounds__(256) k_lane_persistent(View S, EdgeBatchView B
                                                          int lgG, int spt) {
     constexpr int MAXD = LaneDim<View, T1, T2>::value;
     const int D = S.D;
-    const long long T = W.meta[0];
+    const long long T = W.meta[META_SLOTS];
+    plan_clear(W.hist, W.meta);
     unsigned long long n_eval = 0, n_dead = 0, n_slots = 0;
     unsigned rechecks = 0;
     const int lane = threadIdx.x & 63;
@@ -382,17 +398,21 @@ __global__ void __launch_bounds__(256) k_lane_persistent(View S, EdgeBatchView B
             if (ref.e < 0) continue;
             if (edge_dead(B.out, ref.e)) { ++n_dead; continue; }
             EdgeWin w = win_of(W, ref.e, B.incl);
-            const int i = edge_state_index(w, ref.local, B.incl);
-            if (i < 0) continue;
             const double* a = row1(B, ref.e);
-            double q[MAXD];
+            const int step = W.erec[ref.e].z << lgG;
+            for (int local = ref.local; local < w.M; local += step) {  // once unless S was cut
+                const int i = edge_state_index(w, local, B.incl);
+                if (i < 0) continue;
+                double q[MAXD];
 #pragma unroll
-            for (int k = 0; k < MAXD; ++k)
-                if (k < D) q[k] = interp_dir_f64(a[k * B.ds], W.dir[(long long)ref.e * D + k], i);
-            ++n_eval;
-            const int mode = B.modes ? B.modes[ref.e] : 0;
-            (void)mode;
-            if (lane_collides<View, T1, T2>(S, q, B.mask, rechecks)) edge_kill(B.out, ref.e);
+                for (int k = 0; k < MAXD; ++k)
+                    if (k < D) q[k] = interp_dir_f64(a[k * B.ds], W.dir[(long long)ref.e * D + k], i);
+                ++n_eval;
+                if (lane_collides<View, T1, T2>(S, q, B.mask, rechecks)) {
+                    edge_kill(B.out, ref.e);
+                    break;
+                }
+            }
         }
     }
     if (W.stats) {
@@ -406,15 +426,13 @@ __global__ void __launch_bounds__(256) k_lane_persistent(View S, EdgeBatchView B
 // direct form: block = 64 lanes, `wpe` blocks per edge (block b -> edge b / wpe); lane-per-state
 template <class View, int T1, int T2>
 __global__ void __launch_bounds__(64) k_lane_direct(View S, EdgeBatchView B, const int* list,
-                                                    long long n_list, const long long* n_dev,
-                                                    int wpe, int init_out,
+                                                    long long n_list, int wpe, int init_out,
                                                     unsigned long long* stats) {
     constexpr int MAXD = LaneDim<View, T1, T2>::value;
     const int D = S.D;
     const int lane = threadIdx.x;
     unsigned long long n_eval = 0;
     unsigned rechecks = 0;
-    if (n_dev) n_list = *n_dev;
     const long long nblocks = n_list * wpe;
     for (long long blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
         const long long li = blk / wpe;
@@ -513,7 +531,8 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
     const ArmLds Wl = arm_lds(lds_arm, V);
     const ArmRegs R = arm_regs(V, Wl);
     const int lane = wave_lane();
-    const long long T = W.meta[0];
+    const long long T = W.meta[META_SLOTS];
+    plan_clear(W.hist, W.meta);
     const int nw = blockDim.x >> 6;
     const long long n_waves = (long long)gridDim.x * nw;
     // short queues: at most two slots per wave in one chunk each; longer ones at least 8 chunks per
@@ -530,7 +549,7 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
     unsigned recent = 0xffffu;
     const long long nchunks = (T + spt - 1) / spt;
     const int home = blockIdx.x & 7;
-    const int n_pass = (int)W.meta[1];  // passes with slots; pass_start[n_pass] = T
+    const int n_pass = (int)W.meta[META_PASSES];  // passes with slots; pass_start[n_pass] = T
     long long ps_lo = W.pass_start[0], ps_hi = W.pass_start[1];  // pass p's slots (scalar)
     // A wave takes `nb` tickets of one counter at a time (chunks c, c + 8, ...; lane l resolves
     // slot l % spt of the batch's chunk l / spt).  One ticket while the chunks hold states to
@@ -552,6 +571,7 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
         // per-edge word in one round of loads
         int e = -1, i = -1, N = 0, mode = 0, Dact = 0;
         int kl = 0;  // the slot's place among its edge's slots of the pass
+        int next = 0;  // the slot's next place in the edge after the first (0: none; S was not cut)
         int pl = p;
         bool dead = false;
         long long lo = ps_lo;
@@ -603,7 +623,9 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
                         // one slot per pass: the states of a whole edge in the binary order (any
                         // order gives the verdict; this one reaches the middle of a long edge first)
                         i = full && lgG == 0 ? w.first + bfs_index(Mv, local) : edge_state_index(w, local, B.incl);
-                        if (i >= 0) {
+                        const int more = local + (S << lgG);
+                        next = more < Mv ? more : 0;
+                        if (i >= 0 || next) {
                             e = ee;
                             N = Nv;
                             mode = md0;
@@ -666,7 +688,8 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
         unsigned long long tk = 0;
         if (lane == 0 && c_first < nchunks) tk = atomicAdd(W.ticket + 32 * x, (unsigned long long)nb_next);
         while (jn >= 0) {
-            const int jc = jn, ej = en, ij = in_, mj = mn;
+            const int jc = jn, ej = en, mj = mn;
+            int ij = in_, nx = __builtin_amdgcn_readlane(next, jc);
             const double aj = an, dj = dn;
             jn = next_slot();
             if (jn >= 0) {
@@ -685,11 +708,28 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
                 ++n_dead;
                 continue;
             }
-            const double qv = interp_dir_f64(aj, dj, ij);  // lanes >= D: unused
-            ++n_eval;
-            const bool col = arm_state_collides<GRASP, CHAIN, STATS>(V, Wl, R, qv, mj, B.mask, rechecks, cnt,
-                                                                     __builtin_popcount(recent & 0xffffu) >= 8);
-            recent = (recent << 1) | (col ? 1u : 0u);
+            bool col = false;
+            for (;;) {
+                if (ij >= 0) {
+                    const double qv = interp_dir_f64(aj, dj, ij);  // lanes >= D: unused
+                    ++n_eval;
+                    col = arm_state_collides<GRASP, CHAIN, STATS>(V, Wl, R, qv, mj, B.mask, rechecks, cnt,
+                                                                  __builtin_popcount(recent & 0xffffu) >= 8);
+                    recent = (recent << 1) | (col ? 1u : 0u);
+                }
+                if (col || nx == 0) break;
+                const int4 rec = W.erec[ej];  // S was cut: the slot's further states
+                EdgeWin w;
+                w.N = rec.x;
+                w.w0 = erec_w0(rec);
+                w.M = rec.y;
+                w.full = erec_full(rec);
+                w.first = B.incl ? 0 : 1;
+                w.err = 0;
+                ij = w.full && lgG == 0 ? w.first + bfs_index(w.M, nx) : edge_state_index(w, nx, B.incl);
+                nx += rec.z << lgG;
+                if (nx >= rec.y) nx = 0;
+            }
             if (col) {
                 if (lane == 0) edge_kill(B.out, ej);
                 deadm |= __ballot(e == ej);
@@ -731,14 +771,9 @@ __global__ void __launch_bounds__(GRASP ? 64 * MRCC_PERSISTENT_GRASP_NW : 256, G
 // "exception => collision"); entry points with host-side mode ids reject them before launching.
 template <bool GRASP, bool CHAIN>
 __global__ void __launch_bounds__(256) k_arm_direct(ArmK V, EdgeBatchView B, const int* list,
-                                                    long long n_list, const long long* n_dev,
-                                                    int wpe, int init_out,
+                                                    long long n_list, int wpe, int init_out,
                                                     unsigned long long* stats) {
     extern __shared__ double lds_arm[];
-    if (n_dev) {
-        n_list = *n_dev;
-        if (n_list == 0) return;  // no long edges: before the scene is staged
-    }
     arm_stage_scene(lds_arm, V);
     const ArmLds Wl = arm_lds(lds_arm, V);
     const ArmRegs R = arm_regs(V, Wl);
@@ -1254,10 +1289,12 @@ static int grid_for(long long n, int block) {
     return (int)(g < 1 ? 1 : g);
 }
 
-void launch_plan_build(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG,
+void launch_plan_clear(const PlanWork& W, hipStream_t st) { k_plan_init<<<64, 256, 0, st>>>(W); }
+
+void launch_plan_build(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, bool clear,
                        hipStream_t st) {
     const int want_dir = 1;
-    k_plan_init<<<64, 256, 0, st>>>(W);
+    if (clear) launch_plan_clear(W, st);
     // 4 lanes per edge (fewer for D < 4): measured faster than one group of >= D lanes, whose
     // per-edge tail runs on one lane of a wide group; a few edges per group, so each block's LDS
     // histogram covers many edges
@@ -1269,8 +1306,7 @@ void launch_plan_build(const SceneRec& sc, const EdgeBatchView& B, const PlanWor
     if (gs > 1024) gs = 1024;
     k_plan_prep<<<gp, 256, 0, st>>>(B, W, sc.D, lgG, want_dir, lg_lpe, sc.kind == KIND_ARMS ? sc.arm.nm : 0);
     if (arm_screen_applies(sc, B.n, MRCC_SCREEN_MIN_EDGES)) launch_screen_edges(sc, B, W, lgG, st);
-    k_plan_scan<<<1, 1024, 0, st>>>(W, lgG);
-    k_plan_scatter<<<gs, 256, 0, st>>>(W, B.n);
+    k_plan_scatter<<<gs, 256, 0, st>>>(W, B.n, lgG);
 }
 
 void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG,
@@ -1300,6 +1336,7 @@ void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork&
             Q.dir = W.dir;
             Q.stats = W.stats;
             Q.meta = W.meta;
+            Q.hist = W.hist;
             Q.rs = B.rs;
             Q.ds = (int)B.ds;
             Q.n = (int)B.n;
@@ -1335,16 +1372,15 @@ void launch_fill_u8(unsigned char* p, long long n, unsigned char v, hipStream_t 
 }
 
 void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, long long n_list,
-                   const long long* n_dev, int wpe, int init_out, int max_grid,
-                   unsigned long long* stats, hipStream_t st) {
-    long long blocks = n_dev ? (long long)max_grid : n_list * wpe;
+                   int wpe, int init_out, int max_grid, unsigned long long* stats, hipStream_t st) {
+    const long long blocks = n_list * wpe;
     int grid = (int)(blocks < max_grid ? blocks : max_grid);
     if (grid < 1) grid = 1;
     switch (sc.kind) {
         case KIND_DISKS:
         case KIND_PLANAR:
             lane_dispatch(sc, [&](auto view, auto t1, auto t2) {
-                k_lane_direct<decltype(view), t1, t2><<<grid, 64, 0, st>>>(view, B, list, n_list, n_dev, wpe, init_out, stats);
+                k_lane_direct<decltype(view), t1, t2><<<grid, 64, 0, st>>>(view, B, list, n_list, wpe, init_out, stats);
             });
             break;
         case KIND_ARMS: {
@@ -1353,7 +1389,7 @@ void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, 
             const int nw = grid < sc.arm_nw ? 1 : sc.arm_nw;
             const size_t lds = nw == 1 ? sc.arm_lds1 : sc.arm_lds;
             const int blocks = (grid + nw - 1) / nw;
-#define MRCC_ARM_DIRECT(G, C) k_arm_direct<G, C><<<blocks, 64 * nw, lds, st>>>(sc.armk, B, list, n_list, n_dev, wpe, init_out, stats)
+#define MRCC_ARM_DIRECT(G, C) k_arm_direct<G, C><<<blocks, 64 * nw, lds, st>>>(sc.armk, B, list, n_list, wpe, init_out, stats)
             if (sc.arm.chain) {
                 if (sc.arm_has_grasp) MRCC_ARM_DIRECT(true, true);
                 else MRCC_ARM_DIRECT(false, true);

@@ -24,7 +24,7 @@
 // Counters of a run (PlanWork.meta): a run uses the pair (items, errors) of its parity; the parity
 // goes from run to run through two words, each written by the kernel that does not read it, and
 // k_lane_items clears the other pair.  So a workspace needs clearing once, not once per run.
-enum { LOOK_EPOCH = 0, LOOK_EPOCH2 = 1, LOOK_ERRORS = 2, LOOK_PAIR = 3 };
+enum { LOOK_EPOCH = 0, LOOK_EPOCH2 = 1, LOOK_PAIR = 3 };
 __device__ inline long long* look_pair(const PlanWork& W, long long epoch) { return W.meta + LOOK_PAIR + 2 * (epoch & 1); }
 
 // items (waves) of an edge of R rounds
@@ -196,7 +196,7 @@ __global__ void __launch_bounds__(64 * LOOK_NW) k_lane_items(View S, EdgeBatchVi
     const long long n = pair[0] < W.items_cap ? pair[0] : W.items_cap;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         long long* other = look_pair(W, epoch + 1);
-        W.meta[LOOK_ERRORS] = pair[1];
+        W.meta[META_ERRORS] = pair[1];
         other[0] = 0;
         other[1] = 0;
         W.meta[LOOK_EPOCH] = epoch + 1;

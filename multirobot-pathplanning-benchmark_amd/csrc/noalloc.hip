@@ -94,7 +94,7 @@ extern "C" int mrcc_check_edges_noalloc(const mrcc_scene* scene, const mrcc_edge
         mrcc_internal::launch_plan_sequence(*sc, B, W, mrcc_internal::plan_lgG(t), t.slots_per_ticket,
                                             mrcc_internal::plan_grid(sc, t), st, true);
     }
-    if (n_invalid) k_store_count<<<1, 64, 0, st>>>(batch->n_edges > 0 ? W.meta + 2 : nullptr, n_invalid);
+    if (n_invalid) k_store_count<<<1, 64, 0, st>>>(batch->n_edges > 0 ? W.meta + META_ERRORS : nullptr, n_invalid);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return mrcc_internal::fail(MRCC_ERR_HIP, "launch: %s", hipGetErrorString(e));
     return MRCC_OK;

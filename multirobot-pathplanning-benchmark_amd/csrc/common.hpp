@@ -549,14 +549,15 @@ __host__ __device__ inline int batch_mode(const EdgeBatchView& B, long long e) {
 // EdgeBatchView and PlanWork they use, under the same names (fewer scalar registers than both).
 struct ArmQueue {
     const double* q1;
+    const double* q2;
     const int* idx1;
+    const int* idx2;
     const int* modes;
     unsigned char* out;
     const int4* erec;
     const int* order;
     const long long* pass_start;
     unsigned long long* ticket;
-    const double* dir;
     unsigned long long* stats;
     long long* meta;
     int* hist;
@@ -592,7 +593,7 @@ struct PlanWork {
     long long* meta;   // [8], META_*
     unsigned long long* ticket;  // [8 * 32]: one chunk counter per XCD, 256 bytes apart
     unsigned long long* stats;  // [8]
-    double* dir;       // [n*D] (lane-per-state kinds) or null
+    double* dir;       // [n*D] steps (b - a) / (N - 1) of disk and planar scenes
     // lane_looks.hip uses meta in its own way and this list, in the place of erec .. pass_start
     int2* items;       // (edge, part) of long edges
     long long items_cap;

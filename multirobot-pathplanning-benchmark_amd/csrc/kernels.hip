@@ -76,13 +76,12 @@ __device__ inline void prep_load_rows(const EdgeBatchView& B, long long e, int D
     }
 }
 
-// nm > 0: mode ids outside [0, nm) make the edge an error (verdict 0, counted in META_ERR_SUM)
+// (disk and planar scenes)
 __global__ void __launch_bounds__(256) k_plan_prep(EdgeBatchView B, PlanWork W, int D, int lgG,
-                                                   int want_dir, int lg_lpe, int nm_modes) {
+                                                   int lg_lpe) {
     __shared__ int h[PLAN_LDS_BINS];
     __shared__ int smax;
-    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b <= MRCC_MAX_PASSES; b += gridDim.x * blockDim.x) W.cursor[b] = 0;
-    if (blockIdx.x == 0 && threadIdx.x < 8) W.ticket[32 * threadIdx.x] = 0;
+    plan_prep_clear(W);
     for (int i = threadIdx.x; i < PLAN_LDS_BINS; i += blockDim.x) h[i] = 0;
     if (threadIdx.x == 0) smax = 0;
     __syncthreads();
@@ -92,10 +91,9 @@ __global__ void __launch_bounds__(256) k_plan_prep(EdgeBatchView B, PlanWork W, 
     const long long per_grid = (long long)gridDim.x * (blockDim.x >> lg_lpe);
     // the lanes of a group share e, so they run the same iterations and their shuffles stay within
     // active lanes
-    const bool need_rows = (!B.N && B.N0 <= 0) || (want_dir && W.dir);
     const long long e_first = (long long)blockIdx.x * (blockDim.x >> lg_lpe) + (threadIdx.x >> lg_lpe);
     double an[PREP_MAXC], bn[PREP_MAXC];  // rows of the next edge
-    if (need_rows && e_first < B.n) prep_load_rows(B, e_first, D, sub, lg_lpe, an, bn);
+    if (e_first < B.n) prep_load_rows(B, e_first, D, sub, lg_lpe, an, bn);
     for (long long e = e_first; e < B.n; e += per_grid) {
         double av[PREP_MAXC], bv[PREP_MAXC];
 #pragma unroll
@@ -103,7 +101,7 @@ __global__ void __launch_bounds__(256) k_plan_prep(EdgeBatchView B, PlanWork W, 
             av[j] = an[j];
             bv[j] = bn[j];
         }
-        if (need_rows && e + per_grid < B.n) prep_load_rows(B, e + per_grid, D, sub, lg_lpe, an, bn);
+        if (e + per_grid < B.n) prep_load_rows(B, e + per_grid, D, sub, lg_lpe, an, bn);
         int N;
         if (B.N || B.N0 > 0) {
             N = B.N ? B.N[e] : B.N0;
@@ -127,28 +125,15 @@ __global__ void __launch_bounds__(256) k_plan_prep(EdgeBatchView B, PlanWork W, 
             m = __shfl(m, 0, lpe);
             N = edge_N_from_max(m, B.res);
         }
-        if (want_dir && W.dir) {
-            const double den = (double)(N - 1);
 #pragma unroll
-            for (int j = 0; j < PREP_MAXC; ++j) {
-                const int k = sub + (j << lg_lpe);
-                if (k < D) {
-#pragma clang fp contract(off)
-                    W.dir[e * D + k] = (bv[j] - av[j]) / den;
-                }
-            }
+        for (int j = 0; j < PREP_MAXC; ++j) {
+            const int k = sub + (j << lg_lpe);
+            if (k < D) W.dir[e * D + k] = interp_step_f64(av[j], bv[j], N);
         }
         if (sub != 0) continue;
         const int ns = batch_N_start(B, e);
         const int nm = batch_N_max(B, e);
         EdgeWin w = edge_window(N, ns, nm, B.incl);
-        if (nm_modes > 0) {
-            const int md = batch_mode(B, e);
-            if (md < 0 || md >= nm_modes) {
-                w.err = 1;
-                w.M = 0;
-            }
-        }
         int M = w.M;
         long long S = ((long long)M + (1 << lgG) - 1) >> lgG;
         if (w.err) atomicAdd((unsigned long long*)&W.meta[META_ERR_SUM], 1ull);
@@ -165,6 +150,115 @@ __global__ void __launch_bounds__(256) k_plan_prep(EdgeBatchView B, PlanWork W, 
         mymax = u > mymax ? u : mymax;
     }
     if ((threadIdx.x & 63) == 0 && mymax > 0) atomicMax(&smax, mymax);
+    __syncthreads();
+    for (int i = threadIdx.x; i < PLAN_LDS_BINS; i += blockDim.x)
+        if (h[i]) atomicAdd(&W.hist[i], h[i]);
+    if (threadIdx.x == 0 && smax > 0) atomicMax((unsigned long long*)&W.meta[META_MAX_S], (unsigned long long)smax);
+}
+
+// Records of arm edges, as k_plan_prep forms them, without steps (each state's wave divides for
+// itself).  Bound by reading the rows once.  A wave takes `rounds` x 16 edges: the absolute differences of
+// 16 edges' rows go to LDS (FLAT: the rows are one run of 16-byte words, all requested before the
+// first is used), four lanes reduce an edge, and then a lane per edge forms the record.
+// 131,072 edges of 28 coordinates (59 MB): 14.0 us, four lanes per edge loading 8 bytes each 17.4 us (22.7
+// with the steps written); 132,587 of 56 (119 MB): 27.8, 34.9, 42.3.
+// Workgroups of 8 waves and no more than needed: each adds its pass counts to the same few global
+// words (16 edges per wave, 2,048 workgroups of 4: 30 us).
+#define REC_NW 8
+#define REC_EDGES 16
+#define REC_ROUNDS 4
+template <bool FLAT>
+__global__ void __launch_bounds__(64 * REC_NW) k_arm_records(EdgeBatchView B, PlanWork W, int D, int lgG, int nm, int rounds) {
+    extern __shared__ double s_diff[];
+    __shared__ int h[PLAN_LDS_BINS];
+    __shared__ int smax;
+    plan_prep_clear(W);
+    for (int i = threadIdx.x; i < PLAN_LDS_BINS; i += blockDim.x) h[i] = 0;
+    if (threadIdx.x == 0) smax = 0;
+    __syncthreads();
+    const int lane = wave_lane(), wid = threadIdx.x >> 6, r = lane & 3, stride = D | 1;
+    double* d = s_diff + (size_t)wid * REC_EDGES * stride;
+    const float inv = 1.0f / (float)D;  // element t < 1024 of a run is in row (t + 0.5) / D
+    int max_s = 0;
+    const long long per_grid = (long long)gridDim.x * REC_NW * REC_EDGES * rounds;
+    for (long long base = ((long long)blockIdx.x * REC_NW + wid) * (REC_EDGES * rounds); base < B.n; base += per_grid) {
+        int N = B.N0;
+        if (!B.N && N <= 0) {
+            double own = 0.0;
+            for (int j = 0; j < rounds; ++j) {
+                const long long e0 = base + REC_EDGES * j;
+                if (e0 >= B.n) break;
+                const int cnt = B.n - e0 < REC_EDGES ? (int)(B.n - e0) : REC_EDGES;
+                wave_sync();  // the previous round's differences have been read
+                if constexpr (FLAT) {
+                    constexpr int U = REC_EDGES * MRCC_MAX_D / 2 / 64;
+                    const double2* a = (const double2*)(B.q1 + e0 * D);
+                    const double2* b = (const double2*)(B.q2 + e0 * D);
+                    const int words = cnt * D / 2;
+                    double2 x[U], y[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        if (64 * u >= words) break;  // wave-uniform
+                        const int t = lane + 64 * u;
+                        x[u] = a[t < words ? t : 0];
+                        y[u] = b[t < words ? t : 0];
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        if (64 * u >= words) break;
+                        const int t = lane + 64 * u, row = (int)(((float)(2 * t) + 0.5f) * inv);
+                        if (t < words) {  // D is even: both in one row
+                            d[row * stride + 2 * t - row * D] = __builtin_fabs(x[u].x - y[u].x);
+                            d[row * stride + 2 * t + 1 - row * D] = __builtin_fabs(x[u].y - y[u].y);
+                        }
+                    }
+                } else {
+#pragma unroll 4
+                    for (int t = lane; t < cnt * D; t += 64) {
+                        const int row = (int)(((float)t + 0.5f) * inv), k = t - row * D;
+                        d[row * stride + k] = __builtin_fabs(row1(B, e0 + row)[k * B.ds] - row2(B, e0 + row)[k * B.ds]);
+                    }
+                }
+                wave_sync();
+                double m = 0.0;
+                if (lane >> 2 < cnt) {
+                    // edge_N_dev's rule: a NaN in coordinate 0 sticks (lane 0 of the four starts from it), a
+                    // NaN elsewhere is skipped
+                    const double* v = d + (lane >> 2) * stride;
+                    if (r == 0) m = v[0];
+                    for (int k = r ? r : 4; k < D; k += 4) m = v[k] > m ? v[k] : m;
+                }
+                double v = dpp_f64<0xb1>(m);
+                m = v > m ? v : m;
+                v = dpp_f64<0x4e>(m);
+                m = v > m ? v : m;
+                v = __shfl(m, 4 * (lane & 15), 64);
+                own = lane >> 4 == j ? v : own;
+            }
+            N = edge_N_from_max(own, B.res);
+        }
+        const long long e = base + lane;
+        const bool in = lane < REC_EDGES * rounds && e < B.n;
+        int S = 0;
+        bool err = false;
+        if (in) {
+            if (B.N) N = B.N[e];
+            const EdgeWin w = edge_window(N, batch_N_start(B, e), batch_N_max(B, e), B.incl);
+            const int md = batch_mode(B, e);
+            err = w.err || md < 0 || md >= nm;
+            const int M = err ? 0 : w.M;
+            S = min((int)(((long long)M + (1 << lgG) - 1) >> lgG), MRCC_MAX_PASSES);
+            W.erec[e] = make_int4(N, M, S, w.w0 | (w.full << 31));
+            B.out[e] = err ? 0 : 1;
+            if (S < PLAN_LDS_BINS) atomicAdd(&h[S], 1);
+            else atomicAdd(&W.hist[S], 1);
+        }
+        const unsigned long long bad = __ballot(err);
+        if (bad && lane == 0) atomicAdd((unsigned long long*)&W.meta[META_ERR_SUM], (unsigned long long)__popcll(bad));
+        max_s = max(max_s, S);
+    }
+    for (int o = 32; o >= 1; o >>= 1) max_s = max(max_s, __shfl_xor(max_s, o, 64));
+    if (lane == 0 && max_s > 0) atomicMax(&smax, max_s);
     __syncthreads();
     for (int i = threadIdx.x; i < PLAN_LDS_BINS; i += blockDim.x)
         if (h[i]) atomicAdd(&W.hist[i], h[i]);
@@ -671,16 +765,17 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
             }
         };
         int jn = next_slot();
-        int en = -1, in_ = 0, mn = 0;
-        double an = 0.0, dn = 0.0;
+        int en = -1, in_ = 0, mn = 0, nn = 2;
+        double an = 0.0, dn = 0.0;  // coordinate `lane` of the next slot's two rows
         if (jn >= 0) {
             en = __builtin_amdgcn_readlane(e, jn);
             in_ = __builtin_amdgcn_readlane(i, jn);
             mn = __builtin_amdgcn_readlane(mode, jn);
             const int Dn = __builtin_amdgcn_readlane(Dact, jn);
+            nn = __builtin_amdgcn_readlane(N, jn);
             if (lane < Dn) {
                 an = row1(B, en)[lane * B.ds];
-                dn = W.dir[(long long)en * V.D + lane];
+                dn = row2(B, en)[lane * B.ds];
             }
         }
         const int nb_next = jn >= 0 ? 1 : (2 * nb < nb_max ? 2 * nb : nb_max);
@@ -690,24 +785,27 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
         while (jn >= 0) {
             const int jc = jn, ej = en, mj = mn;
             int ij = in_, nx = __builtin_amdgcn_readlane(next, jc);
-            const double aj = an, dj = dn;
+            const double aj = an, bj = dn;
+            const int Nj = nn;
             jn = next_slot();
             if (jn >= 0) {
                 en = __builtin_amdgcn_readlane(e, jn);
                 in_ = __builtin_amdgcn_readlane(i, jn);
                 mn = __builtin_amdgcn_readlane(mode, jn);
                 const int Dn = __builtin_amdgcn_readlane(Dact, jn);
+                nn = __builtin_amdgcn_readlane(N, jn);
                 an = 0.0;
                 dn = 0.0;
                 if (lane < Dn) {
                     an = row1(B, en)[lane * B.ds];
-                    dn = W.dir[(long long)en * V.D + lane];
+                    dn = row2(B, en)[lane * B.ds];
                 }
             }
             if ((deadm >> jc) & 1ull) {  // picked before its edge was found in collision
                 ++n_dead;
                 continue;
             }
+            const double dj = interp_step_f64(aj, bj, Nj);
             bool col = false;
             for (;;) {
                 if (ij >= 0) {
@@ -1289,24 +1387,33 @@ static int grid_for(long long n, int block) {
     return (int)(g < 1 ? 1 : g);
 }
 
+static int plan_blocks(long long n, int per_block) { return std::min(grid_for(n, per_block), 1024); }
+
 void launch_plan_clear(const PlanWork& W, hipStream_t st) { k_plan_init<<<64, 256, 0, st>>>(W); }
 
 void launch_plan_build(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, bool clear,
                        hipStream_t st) {
-    const int want_dir = 1;
     if (clear) launch_plan_clear(W, st);
+    if (sc.kind == KIND_ARMS) {
+        int rounds = 1;  // 64 edges per wave once that leaves two waves per SIMD
+        while (rounds < REC_ROUNDS && B.n >= (long long)REC_EDGES * 2 * rounds * 2048) rounds *= 2;
+        const int D = sc.D, blocks = std::min(grid_for(B.n, REC_NW * REC_EDGES * rounds), 512);
+        const size_t lds = sizeof(double) * REC_NW * REC_EDGES * (D | 1);
+        const bool flat = B.rs == D && B.ds == 1 && !B.idx1 && !B.idx2 && (D & 1) == 0 &&
+                          (((uintptr_t)B.q1 | (uintptr_t)B.q2) & 15) == 0;
+        if (flat) k_arm_records<true><<<blocks, 64 * REC_NW, lds, st>>>(B, W, D, lgG, sc.arm.nm, rounds);
+        else k_arm_records<false><<<blocks, 64 * REC_NW, lds, st>>>(B, W, D, lgG, sc.arm.nm, rounds);
+        if (arm_screen_applies(sc, B.n, MRCC_SCREEN_MIN_EDGES)) launch_screen_edges(sc, B, W, lgG, st);
+        k_plan_scatter<<<plan_blocks(B.n, 256 * SCATTER_EPT), 256, 0, st>>>(W, B.n, lgG);
+        return;
+    }
     // 4 lanes per edge (fewer for D < 4): measured faster than one group of >= D lanes, whose
     // per-edge tail runs on one lane of a wide group; a few edges per group, so each block's LDS
     // histogram covers many edges
     const int lg_lpe = sc.D > 32 ? 3 : (sc.D >= 4 ? 2 : (sc.D >= 2 ? 1 : 0));
     // D <= MRCC_MAX_D = 64 = PREP_MAXC << 3, so every coordinate has a register in k_plan_prep
-    int gp = grid_for(B.n, 4 * (256 >> lg_lpe));
-    if (gp > 1024) gp = 1024;
-    int gs = grid_for(B.n, 256 * SCATTER_EPT);
-    if (gs > 1024) gs = 1024;
-    k_plan_prep<<<gp, 256, 0, st>>>(B, W, sc.D, lgG, want_dir, lg_lpe, sc.kind == KIND_ARMS ? sc.arm.nm : 0);
-    if (arm_screen_applies(sc, B.n, MRCC_SCREEN_MIN_EDGES)) launch_screen_edges(sc, B, W, lgG, st);
-    k_plan_scatter<<<gs, 256, 0, st>>>(W, B.n, lgG);
+    k_plan_prep<<<plan_blocks(B.n, 4 * (256 >> lg_lpe)), 256, 0, st>>>(B, W, sc.D, lgG, lg_lpe);
+    k_plan_scatter<<<plan_blocks(B.n, 256 * SCATTER_EPT), 256, 0, st>>>(W, B.n, lgG);
 }
 
 void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG,
@@ -1333,7 +1440,8 @@ void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork&
             Q.order = W.order;
             Q.pass_start = W.pass_start;
             Q.ticket = W.ticket;
-            Q.dir = W.dir;
+            Q.q2 = B.q2;
+            Q.idx2 = B.idx2;
             Q.stats = W.stats;
             Q.meta = W.meta;
             Q.hist = W.hist;

@@ -24,6 +24,17 @@ __device__ inline const double* row2(const EdgeBatchView& B, long long e) {
     return B.q2 + r * B.rs;
 }
 
+__device__ inline const double* row2(const ArmQueue& B, long long e) {
+    long long r = B.idx2 ? (long long)B.idx2[e] : e;
+    return B.q2 + r * B.rs;
+}
+
+// What the kernel that forms a queue's records clears for the kernels after it.
+__device__ inline void plan_prep_clear(const PlanWork& W) {
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b <= MRCC_MAX_PASSES; b += gridDim.x * blockDim.x) W.cursor[b] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 8) W.ticket[32 * threadIdx.x] = 0;
+}
+
 // interpolated state (abstract_env.py:341, :348): q1 + ((q2 - q1) / (N - 1)) * i, unfused
 __device__ inline double interp_f64(double a, double b, int N, int i) {
 #pragma clang fp contract(off)

@@ -8,9 +8,7 @@
 // to binary32, d^2 - (r_i + r_j)^2 < -M), so a state it reports collides by the binary64 predicate
 // too.  States it does not report go on to the full evaluator, which decides alone; the booleans are
 // the same with and without the screen.
-#include "engine.hpp"
-
-using namespace mrcc;
+#include "lanes.hpp"
 
 #define SCREEN_ITEMS 16       // (state, arm) items per wave and step
 #define SCREEN_QUEUE 80       // pending items: 15 left over + one chunk of 64
@@ -28,7 +26,8 @@ __host__ __device__ inline int screen_wave_bytes(int dof) {
 struct ScreenArgs {
     const double* q1;   // rows of the configurations, or of the edges' first ends
     const int* idx1;
-    const double* dir;  // EDGES: the edges' steps [n*D]
+    const double* q2;   // EDGES: rows of the second ends
+    const int* idx2;
     int4* erec;         // EDGES: per-edge records
     int* hist;          // EDGES: pass histogram
     unsigned long long* stats;
@@ -72,12 +71,12 @@ __device__ inline unsigned long long screen_step(const ArmK& V, const ArmLds& W,
     const double* row = A.q1 + (A.idx1 ? (long long)A.idx1[id] : id) * A.rs;
     double qv[2];
     if constexpr (EDGES) {
-        const double fi = (double)(ent.y & 0xffffff);
+        const double* end = A.q2 + (A.idx2 ? (long long)A.idx2[id] : id) * A.rs;
+        const int N = A.erec[id].x;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-#pragma clang fp contract(off)
             const int k = r + 4 * h, c = a * dof + (k < dof ? k : 0);
-            qv[h] = row[c * A.ds] + A.dir[id * V.D + c] * fi;
+            qv[h] = interp_f64(row[c * A.ds], end[c * A.ds], N, ent.y & 0xffffff);
         }
     } else {
 #pragma unroll
@@ -387,7 +386,8 @@ void launch_screen_edges(const SceneRec& sc, const EdgeBatchView& B, const PlanW
     ScreenArgs A;
     A.q1 = B.q1;
     A.idx1 = B.idx1;
-    A.dir = W.dir;
+    A.q2 = B.q2;
+    A.idx2 = B.idx2;
     A.erec = W.erec;
     A.hist = W.hist;
     A.stats = W.stats;
@@ -408,7 +408,8 @@ void launch_screen_configs(const SceneRec& sc, const double* q, long long n, lon
     ScreenArgs A;
     A.q1 = q;
     A.idx1 = nullptr;
-    A.dir = nullptr;
+    A.q2 = nullptr;
+    A.idx2 = nullptr;
     A.erec = nullptr;
     A.hist = nullptr;
     A.stats = nullptr;

@@ -92,3 +92,32 @@ def test_long_edges_at_one_slot_per_pass():
     a = near_home(rng, desc, 6, 0.3)
     b = a + 0.17 * np.sign(rng.normal(size=a.shape))
     assert np.array_equal(gpu_edges(sc, a, b, 1e-5), o.check_edges(a, b, 1e-5))
+
+
+# records of arm edges: rows as one run of words (strided, indexed, odd and misaligned rows not), a
+# wave's last edges missing, every coordinate count up to the largest, batches beyond one pass of the grid
+@pytest.mark.parametrize("n_arms,dof,n", [(1, 1, 70), (1, 7, 2000), (2, 3, 1), (3, 6, 65), (8, 8, 3001), (2, 1, 270001)])
+@pytest.mark.parametrize("layout", ["rows", "columns", "offset", "index"])
+def test_records(n_arms, dof, n, layout):
+    rng = np.random.default_rng(n + dof)
+    desc = scenes.quad_arms(rng=rng, n_arms=n_arms, dof=dof, n_boxes=3)
+    sc, o = backend().Scene(desc), O.Scene(desc)
+    D = desc.dim
+    a, b = _edges(rng, desc, n, 0.3)
+    if D > 1 and n > 8:
+        a[5, 1] = np.nan  # skipped in the length, a collision at every state
+    ref = o.check_edges(a, b, 0.1)
+    ta, tb = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    kw = {}
+    if layout == "columns":
+        ta, tb = ta.t().contiguous().t(), tb.t().contiguous().t()
+    elif layout == "offset":  # 8 bytes past a 16-byte word
+        ta, tb = (torch.cat([t.new_zeros(1), t.flatten()])[1:].view(n, D) for t in (ta, tb))
+    elif layout == "index":
+        perm = torch.randperm(n, device="cuda")
+        inv = torch.argsort(perm).to(torch.int32)
+        ta, tb, kw = ta[perm], tb[perm], dict(idx1=inv, idx2=inv)
+    out = torch.full((n,), 7, dtype=torch.uint8, device="cuda")
+    sc.check_edges_device(sc.edge_batch(ta, tb, out, 0.1, **kw))
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), ref.astype(np.uint8))

@@ -713,8 +713,7 @@ size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W) {
     };
     const size_t o_rec = sz(16 * n), o_order = sz(4 * n), o_hist = sz(4 * (MRCC_MAX_PASSES + 1)),
                  o_cur = sz(4 * (MRCC_MAX_PASSES + 1)), o_ps = sz(8 * (MRCC_MAX_PASSES + 1)), o_meta = sz(8 * 8),
-                 o_spare = sz(4 * n), o_tick = sz(8 * 32 * 8), o_stats = sz(8 * 8), o_dir = sz(8 * (size_t)n * D);
-    (void)o_spare;  // keeps the size that the no-allocation entry point's limit is stated by
+                 o_long = sz(4 * n), o_tick = sz(8 * 32 * 8), o_stats = sz(8 * 8), o_dir = sz(8 * (size_t)n * D);
     if (W) {
         W->erec = (int4*)(base + o_rec);
         W->order = (int*)(base + o_order);
@@ -722,6 +721,7 @@ size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W) {
         W->cursor = (int*)(base + o_cur);
         W->pass_start = (long long*)(base + o_ps);
         W->meta = (long long*)(base + o_meta);
+        W->long_list = (int*)(base + o_long);
         W->ticket = (unsigned long long*)(base + o_tick);
         W->stats = (unsigned long long*)(base + o_stats);
         W->dir = (double*)(base + o_dir);

@@ -591,6 +591,8 @@ struct PlanWork {
     int* cursor;       // [MAX_PASSES+1]
     long long* pass_start;  // [MAX_PASSES+1] slot offset of each pass (G * sum E)
     long long* meta;   // [8], META_*
+    int* long_list;    // [n] unused: its place keeps the size that the no-allocation check's limit is
+                       // stated by
     unsigned long long* ticket;  // [8 * 32]: one chunk counter per XCD, 256 bytes apart
     unsigned long long* stats;  // [8]
     double* dir;       // [n*D] steps (b - a) / (N - 1) of disk and planar scenes

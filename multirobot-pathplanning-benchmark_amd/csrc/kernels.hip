@@ -629,10 +629,13 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
     plan_clear(W.hist, W.meta);
     const int nw = blockDim.x >> 6;
     const long long n_waves = (long long)gridDim.x * nw;
-    // short queues: at most two slots per wave in one chunk each; longer ones at least 8 chunks per
-    // wave, so that no wave still evaluates a chunk's states one after another when others are done
+    // Chunks of at most 8 slots below 192 slots per wave: one of 16 leaves a wave alone with its live
+    // states at the end (75,065 edges of six arms, 132 slots a wave: 474 us at 16, 375 at 8, 383 at 4);
+    // longer queues pay for the round trips instead (99,840 edges of three arms, 227 slots a wave:
+    // 1,066 / 1,096 / 1,155).  Short queues: one chunk per wave, of one slot below a slot per wave.
+    if (T < 192 * n_waves) spt = min(spt, 8);
     if (T <= 2 * n_waves) spt = min(spt, T > n_waves ? 2 : 1);
-    else if (T < 8 * n_waves * spt) spt = min(spt, max(2, (int)(T / (8 * n_waves))));
+    else if (T < n_waves * spt) spt = min(spt, max(2, (int)(T / n_waves)));
     // statistics (compiled away without STATS)
     typename std::conditional<STATS, unsigned long long, NoCount>::type n_eval{}, n_dead{}, n_slots{};
     RecheckT<STATS> rechecks{};

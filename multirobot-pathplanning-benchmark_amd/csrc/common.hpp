@@ -571,6 +571,14 @@ __host__ __device__ inline int batch_mode(const ArmQueue& B, long long e) {
 }
 
 // Per-edge record of a plan: N, slot count M, passes S, window start | full << 31.
+// Chunks of an arm queue run by n_waves waves: wave w starts on chunk w, and counter x of the 8 hands
+// out this chunk as its k-th.  Together they are all chunks from 0 on, each once, for any number of waves
+// (workgroups of 3, 5, 6, 9 or 10 waves make numbers that are no multiple of 8).
+#define MRCC_QUEUE_COUNTERS 8
+__host__ __device__ inline long long queue_chunk(long long n_waves, int x, long long k) {
+    return n_waves + x + MRCC_QUEUE_COUNTERS * k;
+}
+
 __host__ __device__ inline int erec_w0(int4 r) { return r.w & 0x7fffffff; }
 __host__ __device__ inline int erec_full(int4 r) { return (int)((unsigned)r.w >> 31); }
 

@@ -388,14 +388,14 @@ __device__ inline long long claim_chunk(const WV& W, int& q, long long nchunks) 
 }
 
 // A chunk of any counter that has some left (`q`: its place after `home`, where the wave continues),
-// or -1.  The counters are read before one is drawn from: near the end of a queue every wave comes
+// or -1 (queue_chunk: the counters' chunks are those after the waves' first ones).  The counters are read before one is drawn from: near the end of a queue every wave comes
 // here, and an atomic on each drained counter in turn cost 30 us of a launch (4096 waves, 8
 // counters).  Wave-uniform, all lanes.
 template <class WV>
-__device__ inline long long steal_chunk(const WV& W, int home, int& q, long long nchunks) {
+__device__ inline long long steal_chunk(const WV& W, int home, int& q, long long n_waves, long long nchunks) {
     const int lane = threadIdx.x & 63;
     const int xl = (home + lane) & 7;
-    const long long have = (nchunks - xl + 7) >> 3;  // chunks of counter xl
+    const long long have = (nchunks - n_waves - xl + 7) >> 3;  // chunks of counter xl
     for (;;) {
         bool left = false;
         if (lane < 8)
@@ -408,7 +408,7 @@ __device__ inline long long steal_chunk(const WV& W, int home, int& q, long long
         if (lane == 0) k = atomicAdd(W.ticket + 32 * x, 1ull);
         k = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(k >> 32)) << 32) |
             (unsigned)__builtin_amdgcn_readfirstlane((unsigned)k);
-        const long long c = x + 8 * (long long)k;
+        const long long c = queue_chunk(n_waves, x, (long long)k);
         if (c < nchunks) return c;
     }
 }
@@ -655,8 +655,7 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
     const int nb_max = 64 / spt;
     const int lj = lane / spt, lo_slot = lane - lj * spt;
     int nb = 1;
-    // wave w starts on chunk w; the counters hand out the chunks after the first `c_first`
-    const long long c_first = (n_waves + 7) & ~7ll;
+    // wave w starts on chunk w; the counters hand out the others (queue_chunk)
     long long c = (long long)blockIdx.x * nw + (threadIdx.x >> 6);
     if (c >= nchunks) c = -1;
     while (c >= 0) {
@@ -784,7 +783,7 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
         const int nb_next = jn >= 0 ? 1 : (2 * nb < nb_max ? 2 * nb : nb_max);
         const int x = (home + q) & 7;
         unsigned long long tk = 0;
-        if (lane == 0 && c_first < nchunks) tk = atomicAdd(W.ticket + 32 * x, (unsigned long long)nb_next);
+        if (lane == 0 && n_waves < nchunks) tk = atomicAdd(W.ticket + 32 * x, (unsigned long long)nb_next);
         while (jn >= 0) {
             const int jc = jn, ej = en, mj = mn;
             int ij = in_, nx = __builtin_amdgcn_readlane(next, jc);
@@ -838,12 +837,11 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
         }
         const unsigned long long k = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(tk >> 32)) << 32) |
                                      (unsigned)__builtin_amdgcn_readfirstlane((unsigned)tk);
-        if (c_first >= nchunks) break;  // no chunk beyond the waves' first ones
-        c = c_first + x + 8 * (long long)k;
+        if (n_waves >= nchunks) break;  // no chunk beyond the waves' first ones
+        c = queue_chunk(n_waves, x, (long long)k);
         nb = nb_next;
         if (c >= nchunks) {  // counter x is exhausted: continue on the others
-            c = steal_chunk(W, home, q, nchunks - c_first);
-            if (c >= 0) c += c_first;
+            c = steal_chunk(W, home, q, n_waves, nchunks);
             nb = 1;
         }
     }

@@ -63,7 +63,7 @@ __device__ inline void cell_fill(CellGrid C, double hd, double slack, int i, dou
             n = CELL_HIT;
             continue;
         }
-        ++n;
+        if (n <= CELL_LIST) ++n;  // no further: 65,535 of them would read as CELL_HIT
 #pragma unroll
         for (int k = 1; k <= CELL_LIST; ++k)
             if ((int)n == k) h[k] = (unsigned short)o;

@@ -111,6 +111,13 @@ int upload(SceneRec* sc, Packer& P, size_t extra = 0, size_t* o_extra = nullptr)
 // their centre; no table (n = 0) without obstacles, beyond 65,535 of them (16-bit indices) and
 // beyond MRCC_CELL_EXTENT metres, where binary32 coordinates are too coarse for it.
 #define MRCC_CELL_EXTENT 1.0e5
+// A scene gives its table up when the cells that hold its obstacles leave more than MRCC_CELL_POOR
+// tests open each (of 8): the obstacles stand close in cells that are large because others are far off, no
+// cell is certain contact, and the look of lane_looks.hip ends no edge.  us of 200,000 edges / 200,000
+// configurations with the table and without, 4 boxes and 100 obstacles: even (0 tests) 47 / 22 and 419 / 85, in
+// two groups 40 m apart (3.8) 328 / 55 and 572 / 113, 300 m apart (7.7) 1,257 / 134 and 556 / 113, a wall of 120
+// m (7.7) 822 / 111 and 416 / 85; 16 boxes, 40 obstacles and the wall (4.3) 2,484 / 228 and 1,594 / 367.
+#define MRCC_CELL_POOR 4
 CellGrid cell_grid(const double* lo, const double* hi, double reach, long long n_obs, bool ok) {
     CellGrid C;
     memset(&C, 0, sizeof(C));
@@ -128,12 +135,28 @@ CellGrid cell_grid(const double* lo, const double* hi, double reach, long long n
 }
 size_t cell_bytes(const CellGrid& C, int robots) { return (size_t)robots * C.n * C.n * sizeof(uint4); }
 
-// Builds the table of a scene whose view is complete (on the null stream, and waits for it).
-int build_cells(const SceneRec* sc) {
-    if ((sc->kind == KIND_DISKS ? sc->disk.grid.n : sc->planar.grid.n) == 0) return MRCC_OK;
-    launch_cells(*sc, nullptr);
+// Builds the table of a scene whose view is complete (on the null stream, and waits for it); `tally`:
+// two zeroed words of the scene's memory, r_in: the robots' inscribed radii.  A robot of r_in > 2 hd + slack
+// is in certain contact in every cell that holds an obstacle's centre; with half of the robots like that no
+// scene is poor and nothing is counted (scene creation 50 us, 72 with the count read back).
+int build_cells(SceneRec* sc, int* tally, const std::vector<double>& r_in) {
+    CellGrid& C = sc->kind == KIND_DISKS ? sc->disk.grid : sc->planar.grid;
+    if (C.n == 0) return MRCC_OK;
+    static_assert(2 * MRCC_CELL_POOR >= CELL_LIST + 1, "half of the robots without a test");
+    double hd, slack;
+    cell_size(C, &hd, &slack);
+    size_t sure = 0;
+    for (double r : r_in) sure += r > 2.0 * hd + slack;
+    const bool rich = 2 * sure >= r_in.size();
+    launch_cells(*sc, rich ? nullptr : tally, nullptr);
     HIP_OK(hipGetLastError());
-    HIP_OK(hipStreamSynchronize(nullptr));
+    if (rich) {
+        HIP_OK(hipStreamSynchronize(nullptr));
+        return MRCC_OK;
+    }
+    int seen[2];
+    HIP_OK(hipMemcpy(seen, tally, sizeof(seen), hipMemcpyDeviceToHost));
+    if (seen[1] > (long long)MRCC_CELL_POOR * seen[0]) C.n = 0;
     return MRCC_OK;
 }
 
@@ -869,9 +892,9 @@ int mrcc_scene_create_disks(int n_robots, int robot_dim, const double* robot_rad
     size_t o_r = P.add(r32), o_rrT32 = P.add(rrT32), o_rrT64 = P.add(rrT64), o_sc32 = P.add(sc32),
            o_sc64 = P.add(sc64), o_srT32 = P.add(srT32), o_srT64 = P.add(srT64), o_lo32 = P.add(lo32),
            o_hi32 = P.add(hi32), o_lo64 = P.add(lo64), o_hi64 = P.add(hi64), o_rp32 = P.add(rp2_32),
-           o_rp64 = P.add(rp2_64), o_cells = 0;
+           o_rp64 = P.add(rp2_64), o_tally = P.add(std::vector<int>(2, 0)), o_cells = 0;
     double clo[2] = {1e300, 1e300}, chi[2] = {-1e300, -1e300}, reach = 0.0;
-    bool plane = rd == 2;  // non-negative sizes, finite
+    bool plane = rd == 2 && nr <= 4;  // (disk2_state), non-negative sizes, finite
     for (int i = 0; i < nr && plane; ++i) {
         plane = std::isfinite(robot_radius[i]) && robot_radius[i] >= 0.0;
         reach = std::max(reach, robot_radius[i]);
@@ -913,7 +936,8 @@ int mrcc_scene_create_disks(int n_robots, int robot_dim, const double* robot_rad
     V.rp2_32 = at<float>(d, o_rp32);
     V.rp2_64 = at<double>(d, o_rp64);
     V.grid.rec = at<uint4>(d, o_cells);
-    rc = build_cells(sc);
+    rc = build_cells(sc, (int*)((unsigned char*)d + o_tally),
+                     std::vector<double>(robot_radius, robot_radius + nr));
     if (rc != MRCC_OK) {
         (void)hipFree(sc->dev_mem);
         delete box;
@@ -963,12 +987,15 @@ int mrcc_scene_create_planar_boxes(int n_robots, const double* robot_half_extent
     sc->n_robots = nr;
     (void)hipGetDevice(&sc->device);
     Packer P;
-    size_t o_rh32 = P.add(rh32), o_rh64 = P.add(rh64), o_ob32 = P.add(ob32), o_ob64 = P.add(ob64), o_cells = 0;
+    size_t o_rh32 = P.add(rh32), o_rh64 = P.add(rh64), o_ob32 = P.add(ob32), o_ob64 = P.add(ob64),
+           o_tally = P.add(std::vector<int>(2, 0)), o_cells = 0;
     double clo[2] = {1e300, 1e300}, chi[2] = {-1e300, -1e300}, reach = 0.0;
+    std::vector<double> r_in;
     bool plane = true;  // non-negative sizes, finite, unit axes
     for (int i = 0; i < nr && plane; ++i) {
         plane = std::isfinite(rh64[2 * i]) && std::isfinite(rh64[2 * i + 1]) && rh64[2 * i] >= 0.0 && rh64[2 * i + 1] >= 0.0;
         reach = std::max(reach, std::hypot(rh64[2 * i], rh64[2 * i + 1]));
+        r_in.push_back(std::min(rh64[2 * i], rh64[2 * i + 1]));
     }
     for (int o = 0; o < no && plane; ++o) {
         const double* b = ob64.data() + 8 * o;
@@ -995,7 +1022,7 @@ int mrcc_scene_create_planar_boxes(int n_robots, const double* robot_half_extent
     V.ob32 = at<float>(d, o_ob32);
     V.ob64 = at<double>(d, o_ob64);
     V.grid.rec = at<uint4>(d, o_cells);
-    rc = build_cells(sc);
+    rc = build_cells(sc, (int*)((unsigned char*)d + o_tally), r_in);
     if (rc != MRCC_OK) {
         (void)hipFree(sc->dev_mem);
         delete box;

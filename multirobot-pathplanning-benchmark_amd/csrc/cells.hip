@@ -10,11 +10,13 @@ namespace {
 // exceeds the gap over sqrt 2), within the inscribed radius the overlap is certain.
 // 128 x 128 cells: 10 us (2 disks, 20 rectangles), 30 us (4 boxes, 100 obstacles), once per scene.
 __device__ inline void cell_fill(CellGrid C, double hd, double slack, int i, double r_in, double r_out, int n_obs,
-                                 int t, const DiskView* D, const PlanarView* P) {
+                                 int t, const DiskView* D, const PlanarView* P, int* tally) {
     const int cy = t / C.n, cx = t - cy * C.n;
     const double x = (double)C.x0 + (cx + 0.5) / (double)C.ix, y = (double)C.y0 + (cy + 0.5) / (double)C.iy;
     unsigned short h[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    const double wx = 0.5 / (double)C.ix, wy = 0.5 / (double)C.iy;
     unsigned n = 0;
+    int own = 0;  // obstacles centred in the cell
     // obstacles through LDS, 64 at a time: read one by one they were a chain of dependent round trips
     // (100 boxes: 40 us)
     __shared__ double s_ob[64][8];
@@ -40,8 +42,12 @@ __device__ inline void cell_fill(CellGrid C, double hd, double slack, int i, dou
             }
             __syncthreads();
         }
-        if (n == CELL_HIT) continue;
         const double* b = s_ob[o & 63];
+        if (tally) {
+            const bool rect = !P && o >= D->ns;
+            own += fabs(x - (rect ? 0.5 * (b[0] + b[2]) : b[0])) <= wx && fabs(y - (rect ? 0.5 * (b[1] + b[3]) : b[1])) <= wy;
+        }
+        if (n == CELL_HIT) continue;
         double d2, lo = r_in, hi = r_out;  // squared distance
         if (P) {
             const double tx = x - b[0], ty = y - b[1];
@@ -76,30 +82,42 @@ __device__ inline void cell_fill(CellGrid C, double hd, double slack, int i, dou
     r.z = h[4] | ((unsigned)h[5] << 16);
     r.w = h[6] | ((unsigned)h[7] << 16);
     ((uint4*)C.rec)[(size_t)i * C.n * C.n + t] = r;
+    if (own) {
+        atomicAdd(tally, own);
+        atomicAdd(tally + 1, own * (n == CELL_HIT ? 0 : min((int)n, CELL_LIST + 1)));
+    }
 }
 
-__global__ void __launch_bounds__(256) k_cells_disk(DiskView S, double hd, double slack) {
+__global__ void __launch_bounds__(256) k_cells_disk(DiskView S, double hd, double slack, int* tally) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
     const double r = sqrt(S.rp2_64[i]);
-    cell_fill(S.grid, hd, slack, i, r, r, S.ns + S.nrect, t, &S, nullptr);
+    cell_fill(S.grid, hd, slack, i, r, r, S.ns + S.nrect, t, &S, nullptr, tally);
 }
 
-__global__ void __launch_bounds__(256) k_cells_planar(PlanarView S, double hd, double slack) {
+__global__ void __launch_bounds__(256) k_cells_planar(PlanarView S, double hd, double slack, int* tally) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
     const double a = S.rh64[2 * i], b = S.rh64[2 * i + 1];
-    cell_fill(S.grid, hd, slack, i, fmin(a, b), sqrt(a * a + b * b), S.no, t, nullptr, &S);
+    cell_fill(S.grid, hd, slack, i, fmin(a, b), sqrt(a * a + b * b), S.no, t, nullptr, &S, tally);
 }
 
 }  // namespace
 
-// Fills the table that sc's view points to (grid.rec, corner and scale set).
-void launch_cells(const SceneRec& sc, hipStream_t st) {
+// Fills the table that sc's view points to (grid.rec, corner and scale set).  tally[0] counts the
+// obstacles by the cells that hold their centres, over all robots, tally[1] the tests that those cells
+// leave open (none where contact is certain, 8 for CELL_MANY); null: not counted.
+void launch_cells(const SceneRec& sc, int* tally, hipStream_t st) {
     const CellGrid& C = sc.kind == KIND_DISKS ? sc.disk.grid : sc.planar.grid;
-    const double wx = 1.0 / (double)C.ix, wy = 1.0 / (double)C.iy;
-    const double hd = 0.5 * sqrt(wx * wx + wy * wy);
-    const double ext = std::max(std::max(fabs((double)C.x0), fabs((double)C.y0)), C.n * std::max(wx, wy));
-    const double slack = cell_slack(ext, std::max(wx, wy));
+    double hd, slack;
+    cell_size(C, &hd, &slack);
     const dim3 grid((C.n * C.n + 255) / 256, sc.n_robots);
-    if (sc.kind == KIND_DISKS) k_cells_disk<<<grid, 256, 0, st>>>(sc.disk, hd, slack);
-    else k_cells_planar<<<grid, 256, 0, st>>>(sc.planar, hd, slack);
+    if (sc.kind == KIND_DISKS) k_cells_disk<<<grid, 256, 0, st>>>(sc.disk, hd, slack, tally);
+    else k_cells_planar<<<grid, 256, 0, st>>>(sc.planar, hd, slack, tally);
+}
+
+// half diagonal of a cell, slack of the table
+void cell_size(const CellGrid& C, double* hd, double* slack) {
+    const double wx = 1.0 / (double)C.ix, wy = 1.0 / (double)C.iy;
+    const double ext = std::max(std::max(fabs((double)C.x0), fabs((double)C.y0)), C.n * std::max(wx, wy));
+    *hd = 0.5 * sqrt(wx * wx + wy * wy);
+    *slack = cell_slack(ext, std::max(wx, wy));
 }

@@ -92,8 +92,9 @@ void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, 
 bool lane_looks_apply(const SceneRec& sc);
 void launch_lane_looks(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, bool reset, hipStream_t st);
 #define MRCC_NO_QUEUE (-1)  // lgG of such a run
-// cells.hip: fills the cell table of a plane scene
-void launch_cells(const SceneRec& sc, hipStream_t st);
+// cells.hip: fills the cell table of a plane scene; tally: two zeroed device words or null
+void launch_cells(const SceneRec& sc, int* tally, hipStream_t st);
+void cell_size(const CellGrid& C, double* hd, double* slack);
 void launch_fill_u8(unsigned char* p, long long n, unsigned char v, hipStream_t st);
 // plain per-call form: edge 0 of B in one workgroup (k_arm_edge / k_lane_edge)
 void launch_edge1(const SceneRec& sc, const EdgeBatchView& B, hipStream_t st);

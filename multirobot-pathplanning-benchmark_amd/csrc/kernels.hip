@@ -455,15 +455,19 @@ __device__ inline EdgeWin win_of(const PlanWork& W, int e, int incl) {
 
 // ============================================================================================
 // lane-per-state kinds
-template <class View, int T1, int T2>
+template <class View, int T1, int T2, bool ALL>
 __device__ inline bool lane_collides(const View& S, const double* q, unsigned mask, unsigned& rc) {
     auto at = [&](int k) { return q[k]; };
-    if constexpr (std::is_same<View, PlanarView>::value) return planar_state<T1, false>(S, at, mask, rc);
-    else if constexpr (T1 == 2) return disk2_state<T2, false>(S, at, mask, rc);
-    else return disk_collides<0, 0>(S, q, mask, rc);
+    if constexpr (std::is_same<View, PlanarView>::value) {
+        if constexpr (ALL) return planar_collides<T1>(S, q, mask, rc);
+        else return planar_state<T1, false>(S, at, mask, rc);
+    } else {
+        if constexpr (ALL) return disk_collides<T1, T2>(S, q, mask, rc);
+        else return disk2_state<T2, false>(S, at, mask, rc);
+    }
 }
 
-template <class View, int T1, int T2>
+template <class View, int T1, int T2, bool ALL>
 __global__ void __launch_bounds__(256) k_lane_persistent(View S, EdgeBatchView B, PlanWork W,
                                                          int lgG, int spt) {
     constexpr int MAXD = LaneDim<View, T1, T2>::value;
@@ -507,7 +511,7 @@ __global__ void __launch_bounds__(256) k_lane_persistent(View S, EdgeBatchView B
                     for (int k = 0; k < MAXD; ++k)
                         if (k < D) q[k] = interp_dir_f64(a[k * B.ds], W.dir[(long long)ref.e * D + k], i);
                     ++n_eval;
-                    if (lane_collides<View, T1, T2>(S, q, B.mask, rechecks)) {
+                    if (lane_collides<View, T1, T2, ALL>(S, q, B.mask, rechecks)) {
                         edge_kill(B.out, ref.e);
                         break;
                     }
@@ -526,7 +530,7 @@ __global__ void __launch_bounds__(256) k_lane_persistent(View S, EdgeBatchView B
 }
 
 // direct form: block = 64 lanes, `wpe` blocks per edge (block b -> edge b / wpe); lane-per-state
-template <class View, int T1, int T2>
+template <class View, int T1, int T2, bool ALL>
 __global__ void __launch_bounds__(64) k_lane_direct(View S, EdgeBatchView B, const int* list,
                                                     long long n_list, int wpe, int init_out,
                                                     unsigned long long* stats) {
@@ -558,7 +562,7 @@ __global__ void __launch_bounds__(64) k_lane_direct(View S, EdgeBatchView B, con
                     for (int k = 0; k < MAXD; ++k)
                         if (k < D) q[k] = interp_f64(a[k * B.ds], b[k * B.ds], N, i);
                     ++n_eval;
-                    coll = lane_collides<View, T1, T2>(S, q, B.mask, rechecks);
+                    coll = lane_collides<View, T1, T2, ALL>(S, q, B.mask, rechecks);
                 }
             }
             if (__any(coll)) {
@@ -573,7 +577,7 @@ __global__ void __launch_bounds__(64) k_lane_direct(View S, EdgeBatchView B, con
     }
 }
 
-template <class View, int T1, int T2>
+template <class View, int T1, int T2, bool ALL>
 __global__ void __launch_bounds__(256) k_lane_configs(View S, const double* qv, long long n,
                                                       long long rs, long long ds, unsigned mask,
                                                       unsigned char* out) {
@@ -586,7 +590,7 @@ __global__ void __launch_bounds__(256) k_lane_configs(View S, const double* qv, 
 #pragma unroll
         for (int k = 0; k < MAXD; ++k)
             if (k < D) q[k] = qv[r * rs + k * ds];
-        out[r] = lane_collides<View, T1, T2>(S, q, mask, rechecks) ? 0 : 1;
+        out[r] = lane_collides<View, T1, T2, ALL>(S, q, mask, rechecks) ? 0 : 1;
     }
 }
 
@@ -1430,8 +1434,8 @@ void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork&
     switch (sc.kind) {
         case KIND_DISKS:
         case KIND_PLANAR:
-            lane_dispatch(sc, [&](auto view, auto t1, auto t2) {
-                k_lane_persistent<decltype(view), t1, t2><<<grid, 256, 0, st>>>(view, B, W, lgG, spt);
+            lane_dispatch(sc, [&](auto view, auto t1, auto t2, auto all) {
+                k_lane_persistent<decltype(view), t1, t2, all><<<grid, 256, 0, st>>>(view, B, W, lgG, spt);
             });
             break;
         case KIND_ARMS: {
@@ -1496,8 +1500,8 @@ void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, 
     switch (sc.kind) {
         case KIND_DISKS:
         case KIND_PLANAR:
-            lane_dispatch(sc, [&](auto view, auto t1, auto t2) {
-                k_lane_direct<decltype(view), t1, t2><<<grid, 64, 0, st>>>(view, B, list, n_list, wpe, init_out, stats);
+            lane_dispatch(sc, [&](auto view, auto t1, auto t2, auto all) {
+                k_lane_direct<decltype(view), t1, t2, all><<<grid, 64, 0, st>>>(view, B, list, n_list, wpe, init_out, stats);
             });
             break;
         case KIND_ARMS: {
@@ -1529,8 +1533,8 @@ void launch_configs(const SceneRec& sc, const double* q, long long n, long long 
         case KIND_PLANAR: {
             int g = grid_for(n, 256);
             if (g > max_grid) g = max_grid;
-            lane_dispatch(sc, [&](auto view, auto t1, auto t2) {
-                k_lane_configs<decltype(view), t1, t2><<<g, 256, 0, st>>>(view, q, n, rs, ds, mask, out);
+            lane_dispatch(sc, [&](auto view, auto t1, auto t2, auto all) {
+                k_lane_configs<decltype(view), t1, t2, all><<<g, 256, 0, st>>>(view, q, n, rs, ds, mask, out);
             });
             break;
         }

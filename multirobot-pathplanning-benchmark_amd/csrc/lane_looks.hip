@@ -262,9 +262,9 @@ void launch_lane_looks(const SceneRec& sc, const EdgeBatchView& B, const PlanWor
     const long long waves = (B.n + (1 << lgE) - 1) >> lgE;
     const int blocks = (int)((waves + LOOK_NW - 1) / LOOK_NW);
     const size_t lds = (size_t)LOOK_NW * 2 * (sizeof(double) << lgE) * sc.D;
-    lane_dispatch(sc, [&](auto view, auto t1, auto t2) {
+    lane_dispatch(sc, [&](auto view, auto t1, auto t2, auto all) {
         using V = decltype(view);
-        if constexpr (std::is_same<V, PlanarView>::value || t1 == 2) {
+        if constexpr (!all) {  // scenes with a table
             k_lane_looks<V, t1, t2><<<blocks, 64 * LOOK_NW, lds, st>>>(view, B, W, lgE);
             k_lane_items<V, t1, t2><<<4 * mrcc_internal::device_cus(), 64 * LOOK_NW, 0, st>>>(view, B, W);
         }

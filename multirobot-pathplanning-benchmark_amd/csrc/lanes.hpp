@@ -66,7 +66,9 @@ __device__ inline void edge_kill(unsigned char* out, int e) {
 }
 
 // Disks in the plane: <DiskView, 2, NRB>, at most NRB robots; planar boxes: <PlanarView, NRB, 0>,
-// likewise; other disks: <DiskView, 0, 0>.
+// likewise; other disks: <DiskView, 0, 0>.  ALL: every obstacle is tested (scenes without a cell table,
+// where it is the faster evaluator): <DiskView, 2, 2> two disks, <PlanarView, 4, 0> four boxes,
+// <PlanarView, 0, 0> any number.
 // register length of the per-lane state
 template <class View, int T1, int T2>
 struct LaneDim {
@@ -77,18 +79,31 @@ struct LaneDim<PlanarView, T1, 0> {
     static constexpr int value = 3 * (T1 ? T1 : MRCC_PLANAR_MAX_ROBOTS);
 };
 
-// calls F(view, T1, T2) with the smallest bounds that hold the scene
+// Calls F(view, T1, T2, ALL) with the smallest bounds that hold the scene.
+// Without a table, us of 200,000 configurations by planar_collides / disk_collides (ALL) and by
+// planar_state / disk2_state with every obstacle: 4 boxes 85 / 120, 2 disks 34 / 38; 1 and 2 boxes 87 / 46, 55 /
+// 36, 1, 3 and 4 disks 162 / 37, 568 / 134, 787 / 177; 8 boxes 264 / 249, but queues of 200,000 edges 1,271 /
+// 1,430.
 template <class F>
 static void lane_dispatch(const SceneRec& sc, F f) {
     using std::integral_constant;
+    const std::true_type all{};
+    const std::false_type table{};
+    const integral_constant<int, 0> c0{};
+    const integral_constant<int, 2> c2{};
+    const integral_constant<int, 4> c4{};
     if (sc.kind == KIND_DISKS) {
-        if (sc.disk.rd == 2 && sc.disk.nr <= 2) f(sc.disk, integral_constant<int, 2>(), integral_constant<int, 2>());
-        else if (sc.disk.rd == 2 && sc.disk.nr <= 4) f(sc.disk, integral_constant<int, 2>(), integral_constant<int, 4>());
-        else f(sc.disk, integral_constant<int, 0>(), integral_constant<int, 0>());
+        const bool none = sc.disk.grid.n == 0;
+        if (sc.disk.rd == 2 && sc.disk.nr == 2 && none) f(sc.disk, c2, c2, all);
+        else if (sc.disk.rd == 2 && sc.disk.nr <= 2) f(sc.disk, c2, c2, table);
+        else if (sc.disk.rd == 2 && sc.disk.nr <= 4) f(sc.disk, c2, c4, table);
+        else f(sc.disk, c0, c0, all);
     } else {
-        if (sc.planar.nr <= 4) f(sc.planar, integral_constant<int, 4>(), integral_constant<int, 0>());
-        else if (sc.planar.nr <= 8) f(sc.planar, integral_constant<int, 8>(), integral_constant<int, 0>());
-        else f(sc.planar, integral_constant<int, MRCC_PLANAR_MAX_ROBOTS>(), integral_constant<int, 0>());
+        const bool none = sc.planar.grid.n == 0;
+        if (sc.planar.nr == 4 && none) f(sc.planar, c4, c0, all);
+        else if (sc.planar.nr <= 4) f(sc.planar, c4, c0, table);
+        else if (none) f(sc.planar, c0, c0, all);
+        else if (sc.planar.nr <= 8) f(sc.planar, integral_constant<int, 8>(), c0, table);
+        else f(sc.planar, integral_constant<int, MRCC_PLANAR_MAX_ROBOTS>(), c0, table);
     }
 }
-

@@ -50,3 +50,42 @@ def test_queue_of_edges_beyond_its_passes(rd, nr, incl):
     assert 0 < ref.sum() < n
     tune = B.make_tune(slots_per_pass=1, use_graph=0)
     assert np.array_equal(gpu_edges(sc, a, b, 0.01, tune=tune, N=N, N_start=S, incl=incl), ref)
+
+
+def _spread(desc, how):
+    """Obstacles of a plane scene with one far off, a long wall, or half of them moved away."""
+    disks = desc.kind == "disks"
+    pos = desc.rect_center if disks else desc.obstacle_pose
+    if how == "far":
+        pos[0, :2] = [500.0, 300.0]
+    elif how == "groups":
+        pos[::2, 0] += 300.0
+    else:
+        pos[0, :2] = [0.0, 2.3]
+        if disks:
+            desc.rect_size[0] = [120.0, 0.1]
+        else:
+            desc.obstacle_half[0], desc.obstacle_pose[0, 2] = [60.0, 0.05], 0.0
+
+
+@pytest.mark.parametrize("how", ["far", "wall", "groups"])
+@pytest.mark.parametrize("kind,nr", [("disks", 1), ("disks", 2), ("disks", 3), ("disks", 5), ("planar", 1), ("planar", 4),
+                                     ("planar", 5), ("planar", 9)])
+@pytest.mark.parametrize("no", [12, 70])
+def test_scenes_spread_wide(how, kind, nr, no):
+    # few obstacles leave the table few tests, many make the scene give it up
+    rng = np.random.default_rng(no + nr)
+    desc = (scenes.planar_disks(rng=rng, n_robots=nr, n_rects=no) if kind == "disks" else
+            scenes.planar_boxes(rng=rng, n_robots=nr, n_obstacles=no))
+    if kind == "planar":
+        desc.robot_half *= 0.4
+    else:
+        desc.robot_radius = desc.robot_radius * 0.5
+    _spread(desc, how)
+    sc, o = backend().Scene(desc), O.Scene(desc)
+    n = 5000
+    a = rng.uniform(desc.limits[0], desc.limits[1], (n, desc.dim))
+    b = a + rng.normal(0, 0.15, a.shape)
+    for mask in (0xFFFFFFFF, 0b1):
+        assert np.array_equal(gpu_configs(sc, a, mask=mask), o.check_configs(a, mask=mask)), mask
+        assert np.array_equal(gpu_edges(sc, a, b, 0.02, mask=mask), o.check_edges(a, b, 0.02, mask=mask)), mask

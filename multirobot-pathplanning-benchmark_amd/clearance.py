@@ -59,8 +59,7 @@ class _ClearanceFn:
                     return cost
 
                 @staticmethod
-                @torch.autograd.function.once_differentiable
-                def backward(ctx, grad_cost):
+                def backward(ctx, grad_cost):  # plain: once_differentiable costs 8 us a call
                     q, dq = ctx.saved_tensors
                     g = grad_cost.contiguous().to(torch.float32)
                     grad_q = torch.empty_like(q)
@@ -74,7 +73,11 @@ class _ClearanceFn:
 
 
 def clearance_cost(scene, q, margin: float = 0.02):
-    """q: float32 device tensor [..., D] -> cost [...] (differentiable w.r.t. q)."""
+    """q: float32 device tensor [..., D] -> cost [...] (differentiable w.r.t. q).
+
+    The gradient is formed with the cost when ``q`` requires one; a caller that wants the cost alone says so
+    with ``torch.no_grad()`` (262,144 waypoints of 28 joints: 444 us, 634 with the gradient).  In a graph
+    made with ``create_graph`` the gradient is a constant: there is no second derivative."""
     torch = _torch()
     if q.dtype != torch.float32 or not q.is_cuda:
         raise TypeError("clearance_cost needs a float32 HIP tensor")

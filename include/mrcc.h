@@ -169,7 +169,8 @@ typedef struct mrcc_tune {
     int32_t slots_per_pass;    /* states of one edge issued per pass (coarse-to-fine order); 0: the
                                   library's choice (plane scenes then run without the queue) */
     int32_t slots_per_ticket;  /* queue slots a wave claims per atomic ticket (arm scenes:
-                                  <= 64, one lane resolves one slot) */
+                                  <= 64, one lane resolves one slot); 0: the library's choice (arm
+                                  scenes: by the length of the queue) */
     int32_t waves_per_cu;      /* persistent grid = waves_per_cu * CUs */
     int32_t sorted;            /* 1: edges ordered longest-first */
     int32_t persistent;        /* 1: persistent work-queue kernel; 0: one workgroup per edge */

@@ -26,7 +26,7 @@ DEFAULT = dict(slots_per_pass=0, slots_per_ticket=0, waves_per_cu=0)  # the libr
 LANE_GRID = [dict(slots_per_pass=g, slots_per_ticket=t, waves_per_cu=w)
              for g in (4, 8, 16, 32) for t in (1, 2, 4) for w in (8, 16)] + [DIRECT, DEFAULT]
 ARM_GRID = [dict(slots_per_pass=g, slots_per_ticket=t, waves_per_cu=w)
-            for g in (1, 2, 4, 8) for t in (8, 16, 32) for w in (12, 16)] + [DIRECT]
+            for g in (1, 2, 4, 8) for t in (8, 16, 32) for w in (12, 16)] + [DIRECT, DEFAULT]
 
 
 def candidate_name(cand: dict) -> str:

@@ -703,7 +703,7 @@ int tune_defaults(const SceneRec* sc, const mrcc_tune* tune, mrcc_tune* t) {
     // plane scenes with a cell table take the queue when its shape is asked for, or its statistics
     if (t->slots_per_pass <= 0)
         t->slots_per_pass = arms ? 1 : (lane_looks_apply(*sc) && !t->collect_stats ? 0 : 8);
-    if (t->slots_per_ticket <= 0) t->slots_per_ticket = arms ? 16 : 4;
+    if (t->slots_per_ticket <= 0) t->slots_per_ticket = arms ? 0 : 4;  // 0: queue_cut, by the queue's length
     if (t->waves_per_cu <= 0) t->waves_per_cu = 16;
     if (!tune) {
         t->sorted = 1;

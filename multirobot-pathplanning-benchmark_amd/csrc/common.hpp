@@ -579,6 +579,18 @@ __host__ __device__ inline long long queue_chunk(long long n_waves, int x, long 
     return n_waves + x + MRCC_QUEUE_COUNTERS * k;
 }
 
+// Slots per chunk of an arm queue of T slots on n_waves waves, where the caller asks for none (us at
+// one slot per pass): up to 192 slots a wave 8, since a chunk of 16 leaves a wave alone with its live
+// states at the end (75,065 edges of six arms, 132 slots a wave: 474 at 16, 375 at 8, 383 at 4); longer
+// queues 16, they pay for the round trips instead (99,840 edges of three arms, 227 slots a wave: 1,066 /
+// 1,096 / 1,155); short queues one chunk per wave, so that no wave draws a ticket.
+__host__ __device__ inline int queue_cut(long long T, long long n_waves) {
+    const int spt = T < 192 * n_waves ? 8 : 16;
+    if (T <= 2 * n_waves) return T > n_waves ? 2 : 1;
+    if (T < n_waves * spt) return T / n_waves > 2 ? (int)(T / n_waves) : 2;
+    return spt;
+}
+
 __host__ __device__ inline int erec_w0(int4 r) { return r.w & 0x7fffffff; }
 __host__ __device__ inline int erec_full(int4 r) { return (int)((unsigned)r.w >> 31); }
 

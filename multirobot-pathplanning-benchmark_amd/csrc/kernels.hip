@@ -623,7 +623,7 @@ __device__ inline void arm_stats(unsigned long long* stats, const RecheckT<STATS
     }
 }
 
-// Persistent arm kernel.  A wave claims a chunk of `spt` (<= 64) consecutive slots (after chunks
+// Persistent arm kernel.  A wave claims a chunk of `spt` (<= 64; 0: queue_cut) consecutive slots (after chunks
 // without live states, up to 64 / spt chunks of one counter at once); lane j resolves slot j
 // (slot -> edge, state, mode; edge already dead?) so the dependent loads of all slots overlap;
 // the wave then evaluates the live states one after another, k-major.  The ticket of the next
@@ -641,13 +641,7 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
     plan_clear(W.hist, W.meta);
     const int nw = blockDim.x >> 6;
     const long long n_waves = (long long)gridDim.x * nw;
-    // Chunks of at most 8 slots below 192 slots per wave: one of 16 leaves a wave alone with its live
-    // states at the end (75,065 edges of six arms, 132 slots a wave: 474 us at 16, 375 at 8, 383 at 4);
-    // longer queues pay for the round trips instead (99,840 edges of three arms, 227 slots a wave:
-    // 1,066 / 1,096 / 1,155).  Short queues: one chunk per wave, of one slot below a slot per wave.
-    if (T < 192 * n_waves) spt = min(spt, 8);
-    if (T <= 2 * n_waves) spt = min(spt, T > n_waves ? 2 : 1);
-    else if (T < n_waves * spt) spt = min(spt, max(2, (int)(T / n_waves)));
+    if (spt <= 0) spt = queue_cut(T, n_waves);
     // statistics (compiled away without STATS)
     typename std::conditional<STATS, unsigned long long, NoCount>::type n_eval{}, n_dead{}, n_slots{};
     RecheckT<STATS> rechecks{};

@@ -1,5 +1,7 @@
-"""Chunks of an arm queue (csrc/common.hpp, queue_chunk), on the CPU: for every number of waves, the
-waves' first chunks and those of the eight counters are all chunks of the queue, each once."""
+"""Chunks of an arm queue (csrc/common.hpp), on the CPU: for every number of waves, the waves' first
+chunks and those of the eight counters are all chunks of the queue, each once (queue_chunk); the
+library's chunk size (queue_cut) is one that a wave can resolve, and applies only where the caller
+asks for none (tune_defaults)."""
 import os
 import shutil
 import subprocess
@@ -7,10 +9,11 @@ import subprocess
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "multirobot-pathplanning-benchmark_amd")
 HIPCC = "/opt/rocm/bin/hipcc"
 
 DRIVER = r"""
-#include "evaluators.hpp"
+#include "engine.hpp"
 #include <cstdio>
 #include <vector>
 int main() {
@@ -27,6 +30,24 @@ int main() {
                     return 1;
                 }
         }
+    for (long long n_waves = 1; n_waves <= 5000; n_waves += n_waves < 20 ? 1 : 311)
+        for (long long T = 1; T < 400 * n_waves; T += 1 + T / 7) {
+            const int spt = queue_cut(T, n_waves);
+            if (spt < 1 || spt > 16 || (T >= 8 * n_waves && spt < 8) || (T <= n_waves && spt != 1)) {
+                std::printf("waves %lld, slots %lld: %d slots a chunk\n", n_waves, T, spt);
+                return 1;
+            }
+        }
+    static SceneRec sc;
+    sc.kind = KIND_ARMS;
+    for (int asked : {0, 1, 5, 16, 64}) {
+        mrcc_tune t = {}, d;
+        t.slots_per_ticket = asked;
+        if (mrcc_internal::tune_defaults(&sc, &t, &d) != MRCC_OK || d.slots_per_ticket != asked) {
+            std::printf("slots_per_ticket %d became %d\n", asked, d.slots_per_ticket);
+            return 1;
+        }
+    }
     std::printf("chunks ok\n");
     return 0;
 }
@@ -40,7 +61,8 @@ def test_every_chunk_once(tmp_path):
     src.write_text(DRIVER)
     r = subprocess.run([HIPCC, "-x", "hip", "--offload-arch=gfx950", "-O1", "-std=c++17", "-w", "-Xclang",
                         "-target-feature", "-Xclang", "-packed-fp32-ops",
-                        f"-I{ROOT}/include", f"-I{ROOT}/multirobot-pathplanning-benchmark_amd/csrc", str(src), "-o", str(exe)],
+                        f"-I{ROOT}/include", f"-I{PKG}/csrc", str(src), f"-L{PKG}",
+                        "-lmrcc", f"-Wl,-rpath,{PKG}", "-o", str(exe)],
                        capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr[-2000:]
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)

@@ -775,6 +775,17 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
         int jn = next_slot();
         int en = -1, in_ = 0, mn = 0, nn = 2;
         double an = 0.0, dn = 0.0;  // coordinate `lane` of the next slot's two rows
+        // Other waves may find the batch's edges in collision while this one evaluates: when most edges
+        // collide at their first states, waves that take the next passes early hold slots of edges whose first
+        // state is still being evaluated, and one wave alone went through tens of states that decide
+        // nothing.  There the verdict byte is read again with each next slot's rows: in batches of several tickets,
+        // and beyond the first pass with 6 live slots or more where the last states collided (75,065 edges
+        // of six arms near home 778 -> 448 us, 80,464 of three 322 -> 247, 5,239 of five 122 -> 106).  Elsewhere
+        // it only costs (an agent-scope load; 926 edges of six arms 63 us, 71 with it; states of two
+        // arms do not cover it, 57,803 uniform edges 172, 178 with it).
+        const bool reread = nb > 1 || (p > 0 && V.na > 2 && __builtin_popcountll(__ballot(e >= 0)) >= 6 &&
+                                       __builtin_popcount(recent & 0xffffu) >= 14);
+        bool gone = false;  // the next slot's edge is in collision by now
         if (jn >= 0) {
             en = __builtin_amdgcn_readlane(e, jn);
             in_ = __builtin_amdgcn_readlane(i, jn);
@@ -795,6 +806,7 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
             int ij = in_, nx = __builtin_amdgcn_readlane(next, jc);
             const double aj = an, bj = dn;
             const int Nj = nn;
+            const bool skip = gone;
             jn = next_slot();
             if (jn >= 0) {
                 en = __builtin_amdgcn_readlane(e, jn);
@@ -804,12 +816,13 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
                 nn = __builtin_amdgcn_readlane(N, jn);
                 an = 0.0;
                 dn = 0.0;
+                gone = reread && edge_dead(B.out, en);
                 if (lane < Dn) {
                     an = row1(B, en)[lane * B.ds];
                     dn = row2(B, en)[lane * B.ds];
                 }
             }
-            if ((deadm >> jc) & 1ull) {  // picked before its edge was found in collision
+            if (((deadm >> jc) & 1ull) || __any(skip)) {  // picked before its edge was found in collision
                 ++n_dead;
                 continue;
             }

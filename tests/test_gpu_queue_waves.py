@@ -40,3 +40,17 @@ def test_every_chunk_is_taken(kind, waves_per_cu):
             tune = B.make_tune(slots_per_pass=g, slots_per_ticket=t, waves_per_cu=waves_per_cu)
             got = gpu_edges(sc, a, b, 0.05, N=N, modes=modes, tune=tune)
             assert np.array_equal(got, ref), (n, g, t, int(np.sum(got != ref)))
+
+
+@pytest.mark.parametrize("seed,n_arms,n", [(737, 3, 30000), (195, 5, 5200), (1, 6, 20000)])
+def test_edges_that_collide_near_their_start(seed, n_arms, n):
+    # arms in contact around the home pose: waves hold slots of edges that others are finding in collision
+    rng = np.random.default_rng(seed)
+    desc = scenes.quad_arms(rng=rng, n_arms=n_arms, dof=7, n_boxes=50)
+    sc, o = backend().Scene(desc), O.Scene(desc)
+    a = near_home(rng, desc, n, 0.1)
+    b = np.clip(a + 0.3 * rng.lognormal(0, 1, (n, 1)) * rng.uniform(-1, 1, a.shape), desc.limits[0], desc.limits[1])
+    ref = o.check_edges(a, b, 0.05)
+    assert ref.mean() < 0.5
+    for _ in range(2):
+        assert np.array_equal(gpu_edges(sc, a, b, 0.05), ref)

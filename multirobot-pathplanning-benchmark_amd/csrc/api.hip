@@ -726,6 +726,12 @@ int plan_grid(const SceneRec* sc, const mrcc_tune& t) {
     return sc->kind == KIND_ARMS ? t.waves_per_cu * cus : std::max(1, t.waves_per_cu * cus / 4);
 }
 
+// The queue of plane scenes keeps every edge's step; arms divide for the states they look at, and the
+// runs without a queue hold steps in LDS.
+int plan_step_dim(const SceneRec* sc, const mrcc_tune& t) {
+    return sc->kind != KIND_ARMS && t.persistent && t.slots_per_pass > 0 ? sc->D : 0;
+}
+
 size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W) {
     const long long n = std::max<long long>(n_edges, 1);
     size_t top = 0;
@@ -800,7 +806,7 @@ static void plan_launch_sequence(mrcc_edge_plan* p, hipStream_t st) {
         (void)hipEventRecord(p->ev[2], st);
     } else {
         if (ev) (void)hipEventRecord(p->ev[1], st);
-        launch_direct(*p->sc, p->B, nullptr, p->B.n, 1, 1, 1 << 20, p->W.stats, st);
+        launch_direct(*p->sc, p->B, 1, 1, 1 << 20, p->W.stats, st);
         if (ev) (void)hipEventRecord(p->ev[2], st);
     }
     if (ev) {
@@ -1222,13 +1228,14 @@ int mrcc_edge_plan_create(const mrcc_scene* scene, const mrcc_edge_batch* batch,
     p->lgG = mrcc_internal::plan_lgG(t);
     p->grid = mrcc_internal::plan_grid(sc, t);
     // workspace
-    const size_t work_bytes = mrcc_internal::plan_layout(batch->n_edges, sc->D, nullptr, nullptr);
+    const int step_dim = mrcc_internal::plan_step_dim(sc, t);
+    const size_t work_bytes = mrcc_internal::plan_layout(batch->n_edges, step_dim, nullptr, nullptr);
     if (hipMalloc(&p->work_mem, work_bytes) != hipSuccess) {
         delete p;
         return fail(MRCC_ERR_NOMEM, "workspace of %zu bytes", work_bytes);
     }
     unsigned char* w = (unsigned char*)p->work_mem;
-    mrcc_internal::plan_layout(batch->n_edges, sc->D, w, &p->W);
+    mrcc_internal::plan_layout(batch->n_edges, step_dim, w, &p->W);
     if (!t.collect_stats) p->W.stats = nullptr;
     launch_plan_clear(p->W, (hipStream_t)stream);
     HIP_OK(hipGetLastError());
@@ -1345,14 +1352,15 @@ int mrcc_check_edges(const mrcc_scene* scene, const mrcc_edge_batch* batch, cons
         WorkLease work;
         PlanWork W;
         if (t.persistent) {
-            rc = work.take(box->kept, mrcc_internal::plan_layout(B.n, sc->D, nullptr, nullptr));
+            const int step_dim = mrcc_internal::plan_step_dim(sc, t);
+            rc = work.take(box->kept, mrcc_internal::plan_layout(B.n, step_dim, nullptr, nullptr));
             if (rc != MRCC_OK) return rc;
-            mrcc_internal::plan_layout(B.n, sc->D, work.dev, &W);
+            mrcc_internal::plan_layout(B.n, step_dim, work.dev, &W);
             W.stats = nullptr;
             mrcc_internal::launch_plan_sequence(*sc, B, W, mrcc_internal::plan_lgG(t), t.slots_per_ticket,
                                                 mrcc_internal::plan_grid(sc, t), st, true);
         } else {
-            launch_direct(*sc, B, nullptr, B.n, 1, 1, 1 << 20, nullptr, st);
+            launch_direct(*sc, B, 1, 1, 1 << 20, nullptr, st);
         }
         hipError_t e = hipGetLastError();
         long long* m = work.k ? work.k->meta : meta;
@@ -1651,7 +1659,7 @@ int mrcc_check_edges_host(const mrcc_scene* scene, const double* q1, const doubl
     // ones; no more than the longest edge has states (a wave without one would only stage the scene)
     int wpe = n >= 2048 ? 1 : (int)std::min<int64_t>(64, std::max<int64_t>(1, 2048 / n));
     wpe = std::max(1, std::min(wpe, maxN));
-    launch_direct(*sc, v, nullptr, n, wpe, 0, 32 * device_cus(), nullptr, st);
+    launch_direct(*sc, v, wpe, 0, 32 * device_cus(), nullptr, st);
     HIP_OK(hipGetLastError());
     if (zc) {
         // the flag kernel runs after every wave of the check (stream order) and its write reaches

@@ -85,8 +85,8 @@ void launch_plan_build(const SceneRec& sc, const EdgeBatchView& B, const PlanWor
 void launch_plan_clear(const PlanWork& W, hipStream_t st);
 void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG,
                      int spt, int grid, hipStream_t st);
-void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, long long n_list,
-                   int wpe, int init_out, int max_grid, unsigned long long* stats, hipStream_t st);
+void launch_direct(const SceneRec& sc, const EdgeBatchView& B, int wpe, int init_out, int max_grid,
+                   unsigned long long* stats, hipStream_t st);
 // lane_looks.hip: edge batches of plane scenes with a cell table, two launches, no queue; W.meta is
 // zero before the workspace's first run (`reset`: cleared here, for workspaces used otherwise too)
 bool lane_looks_apply(const SceneRec& sc);
@@ -110,6 +110,11 @@ void launch_configs(const SceneRec& sc, const double* q, long long n, long long 
                     hipStream_t st);
 // self-collision screen of arm states (screen.hip), ahead of the full evaluators
 bool arm_screen_applies(const SceneRec& sc, long long n, long long n_min);
+// From these sizes on.  us with the screen / without, 2, 4 and 6 arms of 7 joints, 50 boxes: 512 uniform edges 50 /
+// 46, 47 / 43, 54 / 43, 1,536: 51 / 56, 50 / 46, 53 / 47, 4,096: 53 / 66, 52 / 60, 55 / 63 (0.4 rad around home: 49 /
+// 58, 54 / 61, 65 / 65; 56 / 87, 58 / 79, 68 / 82; 67 / 92, 74 / 83, 85 / 106).  Configurations 0.4 rad around home,
+// where it catches least: 16,384: 55 / 47, 65 / 52, 99 / 105, 49,152: 97 / 107, 115 / 121, 158 / 270; uniform ones
+// 47 / 43, 43 / 45, 46 / 78 and 68 / 93, 49 / 98, 52 / 196.
 #define MRCC_SCREEN_MIN_EDGES 1536
 #define MRCC_SCREEN_MIN_CONFIGS 49152
 void launch_screen_edges(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, hipStream_t st);
@@ -151,8 +156,10 @@ EdgeBatchView batch_view(const mrcc_edge_batch* b);
 // execution shape: defaults filled in and checked (mrcc_edge_plan_create's rules)
 int tune_defaults(const SceneRec* sc, const mrcc_tune* tune, mrcc_tune* t);
 int plan_grid(const SceneRec* sc, const mrcc_tune& t);
-// Bytes of a plan's workspace for n_edges edges of D coordinates; with W, lays it out from base.
+// Bytes of a plan's workspace for n_edges edges; with W, lays it out from base.  D: coordinates of the
+// stored steps, 0 without them (plan_step_dim).
 size_t plan_layout(long long n_edges, int D, unsigned char* base, PlanWork* W);
+int plan_step_dim(const SceneRec* sc, const mrcc_tune& t);
 // queue build and persistent kernel on stream st (lgG = MRCC_NO_QUEUE: the two launches of
 // lane_looks.hip); `clear` as for launch_plan_build
 void launch_plan_sequence(const SceneRec& sc, const EdgeBatchView& B, const PlanWork& W, int lgG, int spt,

@@ -531,19 +531,17 @@ __global__ void __launch_bounds__(256) k_lane_persistent(View S, EdgeBatchView B
 
 // direct form: block = 64 lanes, `wpe` blocks per edge (block b -> edge b / wpe); lane-per-state
 template <class View, int T1, int T2, bool ALL>
-__global__ void __launch_bounds__(64) k_lane_direct(View S, EdgeBatchView B, const int* list,
-                                                    long long n_list, int wpe, int init_out,
+__global__ void __launch_bounds__(64) k_lane_direct(View S, EdgeBatchView B, int wpe, int init_out,
                                                     unsigned long long* stats) {
     constexpr int MAXD = LaneDim<View, T1, T2>::value;
     const int D = S.D;
     const int lane = threadIdx.x;
     unsigned long long n_eval = 0;
     unsigned rechecks = 0;
-    const long long nblocks = n_list * wpe;
+    const long long nblocks = B.n * wpe;
     for (long long blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
-        const long long li = blk / wpe;
+        const long long e = blk / wpe;
         const int u = (int)(blk % wpe);
-        const long long e = list ? (long long)list[li] : li;
         if (init_out && lane == 0) B.out[e] = 1;  // only with wpe == 1
         const int N = edge_N_dev(B, e, D);
         EdgeWin w = edge_window(N, batch_N_start(B, e), batch_N_max(B, e), B.incl);
@@ -883,13 +881,12 @@ __global__ void __launch_bounds__(GRASP ? 64 * MRCC_PERSISTENT_GRASP_NW : 256, G
     arm_persistent_body<GRASP, CHAIN, STATS>(V, Q, Q, lgG, spt);
 }
 
-// Work item k of n_list * wpe: edge list[k / wpe] (or k / wpe), states k % wpe, k % wpe + wpe, ...
+// Work item k of B.n * wpe: edge k / wpe, states k % wpe, k % wpe + wpe, ...
 // With init_out (wpe == 1 only) the wave owns its edge: it writes the verdict without reading it.
 // A mode id outside [0, nm) makes the edge's verdict 0 (the error contract of mujoco_env.py:797-807,
 // "exception => collision"); entry points with host-side mode ids reject them before launching.
 template <bool GRASP, bool CHAIN>
-__global__ void __launch_bounds__(256) k_arm_direct(ArmK V, EdgeBatchView B, const int* list,
-                                                    long long n_list, int wpe, int init_out,
+__global__ void __launch_bounds__(256) k_arm_direct(ArmK V, EdgeBatchView B, int wpe, int init_out,
                                                     unsigned long long* stats) {
     extern __shared__ double lds_arm[];
     arm_stage_scene(lds_arm, V);
@@ -899,12 +896,11 @@ __global__ void __launch_bounds__(256) k_arm_direct(ArmK V, EdgeBatchView B, con
     unsigned long long n_eval = 0;
     unsigned rechecks = 0;
     ArmCountT<true> cnt = {0, 0, 0, 0};
-    const long long nitems = n_list * wpe;
+    const long long nitems = B.n * wpe;
     const long long w0 = (long long)blockIdx.x * nw + (threadIdx.x >> 6);
     for (long long it = w0; it < nitems; it += (long long)gridDim.x * nw) {
-        const long long li = it / wpe;
+        const long long e = it / wpe;
         const int u = (int)(it % wpe);
-        const long long e = list ? (long long)list[li] : li;
         const int mode = batch_mode(B, e);
         const int md = (mode >= 0 && mode < V.nm) ? mode : 0;
         const int N = edge_N_dev(B, e, V.D);
@@ -1499,16 +1495,15 @@ void launch_fill_u8(unsigned char* p, long long n, unsigned char v, hipStream_t 
     k_fill_u8<<<grid_for(n, 256), 256, 0, st>>>(p, n, v);
 }
 
-void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, long long n_list,
-                   int wpe, int init_out, int max_grid, unsigned long long* stats, hipStream_t st) {
-    const long long blocks = n_list * wpe;
+void launch_direct(const SceneRec& sc, const EdgeBatchView& B, int wpe, int init_out, int max_grid, unsigned long long* stats, hipStream_t st) {
+    const long long blocks = B.n * wpe;
     int grid = (int)(blocks < max_grid ? blocks : max_grid);
     if (grid < 1) grid = 1;
     switch (sc.kind) {
         case KIND_DISKS:
         case KIND_PLANAR:
             lane_dispatch(sc, [&](auto view, auto t1, auto t2, auto all) {
-                k_lane_direct<decltype(view), t1, t2, all><<<grid, 64, 0, st>>>(view, B, list, n_list, wpe, init_out, stats);
+                k_lane_direct<decltype(view), t1, t2, all><<<grid, 64, 0, st>>>(view, B, wpe, init_out, stats);
             });
             break;
         case KIND_ARMS: {
@@ -1517,7 +1512,7 @@ void launch_direct(const SceneRec& sc, const EdgeBatchView& B, const int* list, 
             const int nw = grid < sc.arm_nw ? 1 : sc.arm_nw;
             const size_t lds = nw == 1 ? sc.arm_lds1 : sc.arm_lds;
             const int blocks = (grid + nw - 1) / nw;
-#define MRCC_ARM_DIRECT(G, C) k_arm_direct<G, C><<<blocks, 64 * nw, lds, st>>>(sc.armk, B, list, n_list, wpe, init_out, stats)
+#define MRCC_ARM_DIRECT(G, C) k_arm_direct<G, C><<<blocks, 64 * nw, lds, st>>>(sc.armk, B, wpe, init_out, stats)
             if (sc.arm.chain) {
                 if (sc.arm_has_grasp) MRCC_ARM_DIRECT(true, true);
                 else MRCC_ARM_DIRECT(false, true);

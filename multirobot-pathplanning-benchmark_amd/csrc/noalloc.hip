@@ -1,8 +1,9 @@
 // noalloc.hip — the batched edge check without device allocation (mrcc_check_edges_noalloc).
 //
 // The queue of mrcc_check_edges needs a workspace (per-edge records, the sorted order, the pass
-// tables, the interpolation steps, counters).  mrcc_check_edges allocates it per call; this entry
-// point uses one file-scope device array instead, `scratch`, for callers that cannot allocate:
+// tables, the interpolation steps, counters).  mrcc_check_edges keeps one with the scene and allocates
+// when that is too small or held by another call; this entry point uses one file-scope device array
+// instead, `scratch`, for callers that cannot allocate:
 // code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  Every GPU the
 // library runs on holds its own copy of the array until the process ends.  Host code reaches a
 // device's copy only through the address hipGetSymbolAddress returns with that device current (the
@@ -17,8 +18,9 @@
 
 #include "engine.hpp"
 
-// 16 MiB: per edge 16 + 4 + 4 + 8 D bytes (record, order, long-edge list, interpolation step),
-// plus about 264 KiB of pass tables and counters: about 65,000 edges of 28 coordinates.
+// 16 MiB: per edge 16 + 4 + 4 + 8 D bytes, plus about 264 KiB of pass tables and counters: about 65,000
+// edges of 28 coordinates.  The limit counts the largest layout for every scene (record, order, steps of
+// plane queues, 4 bytes unused), so that which batches are refused depends on their size alone.
 #define MRCC_NOALLOC_SCRATCH_BYTES (16u << 20)
 #define MRCC_NOALLOC_MAX_DEVICES 64
 

@@ -132,13 +132,16 @@ __device__ inline float clr_sq(float ex, float ey, float ez) { return fmaf(ez, e
 // centres (micrometres) with a wide margin.
 #define CLR_CULL_EPS 1e-4f
 
+// within reach (up to rounding)
+__device__ inline bool clr_near(float e2, float R) { return e2 <= R * R * 1.0001f; }
+
 // One penetration term: cost += pen^2 for pen = R - d > 0, and with GRAD the force g e on the first
 // sphere (g = -2 pen / d).  The square root only for pairs within reach: d < R implies
 // e2 < R^2 (1 + 2^-21), so the bound passes every pair with pen > 0.
 template <bool GRAD>
 __device__ inline bool clr_term(float ex, float ey, float ez, float R, float& cost, float& gx, float& gy, float& gz) {
     const float e2 = clr_sq(ex, ey, ez);
-    if (!(e2 <= R * R * 1.0001f)) return false;
+    if (!clr_near(e2, R)) return false;
     const float d = sqrtf(e2);
     const float pen = R - d;
     if (!(pen > 0.f)) return false;
@@ -205,7 +208,9 @@ __device__ inline float clr_suffix8(float v) {
 }
 
 // The full pair set without culling (the scene's broad phase off): lane = sphere i, every partner
-// j >= sph_lo[i] and every box in turn.  Returns the lane's share of the cost.
+// j >= sph_lo[i] and every box in turn.  With the gradient a partner that no lane has in reach ends
+// at its distance (262,144 waypoints 5.16 ms when every lane branched for itself, 4.12 now; the cost alone is
+// faster by lanes, 3.43 against 3.80).  Returns the lane's share of the cost.
 template <bool GRAD>
 __device__ inline float clr_pairs_all(const ClrK& V, const ClrLds& W, float m) {
     const int lane = wave_lane();
@@ -218,8 +223,11 @@ __device__ inline float clr_pairs_all(const ClrK& V, const ClrLds& W, float m) {
         float fx = 0.f, fy = 0.f, fz = 0.f;
         for (int b = 0; b < V.nb; ++b) {
             const float3 e = clr_box_e(ci, V.box32[2 * b], V.box32[2 * b + 1]);
+            const float R = m + ci.w;
+            const bool near = act && clr_near(clr_sq(e.x, e.y, e.z), R);
+            if (GRAD && __ballot(near) == 0ull) continue;
             float gx, gy, gz;
-            if (act && clr_term<GRAD>(e.x, e.y, e.z, m + ci.w, cost, gx, gy, gz)) {
+            if (near && clr_term<GRAD>(e.x, e.y, e.z, R, cost, gx, gy, gz)) {
                 fx += gx;
                 fy += gy;
                 fz += gz;
@@ -228,8 +236,11 @@ __device__ inline float clr_pairs_all(const ClrK& V, const ClrLds& W, float m) {
         const int lo = act ? V.sph_lo[i] : 0x7fffffff;
         for (int j = V.sph_lo[base]; j < S; ++j) {
             const float4 cj = W.sph[j];
+            const float ex = ci.x - cj.x, ey = ci.y - cj.y, ez = ci.z - cj.z, R = m + ci.w + cj.w;
+            const bool near = j >= lo && clr_near(clr_sq(ex, ey, ez), R);
+            if (GRAD && __ballot(near) == 0ull) continue;
             float gx, gy, gz;
-            if (j >= lo && clr_term<GRAD>(ci.x - cj.x, ci.y - cj.y, ci.z - cj.z, m + ci.w + cj.w, cost, gx, gy, gz)) {
+            if (near && clr_term<GRAD>(ex, ey, ez, R, cost, gx, gy, gz)) {
                 fx += gx;
                 fy += gy;
                 fz += gz;

@@ -925,7 +925,7 @@ int mrcc_scene_create_disks(int n_robots, int robot_dim, const double* robot_rad
         return rc;
     }
     void* d = sc->dev_mem;
-    DiskView& V = sc->disk;
+    DiskGridView& V = sc->disk;
     V.nr = nr; V.rd = rd; V.D = nr * rd; V.ns = ns; V.nrect = nq;
     V.Bscene = (float)B;
     V.r32 = at<float>(d, o_r);
@@ -1020,7 +1020,7 @@ int mrcc_scene_create_planar_boxes(int n_robots, const double* robot_half_extent
         return rc;
     }
     void* d = sc->dev_mem;
-    PlanarView& V = sc->planar;
+    PlanarGridView& V = sc->planar;
     V.nr = nr; V.no = no; V.D = 3 * nr;
     V.Bscene = (float)(B + 4.0 * H);
     V.rh32 = at<float>(d, o_rh32);

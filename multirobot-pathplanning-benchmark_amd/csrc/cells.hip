@@ -88,13 +88,13 @@ __device__ inline void cell_fill(CellGrid C, double hd, double slack, int i, dou
     }
 }
 
-__global__ void __launch_bounds__(256) k_cells_disk(DiskView S, double hd, double slack, int* tally) {
+__global__ void __launch_bounds__(256) k_cells_disk(DiskGridView S, double hd, double slack, int* tally) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
     const double r = sqrt(S.rp2_64[i]);
     cell_fill(S.grid, hd, slack, i, r, r, S.ns + S.nrect, t, &S, nullptr, tally);
 }
 
-__global__ void __launch_bounds__(256) k_cells_planar(PlanarView S, double hd, double slack, int* tally) {
+__global__ void __launch_bounds__(256) k_cells_planar(PlanarGridView S, double hd, double slack, int* tally) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
     const double a = S.rh64[2 * i], b = S.rh64[2 * i + 1];
     cell_fill(S.grid, hd, slack, i, fmin(a, b), sqrt(a * a + b * b), S.no, t, nullptr, &S, tally);

@@ -428,7 +428,12 @@ struct DiskView {
     const float* lo32; const float* hi32;     // [nrect*rd]
     const double* lo64; const double* hi64;
     const float* rp2_32; const double* rp2_64;  // [nr] r**2
-    CellGrid grid;                            // rd = 2 (obstacles: spheres, then rectangles)
+};
+// With the cell table (rd = 2; obstacles: spheres, then rectangles).  Apart from the view, which kernels
+// that change it hold in private memory (disks beyond the specialised shapes: 80 bytes of scratch more
+// with the table in it, 39 instead of 37 us a call).
+struct DiskGridView : DiskView {
+    CellGrid grid;
 };
 
 struct PlanarView {
@@ -436,6 +441,8 @@ struct PlanarView {
     float Bscene;
     const float* rh32; const double* rh64;  // [nr*2]
     const float* ob32; const double* ob64;  // [no*8] x y ux uy vx vy h0 h1
+};
+struct PlanarGridView : PlanarView {
     CellGrid grid;
 };
 

@@ -43,8 +43,8 @@ struct SceneRec {
     int D;
     int n_robots;
     int device;
-    DiskView disk;
-    PlanarView planar;
+    DiskGridView disk;
+    PlanarGridView planar;
     ArmView arm;          // every array of an arm scene (clearance and kinematics kernels)
     ArmK armk;            // the edge and configuration kernels' view of the same scene
     ClrK clr;             // the clearance kernels' view

@@ -445,7 +445,7 @@ __device__ inline bool cell_any(uint4 r, int n_all, F test) {
 
 // planar boxes, nr <= NRB robots
 template <int NRB, bool LOOK, class Q>
-__device__ inline bool planar_state(const PlanarView& S, const Q& q, unsigned mask, unsigned& rechecks) {
+__device__ inline bool planar_state(const PlanarGridView& S, const Q& q, unsigned mask, unsigned& rechecks) {
     const int nr = S.nr;
     float x[NRB], y[NRB];
     uint4 rec[NRB];
@@ -519,7 +519,7 @@ __device__ inline bool planar_state(const PlanarView& S, const Q& q, unsigned ma
 
 // disks in the plane, nr <= NRB robots
 template <int NRB, bool LOOK, class Q>
-__device__ inline bool disk2_state(const DiskView& S, const Q& q, unsigned mask, unsigned& rechecks) {
+__device__ inline bool disk2_state(const DiskGridView& S, const Q& q, unsigned mask, unsigned& rechecks) {
     const int nr = S.nr;
     float x[NRB], y[NRB];
     uint4 rec[NRB];

@@ -455,19 +455,19 @@ __device__ inline EdgeWin win_of(const PlanWork& W, int e, int incl) {
 
 // ============================================================================================
 // lane-per-state kinds
-template <class View, int T1, int T2, bool ALL>
+template <class View, int T1, int T2>
 __device__ inline bool lane_collides(const View& S, const double* q, unsigned mask, unsigned& rc) {
     auto at = [&](int k) { return q[k]; };
-    if constexpr (std::is_same<View, PlanarView>::value) {
-        if constexpr (ALL) return planar_collides<T1>(S, q, mask, rc);
+    if constexpr (LaneKind<View>::planar) {
+        if constexpr (LaneKind<View>::all) return planar_collides<T1>(S, q, mask, rc);
         else return planar_state<T1, false>(S, at, mask, rc);
     } else {
-        if constexpr (ALL) return disk_collides<T1, T2>(S, q, mask, rc);
+        if constexpr (LaneKind<View>::all) return disk_collides<T1, T2>(S, q, mask, rc);
         else return disk2_state<T2, false>(S, at, mask, rc);
     }
 }
 
-template <class View, int T1, int T2, bool ALL>
+template <class View, int T1, int T2>
 __global__ void __launch_bounds__(256) k_lane_persistent(View S, EdgeBatchView B, PlanWork W,
                                                          int lgG, int spt) {
     constexpr int MAXD = LaneDim<View, T1, T2>::value;
@@ -511,7 +511,7 @@ __global__ void __launch_bounds__(256) k_lane_persistent(View S, EdgeBatchView B
                     for (int k = 0; k < MAXD; ++k)
                         if (k < D) q[k] = interp_dir_f64(a[k * B.ds], W.dir[(long long)ref.e * D + k], i);
                     ++n_eval;
-                    if (lane_collides<View, T1, T2, ALL>(S, q, B.mask, rechecks)) {
+                    if (lane_collides<View, T1, T2>(S, q, B.mask, rechecks)) {
                         edge_kill(B.out, ref.e);
                         break;
                     }
@@ -530,7 +530,7 @@ __global__ void __launch_bounds__(256) k_lane_persistent(View S, EdgeBatchView B
 }
 
 // direct form: block = 64 lanes, `wpe` blocks per edge (block b -> edge b / wpe); lane-per-state
-template <class View, int T1, int T2, bool ALL>
+template <class View, int T1, int T2>
 __global__ void __launch_bounds__(64) k_lane_direct(View S, EdgeBatchView B, int wpe, int init_out,
                                                     unsigned long long* stats) {
     constexpr int MAXD = LaneDim<View, T1, T2>::value;
@@ -560,7 +560,7 @@ __global__ void __launch_bounds__(64) k_lane_direct(View S, EdgeBatchView B, int
                     for (int k = 0; k < MAXD; ++k)
                         if (k < D) q[k] = interp_f64(a[k * B.ds], b[k * B.ds], N, i);
                     ++n_eval;
-                    coll = lane_collides<View, T1, T2, ALL>(S, q, B.mask, rechecks);
+                    coll = lane_collides<View, T1, T2>(S, q, B.mask, rechecks);
                 }
             }
             if (__any(coll)) {
@@ -575,7 +575,7 @@ __global__ void __launch_bounds__(64) k_lane_direct(View S, EdgeBatchView B, int
     }
 }
 
-template <class View, int T1, int T2, bool ALL>
+template <class View, int T1, int T2>
 __global__ void __launch_bounds__(256) k_lane_configs(View S, const double* qv, long long n,
                                                       long long rs, long long ds, unsigned mask,
                                                       unsigned char* out) {
@@ -588,7 +588,7 @@ __global__ void __launch_bounds__(256) k_lane_configs(View S, const double* qv, 
 #pragma unroll
         for (int k = 0; k < MAXD; ++k)
             if (k < D) q[k] = qv[r * rs + k * ds];
-        out[r] = lane_collides<View, T1, T2, ALL>(S, q, mask, rechecks) ? 0 : 1;
+        out[r] = lane_collides<View, T1, T2>(S, q, mask, rechecks) ? 0 : 1;
     }
 }
 
@@ -881,12 +881,12 @@ __global__ void __launch_bounds__(GRASP ? 64 * MRCC_PERSISTENT_GRASP_NW : 256, G
     arm_persistent_body<GRASP, CHAIN, STATS>(V, Q, Q, lgG, spt);
 }
 
-// Work item k of B.n * wpe: edge k / wpe, states k % wpe, k % wpe + wpe, ...
+// Work item k of n_edges * wpe: edge k / wpe, states k % wpe, k % wpe + wpe, ...
 // With init_out (wpe == 1 only) the wave owns its edge: it writes the verdict without reading it.
 // A mode id outside [0, nm) makes the edge's verdict 0 (the error contract of mujoco_env.py:797-807,
 // "exception => collision"); entry points with host-side mode ids reject them before launching.
 template <bool GRASP, bool CHAIN>
-__global__ void __launch_bounds__(256) k_arm_direct(ArmK V, EdgeBatchView B, int wpe, int init_out,
+__global__ void __launch_bounds__(256) k_arm_direct(ArmK V, EdgeBatchView B, long long n_edges, int wpe, int init_out,
                                                     unsigned long long* stats) {
     extern __shared__ double lds_arm[];
     arm_stage_scene(lds_arm, V);
@@ -896,7 +896,7 @@ __global__ void __launch_bounds__(256) k_arm_direct(ArmK V, EdgeBatchView B, int
     unsigned long long n_eval = 0;
     unsigned rechecks = 0;
     ArmCountT<true> cnt = {0, 0, 0, 0};
-    const long long nitems = B.n * wpe;
+    const long long nitems = n_edges * wpe;  // an argument of its own: B.n here cost the held-box form 4%
     const long long w0 = (long long)blockIdx.x * nw + (threadIdx.x >> 6);
     for (long long it = w0; it < nitems; it += (long long)gridDim.x * nw) {
         const long long e = it / wpe;
@@ -1437,8 +1437,9 @@ void launch_plan_run(const SceneRec& sc, const EdgeBatchView& B, const PlanWork&
     switch (sc.kind) {
         case KIND_DISKS:
         case KIND_PLANAR:
-            lane_dispatch(sc, [&](auto view, auto t1, auto t2, auto all) {
-                k_lane_persistent<decltype(view), t1, t2, all><<<grid, 256, 0, st>>>(view, B, W, lgG, spt);
+            lane_dispatch(sc, [&](const auto& view, auto t1, auto t2) {
+                using View = typename std::decay<decltype(view)>::type;
+                k_lane_persistent<View, t1, t2><<<grid, 256, 0, st>>>(view, B, W, lgG, spt);
             });
             break;
         case KIND_ARMS: {
@@ -1502,8 +1503,9 @@ void launch_direct(const SceneRec& sc, const EdgeBatchView& B, int wpe, int init
     switch (sc.kind) {
         case KIND_DISKS:
         case KIND_PLANAR:
-            lane_dispatch(sc, [&](auto view, auto t1, auto t2, auto all) {
-                k_lane_direct<decltype(view), t1, t2, all><<<grid, 64, 0, st>>>(view, B, wpe, init_out, stats);
+            lane_dispatch(sc, [&](const auto& view, auto t1, auto t2) {
+                using View = typename std::decay<decltype(view)>::type;
+                k_lane_direct<View, t1, t2><<<grid, 64, 0, st>>>(view, B, wpe, init_out, stats);
             });
             break;
         case KIND_ARMS: {
@@ -1512,7 +1514,7 @@ void launch_direct(const SceneRec& sc, const EdgeBatchView& B, int wpe, int init
             const int nw = grid < sc.arm_nw ? 1 : sc.arm_nw;
             const size_t lds = nw == 1 ? sc.arm_lds1 : sc.arm_lds;
             const int blocks = (grid + nw - 1) / nw;
-#define MRCC_ARM_DIRECT(G, C) k_arm_direct<G, C><<<blocks, 64 * nw, lds, st>>>(sc.armk, B, wpe, init_out, stats)
+#define MRCC_ARM_DIRECT(G, C) k_arm_direct<G, C><<<blocks, 64 * nw, lds, st>>>(sc.armk, B, B.n, wpe, init_out, stats)
             if (sc.arm.chain) {
                 if (sc.arm_has_grasp) MRCC_ARM_DIRECT(true, true);
                 else MRCC_ARM_DIRECT(false, true);
@@ -1535,8 +1537,9 @@ void launch_configs(const SceneRec& sc, const double* q, long long n, long long 
         case KIND_PLANAR: {
             int g = grid_for(n, 256);
             if (g > max_grid) g = max_grid;
-            lane_dispatch(sc, [&](auto view, auto t1, auto t2, auto all) {
-                k_lane_configs<decltype(view), t1, t2, all><<<g, 256, 0, st>>>(view, q, n, rs, ds, mask, out);
+            lane_dispatch(sc, [&](const auto& view, auto t1, auto t2) {
+                using View = typename std::decay<decltype(view)>::type;
+                k_lane_configs<View, t1, t2><<<g, 256, 0, st>>>(view, q, n, rs, ds, mask, out);
             });
             break;
         }
@@ -1608,38 +1611,40 @@ template <bool CONFIG>
 static void launch_lane1(const SceneRec& sc, const EdgeBatchView& B, hipStream_t st) {
 #define MRCC_LANE1(VIEW, T1, T2, STG, NT, S) k_lane_edge<VIEW, T1, T2, STG, NT, CONFIG><<<1, NT, 0, st>>>(S, B)
     if (sc.kind == KIND_DISKS) {
-        const bool stg = lane_stage_fits(sc.disk);
+        const DiskView& D = sc.disk;
+        const bool stg = lane_stage_fits(D);
         const bool small = sc.disk.ns + sc.disk.nrect <= LANE_SMALL_SCENE;
         if (sc.disk.rd == 2 && sc.disk.nr == 2) {
             if (small) {
-                if (stg) MRCC_LANE1(DiskView, 2, 2, true, 256, sc.disk);
-                else MRCC_LANE1(DiskView, 2, 2, false, 256, sc.disk);
+                if (stg) MRCC_LANE1(DiskView, 2, 2, true, 256, D);
+                else MRCC_LANE1(DiskView, 2, 2, false, 256, D);
             } else if (stg) {
-                MRCC_LANE1(DiskView, 2, 2, true, 1024, sc.disk);
+                MRCC_LANE1(DiskView, 2, 2, true, 1024, D);
             } else {
-                MRCC_LANE1(DiskView, 2, 2, false, 1024, sc.disk);
+                MRCC_LANE1(DiskView, 2, 2, false, 1024, D);
             }
         } else if (stg) {
-            MRCC_LANE1(DiskView, 0, 0, true, 256, sc.disk);
+            MRCC_LANE1(DiskView, 0, 0, true, 256, D);
         } else {
-            MRCC_LANE1(DiskView, 0, 0, false, 256, sc.disk);
+            MRCC_LANE1(DiskView, 0, 0, false, 256, D);
         }
     } else if (sc.kind == KIND_PLANAR) {
-        const bool stg = lane_stage_fits(sc.planar);
+        const PlanarView& P = sc.planar;
+        const bool stg = lane_stage_fits(P);
         const bool small = sc.planar.no <= LANE_SMALL_SCENE;
         if (sc.planar.nr == 4) {
             if (small) {
-                if (stg) MRCC_LANE1(PlanarView, 4, 0, true, 256, sc.planar);
-                else MRCC_LANE1(PlanarView, 4, 0, false, 256, sc.planar);
+                if (stg) MRCC_LANE1(PlanarView, 4, 0, true, 256, P);
+                else MRCC_LANE1(PlanarView, 4, 0, false, 256, P);
             } else if (stg) {
-                MRCC_LANE1(PlanarView, 4, 0, true, 1024, sc.planar);
+                MRCC_LANE1(PlanarView, 4, 0, true, 1024, P);
             } else {
-                MRCC_LANE1(PlanarView, 4, 0, false, 1024, sc.planar);
+                MRCC_LANE1(PlanarView, 4, 0, false, 1024, P);
             }
         } else if (stg) {
-            MRCC_LANE1(PlanarView, 0, 0, true, 256, sc.planar);
+            MRCC_LANE1(PlanarView, 0, 0, true, 256, P);
         } else {
-            MRCC_LANE1(PlanarView, 0, 0, false, 256, sc.planar);
+            MRCC_LANE1(PlanarView, 0, 0, false, 256, P);
         }
     }
 #undef MRCC_LANE1

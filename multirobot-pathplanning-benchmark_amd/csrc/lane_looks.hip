@@ -34,11 +34,11 @@ __device__ inline int look_parts(int R, long long cap) {
 }
 
 template <int T1, int T2, bool LOOK, class Q>
-__device__ inline bool lane_state(const DiskView& S, const Q& q, unsigned mask, unsigned& rc) {
+__device__ inline bool lane_state(const DiskGridView& S, const Q& q, unsigned mask, unsigned& rc) {
     return disk2_state<T2, LOOK>(S, q, mask, rc);
 }
 template <int T1, int T2, bool LOOK, class Q>
-__device__ inline bool lane_state(const PlanarView& S, const Q& q, unsigned mask, unsigned& rc) {
+__device__ inline bool lane_state(const PlanarGridView& S, const Q& q, unsigned mask, unsigned& rc) {
     return planar_state<T1, LOOK>(S, q, mask, rc);
 }
 
@@ -262,9 +262,9 @@ void launch_lane_looks(const SceneRec& sc, const EdgeBatchView& B, const PlanWor
     const long long waves = (B.n + (1 << lgE) - 1) >> lgE;
     const int blocks = (int)((waves + LOOK_NW - 1) / LOOK_NW);
     const size_t lds = (size_t)LOOK_NW * 2 * (sizeof(double) << lgE) * sc.D;
-    lane_dispatch(sc, [&](auto view, auto t1, auto t2, auto all) {
-        using V = decltype(view);
-        if constexpr (!all) {  // scenes with a table
+    lane_dispatch(sc, [&](const auto& view, auto t1, auto t2) {
+        using V = typename std::decay<decltype(view)>::type;
+        if constexpr (!LaneKind<V>::all) {  // scenes with a table
             k_lane_looks<V, t1, t2><<<blocks, 64 * LOOK_NW, lds, st>>>(view, B, W, lgE);
             k_lane_items<V, t1, t2><<<4 * mrcc_internal::device_cus(), 64 * LOOK_NW, 0, st>>>(view, B, W);
         }

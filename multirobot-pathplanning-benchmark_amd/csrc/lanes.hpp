@@ -65,45 +65,48 @@ __device__ inline void edge_kill(unsigned char* out, int e) {
     __hip_atomic_store(out + e, (unsigned char)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Disks in the plane: <DiskView, 2, NRB>, at most NRB robots; planar boxes: <PlanarView, NRB, 0>,
-// likewise; other disks: <DiskView, 0, 0>.  ALL: every obstacle is tested (scenes without a cell table,
-// where it is the faster evaluator): <DiskView, 2, 2> two disks, <PlanarView, 4, 0> four boxes,
-// <PlanarView, 0, 0> any number.
+// Disks in the plane: <DiskGridView, 2, NRB>, at most NRB robots; planar boxes: <PlanarGridView, NRB, 0>,
+// likewise.  Views without the table (LaneKind::all): every obstacle is tested, by the evaluators that are
+// the faster ones then: <DiskView, 2, 2> two disks in the plane, <DiskView, 0, 0> any disks,
+// <PlanarView, 4, 0> four boxes, <PlanarView, 0, 0> any number.
+template <class View>
+struct LaneKind {
+    static constexpr bool planar = std::is_base_of<PlanarView, View>::value;
+    static constexpr bool all = std::is_same<View, DiskView>::value || std::is_same<View, PlanarView>::value;
+};
 // register length of the per-lane state
 template <class View, int T1, int T2>
 struct LaneDim {
-    static constexpr int value = T1 ? T1 * T2 : MRCC_DISK_MAX_RD * 4;
-};
-template <int T1>
-struct LaneDim<PlanarView, T1, 0> {
-    static constexpr int value = 3 * (T1 ? T1 : MRCC_PLANAR_MAX_ROBOTS);
+    static constexpr int value = LaneKind<View>::planar ? 3 * (T1 ? T1 : MRCC_PLANAR_MAX_ROBOTS)
+                                                        : (T1 ? T1 * T2 : MRCC_DISK_MAX_RD * 4);
 };
 
-// Calls F(view, T1, T2, ALL) with the smallest bounds that hold the scene.
-// Without a table, us of 200,000 configurations by planar_collides / disk_collides (ALL) and by
+// Calls F(view, T1, T2) with the smallest bounds that hold the scene.
+// Without a table, us of 200,000 configurations by planar_collides / disk_collides and by
 // planar_state / disk2_state with every obstacle: 4 boxes 85 / 120, 2 disks 34 / 38; 1 and 2 boxes 87 / 46, 55 /
 // 36, 1, 3 and 4 disks 162 / 37, 568 / 134, 787 / 177; 8 boxes 264 / 249, but queues of 200,000 edges 1,271 /
 // 1,430.
 template <class F>
 static void lane_dispatch(const SceneRec& sc, F f) {
     using std::integral_constant;
-    const std::true_type all{};
-    const std::false_type table{};
     const integral_constant<int, 0> c0{};
     const integral_constant<int, 2> c2{};
     const integral_constant<int, 4> c4{};
     if (sc.kind == KIND_DISKS) {
-        const bool none = sc.disk.grid.n == 0;
-        if (sc.disk.rd == 2 && sc.disk.nr == 2 && none) f(sc.disk, c2, c2, all);
-        else if (sc.disk.rd == 2 && sc.disk.nr <= 2) f(sc.disk, c2, c2, table);
-        else if (sc.disk.rd == 2 && sc.disk.nr <= 4) f(sc.disk, c2, c4, table);
-        else f(sc.disk, c0, c0, all);
+        const DiskGridView& V = sc.disk;
+        const DiskView& all = V;
+        if (V.rd != 2 || V.nr > 4) f(all, c0, c0);
+        else if (V.nr == 2 && V.grid.n == 0) f(all, c2, c2);
+        else if (V.nr <= 2) f(V, c2, c2);
+        else f(V, c2, c4);
     } else {
-        const bool none = sc.planar.grid.n == 0;
-        if (sc.planar.nr == 4 && none) f(sc.planar, c4, c0, all);
-        else if (sc.planar.nr <= 4) f(sc.planar, c4, c0, table);
-        else if (none) f(sc.planar, c0, c0, all);
-        else if (sc.planar.nr <= 8) f(sc.planar, integral_constant<int, 8>(), c0, table);
-        else f(sc.planar, integral_constant<int, MRCC_PLANAR_MAX_ROBOTS>(), c0, table);
+        const PlanarGridView& V = sc.planar;
+        const PlanarView& all = V;
+        const bool none = V.grid.n == 0;
+        if (V.nr == 4 && none) f(all, c4, c0);
+        else if (V.nr <= 4) f(V, c4, c0);
+        else if (none) f(all, c0, c0);
+        else if (V.nr <= 8) f(V, integral_constant<int, 8>(), c0);
+        else f(V, integral_constant<int, MRCC_PLANAR_MAX_ROBOTS>(), c0);
     }
 }

@@ -2,7 +2,8 @@
 //
 // Edge batches run as one pass-ordered work queue (see PlanWork):
 //   prep      : a few lanes per edge: N (abstract_env.py:321-323), window (:325-331), slot count M,
-//               passes S = ceil(M / G) (at most MRCC_MAX_PASSES), histogram of S
+//               passes S = ceil(M / G) (at most MRCC_MAX_PASSES), histogram of S (arms: k_arm_records;
+//               in larger batches k_arm_screen then ends the edges whose middle state surely collides)
 //   scatter   : E_p = #{edges with S > p}, pass offsets PS[p] = G * sum_{p'<p} E_p' (every block sums
 //               the histogram for itself); counting sort, edges longest-first
 //   persistent: waves claim chunks of queue slots from 8 XCD-interleaved counters; slot -> (pass p,
@@ -750,7 +751,7 @@ __device__ inline void arm_persistent_body(const ArmK& V, const ArmQueue& B, con
         // The live slots are evaluated in turn, k-major: the first slot of every edge of the chunk,
         // then the second, ...  Most states of random edges collide, so an edge usually dies at
         // its first state; in this order the state after it belongs to another edge, and the inputs
-        // loaded for it ahead of time (its edge's row and step, binary64) are used.  The slots of
+        // loaded for it ahead of time (its edge's two rows, binary64) are used.  The slots of
         // edges that died in this chunk are skipped.  The next chunk's ticket is requested after
         // the first slot's loads, so none of these round trips sits on the evaluation path.
         const int G = 1 << lgG;
